@@ -32,7 +32,7 @@ METRIC = "Gcell-steps/s at 12M cells; batched scenarios/hr + p99 latency vs plai
 HBM_PEAK_GBS = 8000.0
 B_ALG = {False: 36.0, True: 44.0}  # bytes per cell-step (arrival tracking off / on)
 # the launches of one step, and the profile file stem of its measured HBM traffic
-KERNEL_NAME = {"sweep": "k_sweep_deep + k_sweep (general, hand-back)", "tile": "k_step"}
+KERNEL_NAME = {"sweep": "k_sweep", "tile": "k_step"}
 TRAFFIC_FILE = {"sweep": "sweep_step_12M_traffic.json", "tile": "k_step_12M_traffic.json"}
 
 
@@ -289,7 +289,7 @@ def main():
     if args.kernel == "sweep" and args.strip_rows == 0:
         rows, tms = solver.autotune(reps=9)  # candidates differ by 1-2 %: a median of 9 replays
         tuned = {"strip_rows": rows, "general_rows": solver.general_rows, "ms_per_step": tms}
-        log(f"autotune: {rows}-row strips ({solver.general_rows}-row general strips), {tms:.4f} ms per step")
+        log(f"autotune: {rows}-row strips ({solver.general_rows}-row general tiles), {tms:.4f} ms per step")
     # capture and upload the step sequences of the tuned strips before the clock starts
     # (no step is taken: the run is at its step limit)
     solver.run_more(0)
@@ -337,7 +337,7 @@ def main():
         v64 = ncell * args.steps / wall64 / 1e9
         fp64 = {"value": v64, "unit": "Gcell-steps/s", "ms_per_step": wall64 * 1e3 / args.steps,
                 "bytes_per_cell_step": 2 * B_ALG[track], "roofline_frac": 2 * B_ALG[track] * v64 / HBM_PEAK_GBS,
-                "kernel": "k_sweep_deep<double> + k_sweep<double> (general, hand-back)", "autotune": tuned64}
+                "kernel": "k_sweep<double>", "autotune": tuned64}
         log(f"fp64: {v64:.1f} Gcell-steps/s")
         s64.close()
 

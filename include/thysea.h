@@ -66,13 +66,13 @@ typedef struct thy_params {
     int precision;     /* 0: FP32 state and fluxes; 1: FP64 everywhere */
     int track_arrival; /* 1: arrival times tracked (reference behaviour) */
     int tile_x, tile_y;/* 2D-tile kernel: tile shape, 0: default */
-    int kernel;        /* step kernel: 0 row sweep with a deep-water launch for blocks far from
-                          coast and borders (default), 1 2D LDS tiles, 2 row sweep with the
-                          general faces everywhere */
-    int strip_rows;    /* row-sweep kernel: rows per strip, 0: default (24) */
-    int general_rows;  /* row-sweep kernel: rows per general strip beside the deep-water
-                          launch (must divide strip_rows), 0: default (taller strips when
-                          the general strips are many, 4-row strips when they are few) */
+    int kernel;        /* step kernel: 0 row sweep, deep-water strips and general tiles (default),
+                          1 2D LDS tiles, 2 row sweep with general tiles everywhere */
+    int strip_rows;    /* row-sweep kernel: most rows of a deep-water strip, 0: default (by the
+                          grid's size, 8 to 32; 16 in a batch).  A small grid stepped alone
+                          takes strips of at most 8 rows */
+    int general_rows;  /* row-sweep kernel: rows per general tile, at most 8 are used, 0: default
+                          (by the grid's size, 4 or 8; 8 in a batch) */
 } thy_params;
 
 /* One Okada fault, fields as a parameter-file fault line (src/Problema.cxx:128-148). */
@@ -199,10 +199,10 @@ size_t thy_footprint(int nx, int ny, const thy_params *params);
 int thy_copy_probe(size_t bytes, int reps, double *ms_per_copy);
 
 /* Strip-height autotuner of the row-sweep kernel.  No reference counterpart (the
-   reference has one fixed launch shape).  For pairs of strip height and general strip
-   height (16/4, 16/8, 24/4, 24/8, 24/12, 32/8, 32/16, 36/18, 40/20, 48/16) it captures 12
-   steps from the current state into a graph (each step redoes the same step), times
-   `reps` replays (HIP events, median) and keeps the fastest; the state, control
+   reference has one fixed launch shape).  For pairs of strip height and tile height (16/4,
+   16/8, 24/8, 32/8, 36/8, 40/8, 48/8) it captures 32 steps from the current state
+   into a graph (each step redoes the same step), times `reps` replays (HIP events,
+   median) and keeps the fastest; the state, control
    blocks and dt slots are left as they were.  Call after thy_upload_state, before or
    between runs.  general_rows may be null. */
 int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, double *ms_per_step);
@@ -213,9 +213,8 @@ int thy_last_timing(thy_ctx *ctx, double *ms_step_kernel);
 /* ---- Batched scenarios --------------------------------------------------------
    No counterpart in the reference, which runs one scenario per process
    (src/GPU/ShallowWater.cu:182-190).  A batch advances many contexts together: a step
-   of the batch is three launches over the strips of every running scenario (the
-   deep-water strips, the general strips beside them, then the strips the deep-water
-   launch handed back), and every scenario keeps its own dt, time, faults, gauges and
+   of the batch is one launch over the tiles and strips of every running scenario, and
+   every scenario keeps its own dt, time, faults, gauges and
    metrics, so its results are those of thy_run on the same context.  Contexts are
    created and uploaded by the caller (thy_create, thy_upload_state), admitted with
    their run configuration, and stay owned by the caller; results are read with

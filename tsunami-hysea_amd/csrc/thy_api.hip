@@ -33,6 +33,15 @@ using namespace thy;
 // the device array behind thy_mass_noalloc's partial sums (see kScratchPartials)
 static __device__ __align__(256) double scratch[1024];
 
+// Work lists of a step, on the device: deep-water strips, and the items (one per
+// workgroup: four strips, or a general tile; item_origin)
+struct WorkLists {
+    int2 *deep = nullptr, *items = nullptr;
+    int n_deep = 0, n_items = 0, deep_cap = 0, items_cap = 0;
+    std::vector<int2> tile_h;    // the general tiles, costliest first, and their costs
+    std::vector<int> tcost_h;
+};
+
 struct thy_ctx {
     int nx = 0, ny = 0, pitch = 0;
     int device = -1;    // the device the context lives on
@@ -58,9 +67,8 @@ struct thy_ctx {
     double *mass_partial = nullptr;
     float *outbuf = nullptr;
     hipStream_t stream = nullptr;
-    hipStream_t side = nullptr;          // general launch beside the deep-water launch
+    hipStream_t side = nullptr;          // the other stream of the cached pair
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // two replays in flight: start / end / control-copied events, pinned copies of the
     // control block, the last launch's dt partials and the health flag after each replay
     hipEvent_t rev[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
@@ -71,26 +79,14 @@ struct thy_ctx {
     int cur = 0;                 // host mirror of ctrl.cur after a sync
     int tx = 64, ty = 16;
     int chunk_rows = 1;          // tile (strip) rows per XCD chunk of the step kernel's order
-    int kernel = 0;              // 0 row sweep (deep-water + general split), 1 2D tiles, 2 row sweep general only
-    int srows = 24;              // row sweep: rows per strip
-    int gsrows = 32;             //   rows per general strip beside the deep-water launch
-    int yoff = 0;                //   row offset of the split launches' strip rows
-    int grows_req = 0;           //   requested general strip height (0: the default rule)
+    int kernel = 0;              // 0 row sweep (deep-water strips and general tiles), 1 2D tiles, 2 general tiles only
+    int srows = 24;              // row sweep: rows per deep-water strip
+    int trows = kTileRows;       //   rows per general tile
     int tuning = 0;              // launches recorded for timing replays publish no control block
     int ncu = 256;               // compute units of the device
-    int *order = nullptr;        // row sweep: workgroup -> strip block, costliest first
-    int order_n = 0;
-    std::vector<int> order_h, cls_h;  // host copies: every block costliest first, and the classes
-    // host lists for batched runs, strips of srows rows: the deep-water ones, and the
-    // general ones with their cost classes; the general strips also cut into strips of
-    // gsrows rows (costliest first) with their classes
-    std::vector<int> bdeep_h, bgen_h, bgcls_h, bsub_h, bsubcls_h;
-    int n_order = 0;             // blocks in `order` (the general launch's share)
-    int *deep = nullptr;         // deep-water strips (n_deep of them)
-    int *gen = nullptr;          // general strips beside them (n_gen)
-    int n_deep = 0, n_gen = 0, list_cap = 0;
-    unsigned int *fb_count = nullptr;  // 3 slots
-    int *fb_list = nullptr;            // [3][list_cap]
+    bool uploaded = false;       // row sweep: the lists describe an uploaded state
+    std::vector<int> coastal, cost;  // [s * (ny + 1) + j]: coastal rows, and cost, of segment s before row j
+    WorkLists alone, batched;    // the lists of a run alone and of a batch (built when first prepared)
     unsigned int *health = nullptr;    // non-finite flag raised by the step kernels
     // captured sequences of gk steps, one per launch slot a replay starts at
     hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
@@ -199,28 +195,17 @@ template <> bool tile_supported<float>(int tx, int ty) {
 template <> bool tile_supported<double>(int tx, int ty) { return (tx == 32 && ty == 8) || (tx == 64 && ty == 4); }
 
 template <typename T>
-StepArgs<T> make_args(thy_ctx *c) {
+StepArgs<T> make_args(thy_ctx *c, const bool batch = false) {
     StepArgs<T> a;
     memset(&a, 0, sizeof(a));
     const thy_params &p = c->prm;
     a.nx = c->nx; a.ny = c->ny; a.pitch = c->pitch;
     a.periodic = (std::fabs(p.borde_izq - 2.0) < 2.220446049250313e-16 && std::fabs(p.borde_der - 2.0) < 2.220446049250313e-16) ? 1 : 0;
     if (c->kernel == 0 || c->kernel == 2) {
-        const int nseg = (c->nx + SW_OUT - 1) / SW_OUT;
-        a.tiles_x = (nseg + SW_WAVES - 1) / SW_WAVES;
-        a.tiles_y = (c->ny + c->srows - 1) / c->srows;
-        a.srows = c->srows;
-        a.gsrows = c->gsrows;
-        a.yoff = c->yoff;
-        a.order = c->order;
-        a.n_order = c->n_order;
-        a.nseg = nseg;
-        a.deep = c->n_deep > 0 ? c->deep : nullptr;
-        a.n_deep = c->n_deep;
-        a.gen = c->gen;
-        a.n_gen = c->n_gen;
-        a.fb_count = c->fb_count;
-        a.fb_list = c->fb_list;
+        const WorkLists &w = batch ? c->batched : c->alone;
+        a.items = w.items;
+        a.n_items = w.n_items;
+        a.deep = w.deep;
     } else {
         a.tiles_x = (c->nx + c->tx - 1) / c->tx;
         a.tiles_y = (c->ny + c->ty - 1) / c->ty;
@@ -260,34 +245,12 @@ StepArgs<T> make_args(thy_ctx *c) {
 template <typename T>
 hipError_t launch_step_t(thy_ctx *c, int slot) {
     StepArgs<T> a = make_args<T>(c);
-    const int n_chunks = (a.tiles_y + c->chunk_rows - 1) / c->chunk_rows;
-    dim3 grid(((n_chunks + 7) / 8) * 8 * a.chunk), block(256);
     if (c->kernel == 0 || c->kernel == 2) {
-        {
-            if (a.deep) {
-                // deep-water blocks on the main stream and the general blocks on the side
-                // stream run side by side; after the join, the hand-backs of this step
-                hipError_t e;
-                if ((e = hipEventRecord(c->ev_fork, c->stream)) != hipSuccess) return e;
-                if ((e = hipStreamWaitEvent(c->side, c->ev_fork, 0)) != hipSuccess) return e;
-                const int g_deep = (a.n_deep + SW_WAVES - 1) / SW_WAVES;
-                if (a.n_gen > 0) {
-                    hipLaunchKernelGGL((k_sweep<T>), dim3((a.n_gen + SW_WAVES - 1) / SW_WAVES), dim3(64 * SW_WAVES), 0,
-                                       c->side, a, slot, 1);
-                    if ((e = hipGetLastError()) != hipSuccess) return e;
-                }
-                hipLaunchKernelGGL((k_sweep_deep<T>), dim3(g_deep), dim3(64 * SW_WAVES), 0, c->stream, a, slot);
-                if ((e = hipGetLastError()) != hipSuccess) return e;
-                if ((e = hipEventRecord(c->ev_join, c->side)) != hipSuccess) return e;
-                if ((e = hipStreamWaitEvent(c->stream, c->ev_join, 0)) != hipSuccess) return e;
-                hipLaunchKernelGGL((k_sweep<T>), dim3(g_deep), dim3(64 * SW_WAVES), 0, c->stream, a, slot, 2);
-                return hipGetLastError();
-            }
-        }
-        if (a.order) grid = dim3(std::max(1, a.n_order));
-        hipLaunchKernelGGL((k_sweep<T>), grid, dim3(64 * SW_WAVES), 0, c->stream, a, slot, 0);
+        hipLaunchKernelGGL((k_sweep<T>), dim3(a.n_items), dim3(64 * SW_WAVES), 0, c->stream, a, slot);
         return hipGetLastError();
     }
+    const int n_chunks = (a.tiles_y + c->chunk_rows - 1) / c->chunk_rows;
+    const dim3 grid(((n_chunks + 7) / 8) * 8 * a.chunk), block(256);
 #define THY_TILE(TX_, TY_)                                                                            \
     if (c->tx == TX_ && c->ty == TY_) {                                                              \
         hipLaunchKernelGGL((k_step<T, TX_, TY_>), grid, block, 0, c->stream, a, slot);               \
@@ -382,10 +345,8 @@ int pick_tile(thy_ctx *c) {
     c->kernel = c->prm.kernel;
     if (c->prm.strip_rows < 0 || c->prm.strip_rows > 65536)
         return fail(c, THY_ERR_INVALID, "strip_rows out of range: " + std::to_string(c->prm.strip_rows));
-    if (c->prm.strip_rows > 0) c->srows = c->prm.strip_rows;
     if (c->prm.general_rows < 0 || c->prm.general_rows > 65536)
         return fail(c, THY_ERR_INVALID, "general_rows out of range: " + std::to_string(c->prm.general_rows));
-    c->grows_req = c->prm.general_rows;
     // THYSEA_CHUNK_ROWS overrides the number of tile rows dealt to one XCD at a time
     if (const char *v = std::getenv("THYSEA_CHUNK_ROWS")) {
         const int r = std::atoi(v);
@@ -394,226 +355,202 @@ int pick_tile(thy_ctx *c) {
     return THY_OK;
 }
 
-// Dispatch order of the row-sweep workgroups.  A strip row whose stencil touches
-// shallow water or land runs the general faces, about 2.5x the work of a deep row, so
-// coastal strips are the longest-running workgroups; dispatching them first lets the
-// deep ones fill in behind them instead of leaving a tail of coastal strips at the end
-// of the launch.  Workgroups of equal cost class keep the chunked XCD order of the
-// kernel.  The estimate uses the still-water depth: a row counts as coastal for a
-// 64-column segment when any cell of it is shallower than 3 hpos (or dry).
-// Rows per general strip for strips of S rows: the requested height when it divides S.
-// Otherwise, when the general launch is bound by throughput (8-row strips would number
-// more than 8 per CU), the largest divisor of S between 8 and min(20, S / 2), whose
-// halos are a smaller share; when it is bound by the time of one strip (smaller grids),
-// the smallest divisor of S from 4 up, the shortest walk.  S itself if none.
-int general_rows_of(int S, int req, size_t n_general, int ncu) {
-    if (req > 0 && S % req == 0) return req;
-    const bool throughput = n_general * (size_t)((S + 7) / 8) > (size_t)8 * std::max(1, ncu);
-    if (throughput) {
-        for (int g = std::min(20, S / 2); g >= 8; g--)
-            if (S % g == 0) return g;
-    } else {
-        for (int g = 4; g < S; g++)
-            if (S % g == 0) return g;
-    }
-    return S;
+// Rows per deep-water strip of a grid of `rows` segment rows (56-column segments times
+// rows) that is stepped alone.  A strip's time is a chain of rows with a halo of 5: with few
+// rows the step is the time of one strip, so strips are short; with many they are as tall as
+// leaves the device one round of them (20 wavefronts a CU).  Measured (us per step):
+// 1000x800 (14400) 19.8 / 25.2 / 32.7 at 8 / 16 / 24 rows; 2000x2000 (72000) 58.9 / 54.7 /
+// 54.2 / 62.2 at 8 / 16 / 24 / 32; 4000x3000 (216000) 139.6 / 132.0 / 141.6 at 16 / 32 / 48.
+int default_strip_rows(const size_t rows, const int ncu) {
+    const size_t per = rows / ((size_t)ncu * 20);
+    return (int)std::min<size_t>(32, std::max<size_t>(8, (per + 4) / 8 * 8));
 }
 
-// Row offset of the split launches' strip rows (strip row k covers rows k*S-yoff ..
-// k*S-yoff+S-1, cut to the grid).  A strip row is deep-water capable only clear of the
-// top and bottom border bands and sponges; the offset that makes the rows that are not
-// thinnest, so that they cost the least general work (a general row about five times a
-// deep-water row, halos included), is taken; ties go to the smaller offset.
-int strip_row_offset(int ny, int S, int sps, int spn) {
-    int best = 0;
-    long best_cost = -1;
-    for (int off = 0; off < S; off++) {
-        long cost = 0;
-        for (int y = -off; y < ny; y += S) {
-            const int y0 = std::max(y, 0), y1 = std::min(y + S, ny);
-            const bool ok = y0 - 4 >= 2 && y1 + 3 <= ny - 3 && y0 - 2 >= sps && y1 + 1 < ny - spn;
-            cost += (long)(y1 - y0 + 8) * (ok ? 1 : 5);
-        }
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = off;
-        }
-    }
-    return best;
+// rows per general tile of a grid stepped alone: half tiles while the tiles are few enough
+// to run side by side (the step then waits for one of them: 240x200 14.3 against 17.7 us,
+// 1501x607 21.4 against 34.7), whole ones, with less halo, when they are many (2000x2000
+// 58.9 against 65.0 us)
+int default_tile_rows(const size_t rows, const int ncu) {
+    return rows <= (size_t)ncu * 128 ? kTileRows / 2 : kTileRows;
 }
 
-template <typename T>
-int build_order(thy_ctx *ctx, const T *D) {
-    thy_ctx *c = ctx;
-    if (c->kernel == 1) return THY_OK;
-    const int nx = c->nx, ny = c->ny, P = c->pitch, S = c->srows;
-    const int nseg = (nx + SW_OUT - 1) / SW_OUT;
-    const int tiles_x = (nseg + SW_WAVES - 1) / SW_WAVES, tiles_y = (ny + S - 1) / S;
-    const int n_tiles = tiles_x * tiles_y;
-    const double thr = 3.0 * c->prm.hpos;
-    // coastal[j * nseg + s]: row j has a shallow or dry cell within segment s's 64 columns
-    std::vector<unsigned char> coastal((size_t)ny * nseg, 0);
-    for (int j = 0; j < ny; j++) {
-        for (int sgi = 0; sgi < nseg; sgi++) {
-            const int xa = std::max(0, sgi * SW_OUT - SW_HALO), xb = std::min(nx, sgi * SW_OUT + SW_OUT + SW_HALO);
-            bool any = false;
-            for (int i = xa; i < xb && !any; i++) any = (double)D[(size_t)j * P + i] <= thr;
-            coastal[(size_t)j * nseg + sgi] = any ? 1 : 0;
+// items in order, dealt in eight runs of (nearly) equal length, one per XCD: the workgroup
+// at list slot b runs on XCD b mod 8, so each XCD sweeps one contiguous band and items side
+// by side share their halos in that XCD's L2.  `per` items make a workgroup; runs are
+// padded to whole workgroups with idle items.
+std::vector<int2> xcd_runs(const std::vector<int2> &items, const int per) {
+    std::vector<int2> out;
+    if (items.empty()) return out;
+    const int n = (int)items.size(), q = n / 8, rem = n % 8;
+    const int wmax = (q + (rem > 0 ? 1 : 0) + per - 1) / per;
+    out.assign((size_t)wmax * 8 * per, make_int2(-1, 0));
+    for (int x = 0; x < 8; x++) {
+        const int size = q + (x < rem ? 1 : 0), start = x * q + std::min(x, rem);
+        for (int i = 0; i < size; i++) out[((size_t)(i / per) * 8 + x) * per + i % per] = items[start + i];
+    }
+    return out;
+}
+
+// A step's work items.  What takes longest goes first, so that the short items fill in at
+// the end: a tile takes 10 to 25 us, a strip of deep water about 1 us a row.  Strips of up to
+// 8 rows follow the tiles; taller ones start with them, the tiles spread behind (`lag` times
+// thinner than even: tiles are bound by arithmetic, strips by memory, and side by side they
+// share a CU).  4000x3000 at 32 rows: 160 us tiles first, 147 strips first, 135 lag 2;
+// 2000x2000 at 16 rows: 60.1, 64.4, 57.6 lag 1.5.  Groups of 8 start on the same XCD.
+std::vector<int2> interleave(const std::vector<int2> &tiles, const int n_deep, const int strip_rows) {
+    std::vector<int2> out;
+    const double lag = strip_rows <= 8 ? 0.0 : (strip_rows <= 16 ? 1.5 : 2.0);
+    const size_t tg = (tiles.size() + 7) / 8, dg = (n_deep + 7) / 8;
+    size_t t = 0, d = 0;
+    while (t < tg || d < dg) {
+        const bool tile = t < tg && (d >= dg || (double)t * dg * lag <= (double)d * tg);
+        for (size_t k = 0; k < 8; k++) {
+            if (tile && t * 8 + k < tiles.size()) out.push_back(tiles[t * 8 + k]);
+            if (!tile && (int)(d * 8 + k) < n_deep) out.push_back(make_int2((int)(d * 8 + k) * SW_WAVES, 0));
         }
+        if (tile) t++;
+        else d++;
     }
-    // per strip (segment sgi of strip row ty): cost class, and whether the deep-water
-    // launch may take it: rows y0-4 .. y1+3 and its 64 columns clear of the grid edges
-    // (no clamping, no first-order band), of the sponges, and of coast
-    // the deep-water path addresses each array through a buffer resource with a 32-bit
-    // byte range
-    const bool split = c->kernel == 0;  // (kernel 0: the state block fits 32-bit offsets)
-    const int spi = c->prm.sponge_izq, spd = c->prm.sponge_der, sps = c->prm.sponge_sup, spn = c->prm.sponge_inf;
-    // strips of the split launches: rows shifted up by yoff (the block order of the
-    // launch without a split keeps unshifted tiles)
-    const int yoff = split ? strip_row_offset(ny, S, sps, spn) : 0;
-    c->yoff = yoff;
-    const int strip_rows = (ny + yoff + S - 1) / S;
-    const int n_strips = strip_rows * nseg;
-    std::vector<int> scls(n_strips, 0);
-    std::vector<unsigned char> sdeep(n_strips, 0);
-    for (int ty = 0; ty < strip_rows; ty++) {
-        const int y0 = std::max(ty * S - yoff, 0), y1 = std::min(ty * S - yoff + S, ny);
-        const int rows = (y1 - y0) + 8;
-        const bool yok = y0 - 4 >= 2 && y1 + 3 <= ny - 3 && y0 - 2 >= sps && y1 + 1 < ny - spn;
-        for (int sgi = 0; sgi < nseg; sgi++) {
-            const int x0 = sgi * SW_OUT;
-            int nc = 0;
-            for (int j = std::max(0, y0 - 4); j < std::min(ny, y1 + 4); j++) nc += coastal[(size_t)j * nseg + sgi];
-            const bool xok = x0 - SW_HALO >= 2 && x0 + SW_OUT + SW_HALO - 1 <= nx - 3 && x0 - SW_HALO >= spi &&
-                             x0 + SW_OUT + SW_HALO - 1 < nx - spd;
-            scls[ty * nseg + sgi] = (int)(1.5 * nc / rows * 4.0 + 0.5);
-            sdeep[ty * nseg + sgi] = (split && yok && xok && nc == 0) ? 1 : 0;
-        }
+    return out;
+}
+
+// a list into its device buffer, which grows as needed
+int put_list(thy_ctx *ctx, int2 *&dst, int &cap, const std::vector<int2> &v) {
+    if (v.empty()) return THY_OK;
+    if (cap < (int)v.size()) {
+        dev_free(dst);
+        dst = nullptr;
+        cap = 0;
+        HIPCHK(dev_alloc(&dst, v.size() * sizeof(int2)));
+        cap = (int)v.size();
     }
-    std::vector<int> cls(n_tiles, 0);
-    for (int t = 0; t < n_tiles; t++) {
-        const int ty = t / tiles_x, tx = t - ty * tiles_x;
-        const int sr = (ty * S + yoff) / S;  // the shifted strip row holding the tile's first row
-        for (int w = 0; w < SW_WAVES; w++) {
-            const int sgi = tx * SW_WAVES + w;
-            if (sgi < nseg) cls[t] = std::max(cls[t], scls[sr * nseg + sgi]);
-        }
-    }
-    // chunked XCD order as the base sequence (the kernel's order without a table)
-    std::vector<int> base;
-    base.reserve(n_tiles);
-    const int chunk = tiles_x * c->chunk_rows;
-    const int n_chunks = (tiles_y + c->chunk_rows - 1) / c->chunk_rows;
-    const int grid = ((n_chunks + 7) / 8) * 8 * chunk;
-    for (int bid = 0; bid < grid; bid++) {
-        const int loc = bid >> 3, ch = loc / chunk;
-        const int t = ((ch << 3) + (bid & 7)) * chunk + (loc - ch * chunk);
-        if (t < n_tiles) base.push_back(t);
-    }
-    // General strips in the base order, costliest first, cut into strips of G rows
-    // (items in units of G rows): short enough that the few slow coastal and border
-    // strips do not set the launch's critical path, long enough that their halo rows
-    // stay a modest share.
-    size_t n_general = 0;
-    for (int item = 0; item < n_strips; item++) n_general += sdeep[item] ? 0 : 1;
-    const int G = general_rows_of(S, c->grows_req, n_general, c->ncu);
-    c->gsrows = G;
-    std::vector<int> deep_rm, gen, gcls;
-    c->bgen_h.clear();
-    c->bgcls_h.clear();
-    // the general strips in the chunked XCD order over the shifted strip rows
-    std::vector<int> sbase;
-    {
-        const int st = tiles_x * strip_rows;
-        const int s_chunks = (strip_rows + c->chunk_rows - 1) / c->chunk_rows;
-        const int s_grid = ((s_chunks + 7) / 8) * 8 * chunk;
-        for (int bid = 0; bid < s_grid; bid++) {
-            const int loc = bid >> 3, ch = loc / chunk;
-            const int t = ((ch << 3) + (bid & 7)) * chunk + (loc - ch * chunk);
-            if (t < st) sbase.push_back(t);
-        }
-    }
-    for (int t : sbase) {
-        const int ty = t / tiles_x, tx = t - ty * tiles_x;
-        for (int w = 0; w < SW_WAVES; w++) {
-            const int sgi = tx * SW_WAVES + w;
-            if (sgi >= nseg) continue;
-            const int item = ty * nseg + sgi;
-            if (sdeep[item]) continue;
-            c->bgen_h.push_back(item);
-            c->bgcls_h.push_back(scls[item]);
-            for (int sub = 0; sub < S / G; sub++) {
-                const int y = ty * S + sub * G - yoff;  // the sub-strip's first row, before the cut at 0
-                if (y + G <= 0 || y >= ny) continue;
-                gen.push_back((ty * (S / G) + sub) * nseg + sgi);
-                gcls.push_back(scls[item]);
-            }
-        }
-    }
-    {
-        std::vector<int> idx(gen.size());
-        for (size_t i = 0; i < idx.size(); i++) idx[i] = (int)i;
-        std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return gcls[a] > gcls[b]; });
-        std::vector<int> g2(gen.size()), c2(gen.size());
-        for (size_t i = 0; i < idx.size(); i++) {
-            g2[i] = gen[idx[i]];
-            c2[i] = gcls[idx[i]];
-        }
-        gen.swap(g2);
-        c->bsub_h = gen;
-        c->bsubcls_h.swap(c2);
-    }
-    // Deep-water strips row-major, cut into 8 runs of (nearly) equal length, one per
-    // XCD: the workgroup at list slot b runs on XCD b mod 8, so each XCD sweeps one
-    // contiguous band and strips side by side share their halo columns in that XCD's
-    // L2.  Runs are padded to whole workgroups with -1 (idle wavefronts).
-    for (int item = 0; item < n_strips; item++)
-        if (sdeep[item]) deep_rm.push_back(item);
-    std::vector<int> deep;
-    if (!deep_rm.empty()) {
-        const int nd = (int)deep_rm.size(), q = nd / 8, rem = nd % 8;
-        const int wmax = (q + (rem > 0 ? 1 : 0) + SW_WAVES - 1) / SW_WAVES;
-        deep.assign((size_t)wmax * 8 * SW_WAVES, -1);
-        for (int x = 0; x < 8; x++) {
-            const int size = q + (x < rem ? 1 : 0), start = x * q + std::min(x, rem);
-            for (int i = 0; i < size; i++)
-                deep[((size_t)(i / SW_WAVES) * 8 + x) * SW_WAVES + i % SW_WAVES] = deep_rm[start + i];
-        }
-    }
-    std::stable_sort(base.begin(), base.end(), [&](int a, int b) { return cls[a] > cls[b]; });
-    c->order_h = base;
-    c->cls_h = cls;
-    c->bdeep_h = deep_rm;
-    drop_graphs(c);  // the captured step sequences hold the old tables and grid sizes
-    const int cap = std::max({n_strips, strip_rows * (S / G) * nseg, (int)deep.size()});
-    if (c->list_cap < cap) {
-        void *ptrs[] = {c->order, c->deep, c->gen, c->fb_list};
-        for (void *p : ptrs)
-            dev_free(p);
-        c->order = c->deep = c->gen = c->fb_list = nullptr;
-        HIPCHK(dev_alloc(&c->order, (size_t)cap * sizeof(int)));
-        HIPCHK(dev_alloc(&c->deep, (size_t)cap * sizeof(int)));
-        HIPCHK(dev_alloc(&c->gen, (size_t)cap * sizeof(int)));
-        HIPCHK(dev_alloc(&c->fb_list, (size_t)3 * cap * sizeof(int)));
-        c->list_cap = cap;
-    }
-    if (!c->fb_count) HIPCHK(dev_alloc(&c->fb_count, 3 * sizeof(unsigned int)));
-    HIPCHK(ctx_fill(ctx, c->fb_count, 3 * sizeof(unsigned int)));
-    c->n_order = n_tiles;
-    c->n_deep = (int)deep.size();
-    c->n_gen = (int)gen.size();
-    HIPCHK(ctx_copy(ctx, c->order, base.data(), base.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!deep.empty()) HIPCHK(ctx_copy(ctx, c->deep, deep.data(), deep.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!gen.empty()) HIPCHK(ctx_copy(ctx, c->gen, gen.data(), gen.size() * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(ctx_copy(ctx, dst, v.data(), v.size() * sizeof(int2), hipMemcpyHostToDevice));
     return THY_OK;
 }
 
-// rebuild the dispatch order from the depth on the device (after a strip-height change)
+size_t segment_rows(const thy_ctx *c) { return (size_t)((c->nx + SW_OUT - 1) / SW_OUT) * c->ny; }
+
+// Coast along the row sweep's 56-column segments.  A segment row is coastal when any cell of
+// its 64 columns is shallower than 3 hpos (or dry).  Its cost is an estimate of the faces
+// that will not take the deep form: those of the wet cells shallower than hpos and of the
+// cells on either side of a shoreline.
 template <typename T>
-int rebuild_order_t(thy_ctx *ctx) {
-    std::vector<T> D((size_t)ctx->pitch * ctx->ny);
-    HIPCHK(ctx_copy(ctx, D.data(), ctx->D, D.size() * sizeof(T), hipMemcpyDeviceToHost));
-    return build_order<T>(ctx, D.data());
+void find_coast(thy_ctx *c, const T *D) {
+    const int nx = c->nx, ny = c->ny, P = c->pitch;
+    const int nseg = (nx + SW_OUT - 1) / SW_OUT;
+    const T thr = (T)(3.0 * c->prm.hpos), hpos = (T)c->prm.hpos;
+    c->coastal.assign((size_t)nseg * (ny + 1), 0);
+    c->cost.assign((size_t)nseg * (ny + 1), 0);
+    for (int j = 0; j < ny; j++) {
+        for (int sgi = 0; sgi < nseg; sgi++) {
+            const int xa = std::max(0, sgi * SW_OUT - SW_HALO), xb = std::min(nx, sgi * SW_OUT + SW_OUT + SW_HALO);
+            const T *d = D + (size_t)j * P;
+            bool any = false;
+            for (int i = xa; i < xb && !any; i++) any = d[i] <= thr;
+            int n = 0;
+            for (int i = xa; any && i < xb; i++) {
+                const bool dry = d[i] <= T(0);
+                n += (!dry && d[i] <= hpos) || (i > xa && dry != (d[i - 1] <= T(0)));
+            }
+            const size_t k = (size_t)sgi * (ny + 1) + j;
+            c->coastal[k + 1] = c->coastal[k] + (any ? 1 : 0);
+            c->cost[k + 1] = c->cost[k] + std::min(SW_OUT, 3 * n);
+        }
+    }
+}
+
+// Work lists with deep-water strips of up to S rows and tiles of up to R rows.  Each
+// segment's column is cut into blocks of 8 rows between the border bands; a block is deep
+// when its rows y0-4 .. y1+3 and its 64 columns are clear of the grid edges (no clamping,
+// no first-order band), of the sponges, and of coast.  Runs of deep blocks become strips of
+// nearly equal height, the rest tiles, in order of their cost.
+int build_lists(thy_ctx *ctx, WorkLists &w, int S, const int R) {
+    const int nx = ctx->nx, ny = ctx->ny;
+    const int nseg = (nx + SW_OUT - 1) / SW_OUT;
+    const int spi = ctx->prm.sponge_izq, spd = ctx->prm.sponge_der, sps = ctx->prm.sponge_sup, spn = ctx->prm.sponge_inf;
+    S = std::min(S, 2047);
+    auto between = [&](const std::vector<int> &v, const int sgi, const int y0, const int y1) {
+        const int *row = &v[(size_t)sgi * (ny + 1)];
+        return row[std::min(ny, y1)] - row[std::max(0, y0)];
+    };
+    const int ya = std::max(6, sps + 2), yb = ny - std::max(6, spn + 2);  // rows a deep block may take
+    std::vector<int2> strips;
+    std::vector<std::pair<int, int2>> tiles;  // (cost, tile)
+    auto add_tiles = [&](const int sgi, const int y0, const int y1) {
+        for (int y = y0; y < y1; y += R) {
+            const int n = std::min(R, y1 - y);
+            tiles.emplace_back(between(ctx->cost, sgi, y - 2, y + n + 2), make_int2(sgi * SW_OUT, y << 4 | n));
+        }
+    };
+    for (int sgi = 0; sgi < nseg; sgi++) {
+        const int x0 = sgi * SW_OUT;
+        const bool xok = ctx->kernel == 0 && x0 - SW_HALO >= 2 && x0 + SW_OUT + SW_HALO - 1 <= nx - 3 &&
+                         x0 - SW_HALO >= spi && x0 + SW_OUT + SW_HALO - 1 < nx - spd;
+        int y = 0;  // rows before y are dealt
+        for (int b = ya; xok && b < yb;) {
+            int e = b;  // the run of deep blocks from row b
+            while (e < yb && between(ctx->coastal, sgi, e - 4, std::min(e + 8, yb) + 4) == 0) e = std::min(e + 8, yb);
+            if (e == b) {
+                b += 8;
+                continue;
+            }
+            add_tiles(sgi, y, b);
+            const int n = (e - b + S - 1) / S;
+            for (int k = 0; k < n; k++) {
+                const int s0 = b + (int)((int64_t)(e - b) * k / n), s1 = b + (int)((int64_t)(e - b) * (k + 1) / n);
+                strips.push_back(make_int2(x0, s0 << 11 | (s1 - s0)));
+            }
+            y = b = e;
+        }
+        add_tiles(sgi, y, ny);
+    }
+    // neighbouring strips side by side, in rows
+    std::stable_sort(strips.begin(), strips.end(), [](const int2 &p, const int2 &q) { return (p.y >> 11) < (q.y >> 11); });
+    std::stable_sort(tiles.begin(), tiles.end(), [](const auto &p, const auto &q) { return p.first > q.first; });
+    w.tile_h.clear();
+    w.tcost_h.clear();
+    for (const auto &t : tiles) {
+        w.tile_h.push_back(t.second);
+        w.tcost_h.push_back(t.first);
+    }
+    const std::vector<int2> deep = xcd_runs(strips, SW_WAVES);
+    const std::vector<int2> items = interleave(w.tile_h, (int)deep.size() / SW_WAVES, S);
+    int r;
+    if ((r = put_list(ctx, w.deep, w.deep_cap, deep)) != THY_OK || (r = put_list(ctx, w.items, w.items_cap, items)) != THY_OK)
+        return r;
+    w.n_deep = (int)deep.size();
+    w.n_items = (int)items.size();
+    return THY_OK;
+}
+
+// the lists of a run alone, with deep-water strips of S rows and tiles of R rows
+int build_alone(thy_ctx *ctx, const int S, const int R) {
+    if (ctx->kernel == 1) return THY_OK;
+    drop_graphs(ctx);  // the captured step sequences hold the old lists and grid sizes
+    ctx->srows = S;
+    ctx->trows = R;
+    // where the default is the shortest strip, taller ones only leave the device idle
+    const int def = default_strip_rows(segment_rows(ctx), ctx->ncu);
+    return build_lists(ctx, ctx->alone, def <= 8 ? std::min(S, def) : S, R);
+}
+
+// the lists of an uploaded state
+template <typename T>
+int build_order(thy_ctx *ctx, const T *D) {
+    if (ctx->kernel == 1) return THY_OK;
+    find_coast(ctx, D);
+    ctx->uploaded = true;
+    ctx->batched.n_items = 0;  // built again when a batch asks for them
+    const size_t rows = segment_rows(ctx);
+    return build_alone(ctx, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : default_strip_rows(rows, ctx->ncu),
+                       ctx->prm.general_rows > 0 ? std::min(ctx->prm.general_rows, kTileRows) : default_tile_rows(rows, ctx->ncu));
+}
+
+// The lists a batch steps the scenario by.  Its scenarios fill the device whatever their
+// grids: tiles are whole, and strips of 16 rows cost the least (24 scenarios of 1000x800:
+// 128.6 / 123.0 / 126.4 / 126.4 / 133.3 ms at 8 / 16 / 24 / 32 / 48 rows).
+int build_batched(thy_ctx *ctx) {
+    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 16, kTileRows);
 }
 
 template <typename T>
@@ -737,7 +674,6 @@ int clear_dt_slots(thy_ctx *ctx, const int s) {
 int reset_dt_slots(thy_ctx *ctx) {
     int r;
     if ((r = clear_dt_slots(ctx, -1)) != THY_OK) return r;
-    if (ctx->fb_count) HIPCHK(ctx_fill(ctx, ctx->fb_count, 3 * sizeof(unsigned int)));
     return THY_OK;
 }
 
@@ -1130,8 +1066,6 @@ int thy_create(const thy_grid *g, const thy_params *p, thy_ctx **out) {
     }
     HIPCHK(hipEventCreate(&ctx->ev0));
     HIPCHK(hipEventCreate(&ctx->ev1));
-    HIPCHK(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming));
     for (int i = 0; i < 2; i++) {
         HIPCHK(hipEventCreate(&ctx->rev[i][0]));
         HIPCHK(hipEventCreate(&ctx->rev[i][1]));
@@ -1209,13 +1143,11 @@ void thy_destroy(thy_ctx *ctx) {
     drop_graphs(ctx);
     void *ptrs[] = {ctx->state, ctx->row, ctx->fy, ctx->area_d, ctx->ctrl, ctx->dtmin, ctx->scratch_u,
                     ctx->ftime, ctx->gpos, ctx->gbuf, ctx->gtime, ctx->okada_def, ctx->mass_partial, ctx->outbuf,
-                    ctx->steplog, ctx->order, ctx->deep, ctx->gen, ctx->fb_count, ctx->fb_list, ctx->health};
+                    ctx->steplog, ctx->alone.deep, ctx->alone.items, ctx->batched.deep, ctx->batched.items, ctx->health};
     for (void *q : ptrs)
         dev_free(q);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
-    if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
-    if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     for (int i = 0; i < 2; i++)
         for (int j = 0; j < 3; j++)
             if (ctx->rev[i][j]) (void)hipEventDestroy(ctx->rev[i][j]);
@@ -1269,7 +1201,7 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
     RelaxedCapture relaxed;
     if (!ctx) return THY_ERR_INVALID;
     if (ctx->kernel == 1) return fail(ctx, THY_ERR_INVALID, "autotune covers the row-sweep kernel");
-    if (ctx->order_h.empty()) return fail(ctx, THY_ERR_INVALID, "autotune needs an uploaded state");
+    if (!ctx->uploaded) return fail(ctx, THY_ERR_INVALID, "autotune needs an uploaded state");
     if (reps <= 0) reps = 5;
     int r;
     // the run's control blocks and dt slots are restored afterwards
@@ -1286,22 +1218,18 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
     c.dt = dt;
     c.dt_valid = 1;
     c.cur = ctx->cur;
-    // (strip rows, general strip rows)
-    const int cand[][2] = {{16, 4}, {16, 8}, {24, 4}, {24, 8}, {24, 12}, {32, 8}, {32, 16}, {36, 18}, {40, 20}, {48, 16}};
-    int best = ctx->srows, best_g = ctx->grows_req;
+    // (strip rows, tile rows)
+    const int cand[][2] = {{16, 4}, {16, 8}, {24, 8}, {32, 8}, {36, 8}, {40, 8}, {48, 8}};
+    int best = ctx->srows, best_g = ctx->trows;
     double best_ms = 1e30;
     for (const auto &sg : cand) {
         const int S = sg[0];
         if (S > ctx->ny && S != cand[0][0]) continue;
-        ctx->srows = S;
-        ctx->grows_req = sg[1];
-        r = ctx->prec ? rebuild_order_t<double>(ctx) : rebuild_order_t<float>(ctx);
-        if (r != THY_OK) return r;
+        if ((r = build_alone(ctx, S, sg[1])) != THY_OK) return r;
         // kSeq steps captured into one graph and replayed, as a run replays its steps.
-        // The launches cycle through the three launch slots as in a run (so each step's
-        // hand-back list starts empty), but publish no control block: every slot holds
-        // the same control block, each step reads the same state and redoes the same
-        // step, and the run's state stays.
+        // The launches cycle through the three launch slots as in a run, but publish no
+        // control block: every slot holds the same control block, each step reads the
+        // same state and redoes the same step, and the run's state stays.
         constexpr int kSeq = 32;  // long enough that the replay launch is a small share
         hipGraph_t g = nullptr;
         hipGraphExec_t ge = nullptr;
@@ -1326,8 +1254,7 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
         const Ctrl c3[3] = {c, c, c};
         for (int k = 0; k <= reps; k++) {  // the first replay is a warm-up
             hipError_t e = hipSuccess;
-            if ((e = ctx_copy(ctx, ctx->ctrl, c3, sizeof(c3), hipMemcpyHostToDevice)) == hipSuccess && ctx->fb_count)
-                e = ctx_fill(ctx, ctx->fb_count, 3 * sizeof(unsigned int));
+            e = ctx_copy(ctx, ctx->ctrl, c3, sizeof(c3), hipMemcpyHostToDevice);
             if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
             if (e == hipSuccess) e = hipGraphLaunch(ge, ctx->stream);
             if (e == hipSuccess) e = hipEventRecord(ctx->ev1, ctx->stream);
@@ -1349,17 +1276,12 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
             best_g = sg[1];
         }
     }
-    ctx->srows = best;
-    ctx->grows_req = best_g;
-    r = ctx->prec ? rebuild_order_t<double>(ctx) : rebuild_order_t<float>(ctx);
-    if (r != THY_OK) return r;
+    if ((r = build_alone(ctx, best, best_g)) != THY_OK) return r;
     ctx->slot = saved_slot;
     HIPCHK(ctx_copy(ctx, ctx->ctrl, saved, sizeof(saved), hipMemcpyHostToDevice));
     HIPCHK(ctx_copy(ctx, ctx->dtmin, saved_dt.data(), saved_dt.size() * sizeof(unsigned int), hipMemcpyHostToDevice));
-    // the hand-back counts as a run leaves them between steps (the next launch resets its own)
-    if (ctx->fb_count) HIPCHK(ctx_fill(ctx, ctx->fb_count, 3 * sizeof(unsigned int)));
     if (strip_rows) *strip_rows = best;
-    if (general_rows) *general_rows = ctx->gsrows;
+    if (general_rows) *general_rows = ctx->trows;
     if (ms_best) *ms_best = best_ms;
     return THY_OK;
 }
@@ -1375,7 +1297,6 @@ int thy_step(thy_ctx *ctx, double dt, double *dt_next) {
     if ((r = write_ctrl(ctx, c)) != THY_OK) return r;
     const int s = ctx->slot;
     if ((r = clear_dt_slots(ctx, s)) != THY_OK) return r;
-    if (ctx->fb_count) HIPCHK(ctx_fill(ctx, &ctx->fb_count[s], sizeof(unsigned int)));
     hipError_t e = launch_step(ctx);
     if (e != hipSuccess) return fail(ctx, THY_ERR_HIP, std::string("step launch: ") + hipGetErrorString(e));
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1658,16 +1579,15 @@ int thy_run_more(thy_ctx *ctx, int64_t n_steps, thy_run_result *res) {
 }  // extern "C"
 
 // ===========================================================================
-// Batched scenarios: many contexts advanced together, three launches per step (the
-// deep-water strips of every scenario, the general strips beside them on a second
-// stream, then the hand-backs), captured once for K steps.
+// Batched scenarios: many contexts advanced together, one launch per step, captured once
+// for K steps.
 // ===========================================================================
 struct thy_batch {
     int capacity = 0;
     size_t budget = 0, used = 0;
     int K = 24;
     hipStream_t stream = nullptr, side = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_fork = nullptr, ev_join = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_done = nullptr;   // end of a launch's work (admissions queue copies after it)
     std::vector<thy_ctx *> ctx;     // per slot; nullptr when free
     std::vector<size_t> bytes;      // admitted footprint per slot
@@ -1675,16 +1595,11 @@ struct thy_batch {
     std::vector<int> state;         // THY_SLOT_*
     std::vector<thy_run_result> res;
     StepArgs<float> *d_args = nullptr;
-    // item lists (scenario slot, strip << 1 | writer) and their device counts; the
-    // captured grids cover deep_cap and gen_cap items
-    int2 *d_deep = nullptr, *d_gen = nullptr, *d_fb = nullptr;
-    int *d_counts = nullptr;        // [0] deep items, [1] general items
-    unsigned int *d_fb_count = nullptr;
-    int deep_cap = 0, gen_cap = 0;
-    int gen_sub = 0;                // general items are gsrows-row sub-strips
-    std::vector<int2> h_deep, h_gen;
-    int h_counts[2] = {0, 0};
-    int fb_grid = 1;
+    BatchItem *d_items = nullptr;   // a workgroup's work each; the captured grid covers item_cap
+    int *d_count = nullptr;         // items in the list
+    int item_cap = 0;
+    std::vector<BatchItem> h_items;
+    int h_count = 0;
     Ctrl *d_ctrl = nullptr;
     Ctrl *h_ctrl = nullptr;              // pinned: control blocks gathered after a launch
     StepArgs<float> *h_args = nullptr;   // pinned: argument blocks of admitted scenarios
@@ -1719,117 +1634,68 @@ int list_cap(size_t n) {
     return c;
 }
 
-// Item lists of the running scenarios: every deep-water strip, scenario by scenario in
-// its own order (neighbouring strips stay together); every general strip, costliest
-// cost class first.  A scenario's writer is its first deep-water strip, or its first
-// general strip when it has none.  With few general strips in all (a launch bound by
-// the time one wavefront takes for one strip rather than by the number of strips) the
-// general strips are cut into sub-strips of each scenario's gsrows rows, as in a run
-// alone.
+// The workgroups of the running scenarios: every general tile, costliest cost class first,
+// then the deep-water strips, scenario by scenario, four to a workgroup in the scenario's
+// own order (its runs per XCD: each scenario starts at a multiple of 8).  A scenario's
+// writer is its first item.
 int batch_items(thy_batch *b) {
-    struct G { int cls; int2 it; };
+    struct G { int cls; BatchItem it; };
     std::vector<G> gv;
-    b->h_deep.clear();
-    size_t n_full = 0;
-    for (int i = 0; i < b->capacity; i++)
-        if (b->state[i] == THY_SLOT_RUNNING) n_full += b->ctx[i]->bgen_h.size();
-    const int sub = n_full < (size_t)8 * b->fb_grid ? 1 : 0;
+    b->h_items.clear();
     for (int i = 0; i < b->capacity; i++) {
         if (b->state[i] != THY_SLOT_RUNNING) continue;
         const thy_ctx *c = b->ctx[i];
-        // the strip lists must describe the strips of the argument block
+        // the lists must be those of the argument block
         if (c->srows != b->srows[i]) return bfail(b, THY_ERR_INVALID, "strip height changed after admission");
-        const bool nd = c->bdeep_h.empty();
-        for (size_t p = 0; p < c->bdeep_h.size(); p++)
-            b->h_deep.push_back(make_int2(i, (c->bdeep_h[p] << 1) | (p == 0 ? 1 : 0)));
-        const std::vector<int> &gl = sub ? c->bsub_h : c->bgen_h, &gc = sub ? c->bsubcls_h : c->bgcls_h;
-        for (size_t p = 0; p < gl.size(); p++)
-            gv.push_back({gc[p], make_int2(i, (gl[p] << 1) | (nd && p == 0 ? 1 : 0))});
-    }
-    // the deep-water items as in a run alone (build_order): row-major, scenario by
-    // scenario, cut into 8 runs of (nearly) equal length, one per XCD, padded to whole
-    // workgroups with idle items (scenario -1), so that each XCD sweeps one band and
-    // strips side by side share their halo columns in its L2
-    if (!b->h_deep.empty()) {
-        const std::vector<int2> rm = b->h_deep;
-        const int nd = (int)rm.size(), q = nd / 8, rem = nd % 8;
-        const int wmax = (q + (rem > 0 ? 1 : 0) + SW_WAVES - 1) / SW_WAVES;
-        b->h_deep.assign((size_t)wmax * 8 * SW_WAVES, make_int2(-1, 0));
-        for (int x = 0; x < 8; x++) {
-            const int size = q + (x < rem ? 1 : 0), start = x * q + std::min(x, rem);
-            for (int i = 0; i < size; i++)
-                b->h_deep[((size_t)(i / SW_WAVES) * 8 + x) * SW_WAVES + i % SW_WAVES] = rm[start + i];
-        }
+        const WorkLists &w = c->batched;
+        for (size_t p = 0; p < w.tile_h.size(); p++)
+            gv.push_back({w.tcost_h[p], BatchItem{i, p == 0 ? 1 : 0, w.tile_h[p]}});
     }
     std::stable_sort(gv.begin(), gv.end(), [](const G &x, const G &y) { return x.cls > y.cls; });
-    b->h_gen.resize(gv.size());
-    for (size_t k = 0; k < gv.size(); k++) b->h_gen[k] = gv[k].it;
-    const int dc = list_cap(b->h_deep.size()), gc = list_cap(b->h_gen.size());
-    if (sub != b->gen_sub && b->gexec) {  // captured with the other strip height
-        (void)hipGraphExecDestroy(b->gexec);
-        b->gexec = nullptr;
+    for (const G &g : gv) b->h_items.push_back(g.it);
+    for (int i = 0; i < b->capacity; i++) {
+        if (b->state[i] != THY_SLOT_RUNNING) continue;
+        const WorkLists &w = b->ctx[i]->batched;
+        if (w.n_deep > 0)
+            while (b->h_items.size() % 8) b->h_items.push_back(BatchItem{-1, 0, make_int2(0, 0)});
+        for (int p = 0; p < w.n_deep; p += SW_WAVES)
+            b->h_items.push_back(BatchItem{i, (p == 0 && w.tile_h.empty()) ? 1 : 0, make_int2(p, 0)});
     }
-    b->gen_sub = sub;
-    if (dc != b->deep_cap || gc != b->gen_cap) {
-        // the captured launches hold the old lists and grid sizes
+    const int cap = list_cap(b->h_items.size());
+    if (cap != b->item_cap) {
+        // the captured launches hold the old list and grid size
         if (b->gexec) {
             (void)hipGraphExecDestroy(b->gexec);
             b->gexec = nullptr;
         }
-        void *ptrs[] = {b->d_deep, b->d_gen, b->d_fb};
-        for (void *q : ptrs)
-            dev_free(q);
-        b->d_deep = b->d_gen = b->d_fb = nullptr;
-        b->deep_cap = b->gen_cap = 0;
-        BHIPCHK(dev_alloc(&b->d_deep, (size_t)dc * sizeof(int2)));
-        BHIPCHK(dev_alloc(&b->d_gen, (size_t)gc * sizeof(int2)));
-        BHIPCHK(dev_alloc(&b->d_fb, (size_t)3 * dc * sizeof(int2)));
-        b->deep_cap = dc;
-        b->gen_cap = gc;
+        dev_free(b->d_items);
+        b->d_items = nullptr;
+        b->item_cap = 0;
+        BHIPCHK(dev_alloc(&b->d_items, (size_t)cap * sizeof(BatchItem)));
+        b->item_cap = cap;
     }
-    b->h_counts[0] = (int)b->h_deep.size();
-    b->h_counts[1] = (int)b->h_gen.size();
-    // ordered before the next launch on the batch stream; the host lists live in b
-    if (!b->h_deep.empty())
-        BHIPCHK(hipMemcpyAsync(b->d_deep, b->h_deep.data(), b->h_deep.size() * sizeof(int2), hipMemcpyHostToDevice,
+    b->h_count = (int)b->h_items.size();
+    // ordered before the next launch on the batch stream; the host list lives in b
+    if (!b->h_items.empty())
+        BHIPCHK(hipMemcpyAsync(b->d_items, b->h_items.data(), b->h_items.size() * sizeof(BatchItem), hipMemcpyHostToDevice,
                                b->stream));
-    if (!b->h_gen.empty())
-        BHIPCHK(hipMemcpyAsync(b->d_gen, b->h_gen.data(), b->h_gen.size() * sizeof(int2), hipMemcpyHostToDevice,
-                               b->stream));
-    BHIPCHK(hipMemcpyAsync(b->d_counts, b->h_counts, sizeof(b->h_counts), hipMemcpyHostToDevice, b->stream));
+    BHIPCHK(hipMemcpyAsync(b->d_count, &b->h_count, sizeof(int), hipMemcpyHostToDevice, b->stream));
     BHIPCHK(hipStreamSynchronize(b->stream));
     b->dirty = false;
     return THY_OK;
 }
 
-// K steps (launch slots 0, 1, 2, ...), captured once: per step the deep-water launch on
-// the batch stream, the general launch beside it on the side stream, and after both
-// the hand-back launch
+// K steps (launch slots 0, 1, 2, ...), captured once, one launch each
 int batch_graph(thy_batch *b) {
     if (b->gexec) return THY_OK;
     BatchArgs q;
     q.args = b->d_args;
-    q.deep = b->d_deep;
-    q.n_deep = b->d_counts;
-    q.gen = b->d_gen;
-    q.n_gen = b->d_counts + 1;
-    q.fb_list = b->d_fb;
-    q.fb_count = b->d_fb_count;
-    q.fb_cap = b->deep_cap;
-    q.gen_sub = b->gen_sub;
-    const dim3 blk(64 * SW_WAVES);
+    q.items = b->d_items;
+    q.n_items = b->d_count;
     hipGraph_t g;
     BHIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < b->K; k++) {
-        const int slot = k % 3;
-        BHIPCHK(hipEventRecord(b->ev_fork, b->stream));
-        BHIPCHK(hipStreamWaitEvent(b->side, b->ev_fork, 0));
-        hipLaunchKernelGGL(k_batch_general<false>, dim3(b->gen_cap / SW_WAVES), blk, 0, b->side, q, slot);
-        BHIPCHK(hipEventRecord(b->ev_join, b->side));
-        hipLaunchKernelGGL(k_batch_deep, dim3(b->deep_cap / SW_WAVES), blk, 0, b->stream, q, slot);
-        BHIPCHK(hipStreamWaitEvent(b->stream, b->ev_join, 0));
-        hipLaunchKernelGGL(k_batch_general<true>, dim3(b->fb_grid), blk, 0, b->stream, q, slot);
-    }
+    for (int k = 0; k < b->K; k++)
+        hipLaunchKernelGGL(k_batch, dim3(b->item_cap), dim3(64 * SW_WAVES), 0, b->stream, q, k % 3);
     BHIPCHK(hipStreamEndCapture(b->stream, &g));
     BHIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
     (void)hipGraphDestroy(g);
@@ -1866,8 +1732,9 @@ int prepare_for_batch(thy_ctx *ctx, const thy_run_config *cfg, thy_run_result &r
     if (ctx->prec != 0 || ctx->kernel == 1)
         return fail(ctx, THY_ERR_INVALID, "batched scenarios run the FP32 row-sweep kernel only");
     if (cfg->save_interval >= 0.0) return fail(ctx, THY_ERR_INVALID, "batched scenarios take no snapshots");
-    if (ctx->order_h.empty()) return fail(ctx, THY_ERR_INVALID, "scenario state not uploaded");
+    if (!ctx->uploaded) return fail(ctx, THY_ERR_INVALID, "scenario state not uploaded");
     int r;
+    if (ctx->batched.n_items == 0 && (r = build_batched(ctx)) != THY_OK) return r;
     if ((r = prepare_run(ctx, cfg, &res)) != THY_OK) return r;
     Ctrl cb;
     if ((r = read_ctrl(ctx, &cb)) != THY_OK) return r;
@@ -1895,27 +1762,18 @@ int thy_batch_create(int capacity, size_t hbm_budget, int steps_per_sync, thy_ba
     b->res.assign(capacity, thy_run_result{});
     b->launched.assign(capacity, 0);
     // cached streams: creating and destroying streams with every batch would shift how
-    // the runtime spreads streams over the hardware queues, and the two launches of a
-    // step only overlap when the pair sits on two different queues
+    // the runtime spreads streams over the hardware queues
     BHIPCHK(Pool::get().get_streams(b->stream, b->side));
     BHIPCHK(hipEventCreate(&b->ev0));
     BHIPCHK(hipEventCreate(&b->ev1));
-    BHIPCHK(hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
-    BHIPCHK(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
     BHIPCHK(hipEventCreateWithFlags(&b->ev_done, hipEventDisableTiming));
     BHIPCHK(dev_alloc(&b->d_args, (size_t)capacity * sizeof(StepArgs<float>)));
     BHIPCHK(hipMemsetAsync(b->d_args, 0, (size_t)capacity * sizeof(StepArgs<float>), b->stream));
-    BHIPCHK(dev_alloc(&b->d_counts, 2 * sizeof(int)));
-    BHIPCHK(hipMemsetAsync(b->d_counts, 0, 2 * sizeof(int), b->stream));
-    BHIPCHK(dev_alloc(&b->d_fb_count, 3 * sizeof(unsigned int)));
-    BHIPCHK(hipMemsetAsync(b->d_fb_count, 0, 3 * sizeof(unsigned int), b->stream));
+    BHIPCHK(dev_alloc(&b->d_count, sizeof(int)));
+    BHIPCHK(hipMemsetAsync(b->d_count, 0, sizeof(int), b->stream));
     BHIPCHK(dev_alloc(&b->d_ctrl, (size_t)capacity * sizeof(Ctrl)));
     BHIPCHK(Pool::get().host_alloc((void **)&b->h_ctrl, (size_t)capacity * sizeof(Ctrl)));
     BHIPCHK(Pool::get().host_alloc((void **)&b->h_args, (size_t)capacity * sizeof(StepArgs<float>)));
-    int dev = 0, ncu = 0;
-    BHIPCHK(hipGetDevice(&dev));
-    BHIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    b->fb_grid = std::max(1, ncu);
     return THY_OK;
 }
 
@@ -1927,10 +1785,10 @@ void thy_batch_destroy(thy_batch *b) {
     Pool::get().host_free(b->h_ctrl);
     Pool::get().host_free(b->h_args);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
-    void *ptrs[] = {b->d_args, b->d_deep, b->d_gen, b->d_fb, b->d_counts, b->d_fb_count, b->d_ctrl};
+    void *ptrs[] = {b->d_args, b->d_items, b->d_count, b->d_ctrl};
     for (void *p : ptrs)
         dev_free(p);
-    hipEvent_t evs[] = {b->ev0, b->ev1, b->ev_fork, b->ev_join, b->ev_done};
+    hipEvent_t evs[] = {b->ev0, b->ev1, b->ev_done};
     for (hipEvent_t e : evs)
         if (e) (void)hipEventDestroy(e);
     if (b->stream) Pool::get().put_streams(b->stream, b->side);
@@ -1969,12 +1827,12 @@ int thy_batch_add(thy_batch *b, thy_ctx *ctx, const thy_run_config *cfg, int *sl
     }
     ctx->batch_ready = false;
     ctx->ctrl_h_valid = false;  // the batch's launches advance its control blocks
-    const StepArgs<float> a = make_args<float>(ctx);
+    const StepArgs<float> a = make_args<float>(ctx, true);
     // ordered after a launch in flight, which does not read this free slot
     b->h_args[slot] = a;
     BHIPCHK(hipMemcpyAsync(b->d_args + slot, b->h_args + slot, sizeof(a), hipMemcpyHostToDevice, b->stream));
     b->ctx[slot] = ctx;
-    b->srows[slot] = a.srows;
+    b->srows[slot] = ctx->srows;
     b->bytes[slot] = need;
     b->used += need;
     b->state[slot] = THY_SLOT_RUNNING;

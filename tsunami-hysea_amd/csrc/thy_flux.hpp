@@ -157,14 +157,11 @@ template <typename T> __device__ __forceinline__ T orient(int border, const Prm<
 // g0/g1: 1/cos(phi_row) for x faces (both sides), cos0/cos1 for y faces; k0/k1: the
 // positivity factors g A / 4 of the two rows (A / 4 for x faces).
 // ---------------------------------------------------------------------------
-template <typename T, bool YFACE>
-__device__ __forceinline__ T mass_flux(SC<T> m, SC<T> a, SC<T> b, SC<T> q, int border, bool alfa_cero,
-                                       T len, T g0, T g1, T k0, T k1, T valf, T dt, const Prm<T> &p) {
-    // deep branch (2s): all four depths above hpos and outside the first-order band
-    if (!alfa_cero && m.h > p.hpos && a.h > p.hpos && b.h > p.hpos && q.h > p.hpos) {
-        T F = a.qn * (len * g0);
-        return positivity(F, a.h, b.h, k0, k1, dt);
-    }
+// mass_waf: every branch but the deep-water one.  YFACE may vary from lane to lane: an x face
+// is the y form with g0 = g1 = 1 (every product with them is exact).
+template <typename T>
+__device__ __forceinline__ T mass_waf(const bool yface, SC<T> m, SC<T> a, SC<T> b, SC<T> q, int border, bool alfa_cero,
+                                      T len, T g0, T g1, T k0, T k1, T valf, T dt, const Prm<T> &p) {
     T normal = orient(border, p, m, a, b, q);
     if (border == 1) { T t = g0; g0 = g1; g1 = t; t = k0; k0 = k1; k1 = t; }
     if (!(a.h > Num<T>::eps || b.h > Num<T>::eps)) return T(0);
@@ -195,20 +192,24 @@ __device__ __forceinline__ T mass_flux(SC<T> m, SC<T> a, SC<T> b, SC<T> q, int b
     } else {
         a0 = lmax;
     }
-    T F2s, Fw;
-    if (YFACE) {
-        F2s = len * q0 * g0 * normal;
-        T deta = Num<T>::mad(-(uij * uij), g1 - g0, T(0.5) * (g0 + g1) * deta_of(a.e, b.e, a.D, b.D));
-        Fw = T(0.5) * Num<T>::mad(-a0, deta, Num<T>::mad(q0, g0, q1 * g1)) * len;
-    } else {
-        T il = len * g0;
-        F2s = il * q0 * normal;
-        T deta = deta_of(a.e, b.e, a.D, b.D);
-        Fw = T(0.5) * Num<T>::mad(-a0, deta, q1 + q0) * il;
-    }
+    T F2s = len * q0 * g0 * normal;
+    T deta = deta_of(a.e, b.e, a.D, b.D);
+    if (yface) deta = Num<T>::mad(-(uij * uij), g1 - g0, T(0.5) * (g0 + g1) * deta);
+    T Fw = T(0.5) * Num<T>::mad(-a0, deta, Num<T>::mad(q0, g0, q1 * g1)) * len;
     T alfa = blend(hij, p.hpos, alfa_cero);
     T F = Num<T>::mad(alfa, F2s, (T(1) - alfa) * Fw);
     return positivity(F, a.h, b.h, k0, k1, dt);
+}
+
+template <typename T, bool YFACE>
+__device__ __forceinline__ T mass_flux(SC<T> m, SC<T> a, SC<T> b, SC<T> q, int border, bool alfa_cero,
+                                       T len, T g0, T g1, T k0, T k1, T valf, T dt, const Prm<T> &p) {
+    // deep branch (2s): all four depths above hpos and outside the first-order band
+    if (!alfa_cero && m.h > p.hpos && a.h > p.hpos && b.h > p.hpos && q.h > p.hpos) {
+        T F = a.qn * (len * g0);
+        return positivity(F, a.h, b.h, k0, k1, dt);
+    }
+    return mass_waf<T>(YFACE, m, a, b, q, border, alfa_cero, len, g0, g1, k0, k1, valf, dt, p);
 }
 
 // Momentum face result: low cell acc2 -= (mn, mt), high cell acc2 -= (pn, pt),
@@ -224,12 +225,120 @@ template <typename T> struct MF {
 // For y faces: g0 = cos0, g1 = cos1 with ic0 = 1/cos0, ic1 = 1/cos1 (the row table's
 // values, shared with the deep-water forms), qn = qy, qt = qx.
 // ---------------------------------------------------------------------------
+// mom_waf: every branch but the deep-water one; as mass_waf, an x face is the y form with
+// g0 = g1 = ic0 = ic1 = 1 where the two forms do not differ by more.
+template <typename T>
+__device__ __forceinline__ MF<T> mom_waf(const bool yface, SC<T> m, SC<T> a, SC<T> b, SC<T> q, int border, bool alfa_cero,
+                                         T len, T g0, T g1, T ic0, T ic1, T valf, T dt, const Prm<T> &p) {
+    MF<T> o;
+    T normal = orient(border, p, m, a, b, q);
+    if (border == 1) {
+        T t = g0; g0 = g1; g1 = t;
+        t = ic0; ic0 = ic1; ic1 = t;
+    }
+    if (!(a.h > Num<T>::eps || b.h > Num<T>::eps)) {
+        o.mn = o.mt = o.pn = o.pt = o.w = T(0);
+        return o;
+    }
+    const T L = len;   // face length factor (len/cos for x)
+    T h0 = a.h, h1 = b.h;
+    T q0 = a.qn * normal, q1 = b.qn * normal;
+    T hij = T(0.5) * (h0 + h1);
+    wet_dry(a, b, p.eps_h, q0, q1);
+    T f0 = a.f, f1 = b.f;
+    T u0 = f0 * q0, u1 = f1 * q1;
+    if (!yface) { q0 = u0 * h0; q1 = u1 * h1; }
+    T s0 = Num<T>::sqrt(h0), s1 = Num<T>::sqrt(h1);
+    T uij = Num<T>::div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
+    T val = valf * dt;
+    T c0 = Num<T>::sqrt(hij);
+    T l1 = tmin(uij - c0, u0 - s0);
+    T l2 = tmax(uij + c0, u1 + s1);
+    T lmax = tmax(tabs(l2), tabs(l1));
+    T deta = deta_of(a.e, b.e, a.D, b.D);
+    T fl0x, fl0y, fl1x, fl1y;
+    if (yface) deta = Num<T>::mad(-(uij * uij), g1 - g0, T(0.5) * (g0 + g1) * deta);
+    fl1x = q1 * g1; fl1y = u1 * fl1x;
+    fl0x = q0 * g0; fl0y = u0 * fl0x;
+    T dq = fl1x - fl0x;
+    // 2s part (s: normal momentum, z: tangential)
+    bool up = uij < T(0);
+    T sm_n, sp_n, sm_t, sp_t;
+    {
+        T uu = up ? u1 : u0;
+        T qq = up ? q1 : q0;
+        T qt = up ? b.qt : a.qt;
+        T fn = uu * qq * L * normal;
+        if (up) { sp_n = -fn; sm_n = fn * (g1 * ic0); }
+        else { sm_n = fn; sp_n = -fn * g0 * ic1; }
+        sm_n += hij * deta * L * ic0;
+        T ft = uu * qt * L;
+        sm_t = ft;
+        sp_t = -ft;
+        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::div(p.hpos, hij)))));
+        T des = cd * val * lmax * lmax * dq * L;
+        if (!yface) des *= normal;
+        sm_n -= des * ic0;
+        sp_n += des * ic1;
+    }
+    // WAF part
+    T xiL = T(0), xiR = T(0);
+    if (!alfa_cero) {
+        xiL = limiter(m.e, a.e, b.e, q.e, l1);
+        xiR = limiter(m.e, a.e, b.e, q.e, l2);
+    }
+    T a0, a1;
+    if (tabs(l1 - l2) >= Num<T>::eps) {
+        T alr = Num<T>::mad(val * l1, xiL, sgn(l1) * (T(1) - xiL));
+        T blr = Num<T>::mad(val * l2, xiR, sgn(l2) * (T(1) - xiR));
+        T aux = Num<T>::rcp(l2 - l1);
+        a0 = (alr - blr) * (l1 * l2) * aux;
+        a1 = Num<T>::mad(blr, l2, -(alr * l1)) * aux;
+    } else {
+        a0 = lmax;
+        a1 = T(0);
+    }
+    T wy = T(0.5) * Num<T>::mad(hij, deta, fl1y - fl0y);
+    T DESx = T(0.5) * a0 * deta;
+    T DESy = Num<T>::mad(a1, wy, T(0.5) * a0 * dq);
+    T mxw = Num<T>::mad(T(0.5), dq, fl0x - DESx) * L;
+    T myw = (wy + (fl0y - DESy)) * L;
+    T pyw = (wy + (DESy - fl1y)) * L;
+    // limited upwinding of the tangential velocity
+    const T tsign = yface ? T(-1) : T(1);
+    T q0mt = tsign * m.qt * normal, q0t = tsign * a.qt * normal;
+    T q1t = tsign * b.qt * normal, q1pt = tsign * q.qt * normal;
+    T p0m = m.f * q0mt;
+    T p0 = f0 * q0t;
+    T p1 = f1 * q1t;
+    T p1p = q.f * q1pt;
+    T sgm = sgn(mxw);
+    T us = tabs(uij) * sgm;
+    T xi = alfa_cero ? T(0) : limiter(p0m, p0, p1, p1p, us);
+    T uijt;
+    const T wt = T(-0.5) * Num<T>::mad(xi * us, val, (T(1) - xi) * sgm);
+    uijt = Num<T>::mad(wt, Num<T>::mad(p1, ic1, -(p0 * ic0)), T(0.5) * Num<T>::mad(p0, ic0, p1 * ic1));
+    T aux = mxw * uijt;
+    T f3m_n, f3m_t, f3p_n, f3p_t;
+    f3m_t = tsign * aux * normal; f3m_n = myw * normal * ic0;
+    f3p_t = -f3m_t;               f3p_n = pyw * normal * ic1;
+    T alfa = blend(hij, p.hpos, alfa_cero);
+    T oma = T(1) - alfa;
+    o.mn = Num<T>::mad(alfa, sm_n, oma * f3m_n);
+    o.mt = Num<T>::mad(alfa, sm_t, oma * f3m_t);
+    o.pn = Num<T>::mad(alfa, sp_n, oma * f3p_n);
+    o.pt = Num<T>::mad(alfa, sp_t, oma * f3p_t);
+    if (lmax < p.eps_h) lmax += p.eps_h;
+    o.w = L * lmax;
+    return o;
+}
+
 template <typename T, bool YFACE>
 __device__ __forceinline__ MF<T> mom_flux(SC<T> m, SC<T> a, SC<T> b, SC<T> q, int border, bool alfa_cero,
                                           T len, T g0, T g1, T ic0, T ic1, T valf, T kdes, T dt, const Prm<T> &p) {
-    MF<T> o;
     if (!alfa_cero && m.h > p.hpos && a.h > p.hpos && b.h > p.hpos && q.h > p.hpos) {
         // deep-water 2s branch
+        MF<T> o;
         T hij = T(0.5) * (a.h + b.h);
         T ia = Num<T>::rcp(a.h), ib = Num<T>::rcp(b.h);
         T u0 = a.qn * ia, u1 = b.qn * ib;
@@ -268,122 +377,8 @@ __device__ __forceinline__ MF<T> mom_flux(SC<T> m, SC<T> a, SC<T> b, SC<T> q, in
         }
         return o;
     }
-    T normal = orient(border, p, m, a, b, q);
-    if (border == 1) {
-        T t = g0; g0 = g1; g1 = t;
-        t = ic0; ic0 = ic1; ic1 = t;
-    }
-    if (!(a.h > Num<T>::eps || b.h > Num<T>::eps)) {
-        o.mn = o.mt = o.pn = o.pt = o.w = T(0);
-        return o;
-    }
-    if (!YFACE) ic0 = ic1 = T(1);
-    T L = YFACE ? len : len * g0;   // face length factor (len/cos for x)
-    T h0 = a.h, h1 = b.h;
-    T q0 = a.qn * normal, q1 = b.qn * normal;
-    T hij = T(0.5) * (h0 + h1);
-    wet_dry(a, b, p.eps_h, q0, q1);
-    T f0 = a.f, f1 = b.f;
-    T u0 = f0 * q0, u1 = f1 * q1;
-    if (!YFACE) { q0 = u0 * h0; q1 = u1 * h1; }
-    T s0 = Num<T>::sqrt(h0), s1 = Num<T>::sqrt(h1);
-    T uij = Num<T>::div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
-    T val = valf * dt;
-    T c0 = Num<T>::sqrt(hij);
-    T l1 = tmin(uij - c0, u0 - s0);
-    T l2 = tmax(uij + c0, u1 + s1);
-    T lmax = tmax(tabs(l2), tabs(l1));
-    T deta = deta_of(a.e, b.e, a.D, b.D);
-    T fl0x, fl0y, fl1x, fl1y;
-    if (YFACE) {
-        deta = Num<T>::mad(-(uij * uij), g1 - g0, T(0.5) * (g0 + g1) * deta);
-        fl1x = q1 * g1; fl1y = u1 * fl1x;
-        fl0x = q0 * g0; fl0y = u0 * fl0x;
-    } else {
-        fl1x = q1; fl1y = u1 * q1;
-        fl0x = q0; fl0y = u0 * q0;
-    }
-    T dq = fl1x - fl0x;
-    // 2s part (s: normal momentum, z: tangential)
-    bool up = uij < T(0);
-    T sm_n, sp_n, sm_t, sp_t;
-    {
-        T uu = up ? u1 : u0;
-        T qq = up ? q1 : q0;
-        T qt = up ? b.qt : a.qt;
-        T fn = uu * qq * L * normal;
-        if (YFACE) {
-            if (up) { sp_n = -fn; sm_n = fn * (g1 * ic0); }
-            else { sm_n = fn; sp_n = -fn * g0 * ic1; }
-            sm_n += hij * deta * L * ic0;
-        } else {
-            sp_n = -fn;
-            sm_n = fn + hij * deta * L;
-        }
-        T ft = uu * qt * L;
-        sm_t = ft;
-        sp_t = -ft;
-        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::div(p.hpos, hij)))));
-        T des = cd * val * lmax * lmax * dq * L;
-        if (YFACE) { sm_n -= des * ic0; sp_n += des * ic1; }
-        else { des *= normal; sm_n -= des; sp_n += des; }
-    }
-    // WAF part
-    T xiL = T(0), xiR = T(0);
-    if (!alfa_cero) {
-        xiL = limiter(m.e, a.e, b.e, q.e, l1);
-        xiR = limiter(m.e, a.e, b.e, q.e, l2);
-    }
-    T a0, a1;
-    if (tabs(l1 - l2) >= Num<T>::eps) {
-        T alr = Num<T>::mad(val * l1, xiL, sgn(l1) * (T(1) - xiL));
-        T blr = Num<T>::mad(val * l2, xiR, sgn(l2) * (T(1) - xiR));
-        T aux = Num<T>::rcp(l2 - l1);
-        a0 = (alr - blr) * (l1 * l2) * aux;
-        a1 = Num<T>::mad(blr, l2, -(alr * l1)) * aux;
-    } else {
-        a0 = lmax;
-        a1 = T(0);
-    }
-    T wy = T(0.5) * Num<T>::mad(hij, deta, fl1y - fl0y);
-    T DESx = T(0.5) * a0 * deta;
-    T DESy = Num<T>::mad(a1, wy, T(0.5) * a0 * dq);
-    T mxw = Num<T>::mad(T(0.5), dq, fl0x - DESx) * L;
-    T myw = (wy + (fl0y - DESy)) * L;
-    T pyw = (wy + (DESy - fl1y)) * L;
-    // limited upwinding of the tangential velocity
-    T tsign = YFACE ? T(-1) : T(1);
-    T q0mt = tsign * m.qt * normal, q0t = tsign * a.qt * normal;
-    T q1t = tsign * b.qt * normal, q1pt = tsign * q.qt * normal;
-    T p0m = m.f * q0mt;
-    T p0 = f0 * q0t;
-    T p1 = f1 * q1t;
-    T p1p = q.f * q1pt;
-    T sgm = sgn(mxw);
-    T us = tabs(uij) * sgm;
-    T xi = alfa_cero ? T(0) : limiter(p0m, p0, p1, p1p, us);
-    T uijt;
-    const T wt = T(-0.5) * Num<T>::mad(xi * us, val, (T(1) - xi) * sgm);
-    if (YFACE) uijt = Num<T>::mad(wt, Num<T>::mad(p1, ic1, -(p0 * ic0)), T(0.5) * Num<T>::mad(p0, ic0, p1 * ic1));
-    else uijt = Num<T>::mad(wt, p1 - p0, T(0.5) * (p0 + p1));
-    T aux = mxw * uijt;
-    T f3m_n, f3m_t, f3p_n, f3p_t;
-    if (YFACE) {
-        f3p_t = aux * normal;  f3p_n = pyw * normal * ic1;
-        f3m_t = -aux * normal; f3m_n = myw * normal * ic0;
-    } else {
-        f3p_n = pyw * normal;  f3p_t = -aux * normal;
-        f3m_n = myw * normal;  f3m_t = aux * normal;
-    }
-    T alfa = blend(hij, p.hpos, alfa_cero);
-    T oma = T(1) - alfa;
-    o.mn = Num<T>::mad(alfa, sm_n, oma * f3m_n);
-    o.mt = Num<T>::mad(alfa, sm_t, oma * f3m_t);
-    o.pn = Num<T>::mad(alfa, sp_n, oma * f3p_n);
-    o.pt = Num<T>::mad(alfa, sp_t, oma * f3p_t);
-    if (lmax < p.eps_h) lmax += p.eps_h;
-    o.w = L * lmax;
-    return o;
+    if (!YFACE) return mom_waf<T>(false, m, a, b, q, border, alfa_cero, len * g0, T(1), T(1), T(1), T(1), valf, dt, p);
+    return mom_waf<T>(true, m, a, b, q, border, alfa_cero, len, g0, g1, ic0, ic1, valf, dt, p);
 }
 
 // Initial-dt wave speed across a face: src/GPU/Arista_kernel.cu:1237-1280

@@ -96,18 +96,9 @@ __host__ __device__ __forceinline__ int dt_at(const int slot, const int part) {
 template <typename T> struct StepArgs {
     int nx, ny, pitch, periodic;
     int tiles_x, tiles_y, n_tiles, chunk;  // chunk: tiles per XCD chunk (whole tile rows)
-    int srows;                             // row-sweep kernel: rows per strip
-    int gsrows;                            //   rows per general strip beside a deep-water launch
-    int yoff;                              //   split launches: strip row k covers rows k*rows-yoff ..
-    int nseg;                              // row-sweep kernel: 56-column segments per row
-    const int *order;                      // row-sweep kernel: every block, costliest first (or null)
-    int n_order;                           //   number of them
-    const int *deep;                       // deep-water strips (strip row * nseg + segment; null: no split)
-    int n_deep;
-    const int *gen;                        // general strips beside a deep-water launch, costliest first
-    int n_gen;
-    unsigned int *fb_count;                // 3 slots: strips the deep-water sweep hands back
-    int *fb_list;                          // [3][n_deep]
+    const int2 *items;                     // row-sweep kernel: work items of a step, one per workgroup (item_origin)
+    int n_items;
+    const int2 *deep;                      // deep-water strips (x0, y0 << 11 | rows), four to an item (x0 < 0: none)
     int sp_sup, sp_inf, sp_izq, sp_der;
     int track_arrival, n_gauges;
     T bsup, binf, bizq, bder;
@@ -193,11 +184,15 @@ template <typename T>
 __device__ __forceinline__ void begin_step(const StepArgs<T> &a, const int slot, const bool writer, BlockCtl<T> &bc,
                                            const int parts = 1) {
     Ctrl c = a.ctrl[slot];
-    // the health flag raised by the previous step's cells stops the run here
-    if (a.health && *a.health) c.nonfinite = 1;
-    int skip;
+    const unsigned int health = a.health ? *a.health : 0u;
     unsigned int raw = kDtNone;
     for (int p = 0; p < parts; p++) raw = min(raw, a.dtmin[dt_at((slot + 2) % 3, p)]);
+    // all of these loads are in flight together: each would otherwise be waited for before
+    // the next is issued (a memory latency at the head of every workgroup)
+    asm volatile("" : : "s"(health), "v"(raw));
+    // the health flag raised by the previous step's cells stops the run here
+    if (health) c.nonfinite = 1;
+    int skip;
     const double dt = step_dt(c, a.ftime, __uint_as_float(raw), skip);
     const bool stop = must_stop(c, a.ftime);
     const bool sample = !stop && (c.t >= c.next_series);

@@ -1,23 +1,18 @@
 // thy_sweep.hpp -- row-sweep step kernel of the Tsunami-HySEA scheme for gfx950.
 //
-// Same step as k_step (src/GPU/Timestep.cu:70-120 plus the metric update and the
-// gauge gather), organised for the CDNA execution model instead of 2D LDS tiles:
-//   * one wavefront owns 64 adjacent columns (56 output columns plus a 4-column halo
-//     on each side, the reach of the 2s+WAF stencil through the two passes) and walks
-//     a strip of rows from top to bottom;
-//   * each row flows through a register pipeline: load row r, mass x-faces of row r,
-//     mass y-face between rows r-2 and r-1, h* of row r-2, momentum x-faces of row
-//     r-2, momentum y-face between rows r-4 and r-3, cell update of row r-4;
-//   * x-neighbours come from adjacent lanes (cross-lane moves), y-neighbours from the
-//     previous rows kept in registers, so every face is evaluated exactly once and no
-//     LDS, barrier or halo re-load is needed inside a strip;
-//   * the row geometry is uniform across the wavefront (scalar loads) and each row is
-//     fetched one iteration before it is used;
-//   * each stage votes across the wavefront: when every lane's stencil is deeper than
-//     hpos and clear of the first-order band, the stage uses the deep-water 2s forms
-//     below; otherwise it uses the general per-face functions of k_step
-//     (thy_flux.hpp), with the same border, first-order band and clamped-stencil
-//     conventions.
+// Same step as k_step (src/GPU/Timestep.cu:70-120 plus the metric update and the gauge
+// gather) in one launch, organised for the CDNA execution model instead of 2D LDS tiles.
+// The grid is cut into segments of 56 columns, one lane each with a 4-column halo on either
+// side of the wavefront (the reach of the 2s+WAF stencil through the two passes), and each
+// segment into
+//   * deep-water strips: rows far from coast, borders and sponges.  One wavefront walks a
+//     strip from top to bottom; each row flows through a register pipeline, x-neighbours
+//     come from adjacent lanes, y-neighbours from the rows before, so every face is
+//     evaluated once, with no LDS tile, barrier or halo re-load inside the strip;
+//   * general tiles: everything else.  One workgroup evaluates up to 8 rows out of LDS, the
+//     deep-water faces in place and the others from a work list.
+// Both evaluate a face through the same functions with the same border, first-order band
+// and clamped-stencil conventions, so the cut changes no result.
 #pragma once
 #include "thy_step.hpp"
 
@@ -33,15 +28,13 @@ constexpr int SW_WAVES = 4;               // wavefronts per workgroup (side by s
 // unit this kernel saturates) to the flux arithmetic; DPP row moves were measured
 // slower here for that reason.
 template <typename T> __device__ __forceinline__ T from_left(T v) { return __shfl_up(v, 1, 64); }
-template <typename T> __device__ __forceinline__ T from_left2(T v) { return __shfl_up(v, 2, 64); }
 template <typename T> __device__ __forceinline__ T from_right(T v) { return __shfl_down(v, 1, 64); }
 
 // The same moves as VALU data-parallel-primitive moves across the whole wavefront
 // (wave_shr:1 / wave_shl:1; the lane without a source keeps its own value): a few cycles
-// of latency instead of an LDS round trip.  The general strips, whose wavefronts are few
-// and walk long dependency chains, use these; the deep-water strips keep the LDS moves,
-// which leave the VALU to their flux arithmetic.  (dpp_left2 differs from from_left2 only
-// in lane 1, which lies outside every output cell's stencil.)
+// of latency instead of an LDS round trip.  The general tiles, whose time is a chain of
+// latencies, use these; the deep-water strips keep the LDS moves, which leave the VALU to
+// their flux arithmetic.
 __device__ __forceinline__ int dpp_shr1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false); }
 __device__ __forceinline__ int dpp_shl1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false); }
 __device__ __forceinline__ float dpp_left(float v) { return __int_as_float(dpp_shr1(__float_as_int(v))); }
@@ -56,7 +49,6 @@ __device__ __forceinline__ double dpp_right(double v) {
     const int lo = dpp_shl1((int)(b & 0xffffffffll)), hi = dpp_shl1((int)(b >> 32));
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-template <typename T> __device__ __forceinline__ T dpp_left2(T v) { return dpp_left(dpp_left(v)); }
 
 // read-only table entry at a wavefront-uniform address (scalar load)
 template <typename S> __device__ __forceinline__ S uniform_load(const S *p) {
@@ -64,6 +56,17 @@ template <typename S> __device__ __forceinline__ S uniform_load(const S *p) {
     S out;
     __builtin_memcpy(&out, (const __attribute__((address_space(4))) S *)p, sizeof(S));
     return out;
+}
+
+// The argument block at a wavefront-uniform address, read again from here on.  The block's
+// fields are scalar loads that hit the scalar cache; without this the compiler loads each
+// once, at the top, and keeps it: the kernels below then hold some 120 scalars more than
+// there are registers, spilled to lanes of vector registers, and every phase starts with
+// dozens of lane reads (half of a tile's vector instructions).
+template <typename T> using ArgsAt = const __attribute__((address_space(4))) StepArgs<T> *;
+template <typename T> __device__ __forceinline__ const StepArgs<T> &again(ArgsAt<T> p) {
+    asm volatile("" : "+s"(p));
+    return *(const StepArgs<T> *)p;
 }
 
 // ---------------------------------------------------------------------------
@@ -199,8 +202,7 @@ __device__ __forceinline__ void buf_store<double>(double v, __amdgpu_buffer_rsrc
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, on ? voff : kDropOffset, soff, 0);
 }
 
-// a stencil cell with its desingularisation factor f (shared by the x faces of a lane
-// through lane moves) ...
+// a stencil cell with a given desingularisation factor f ...
 template <typename T> __device__ __forceinline__ SC<T> sc_of(T e, T D, T qn, T qt, T f) {
     SC<T> c;
     c.e = e;
@@ -211,361 +213,508 @@ template <typename T> __device__ __forceinline__ SC<T> sc_of(T e, T D, T qn, T q
     c.f = f;
     return c;
 }
-// ... or computed for this cell alone (the compiler drops it where no face uses it)
+// ... or with its own (the compiler drops it where no face uses it)
 template <typename T> __device__ __forceinline__ SC<T> sc_of(T e, T D, T qn, T qt, const Prm<T> &p) {
     return sc_of(e, D, qn, qt, desing(e + D, p.eps_h));
 }
 
-// One wavefront's share of a step: the strip of a.srows rows whose 56 output columns
-// start at x0 and whose first row is y0, with bc filled by begin_step for this launch.
-// Returns this lane's minimum of the per-cell dt of the next step (3e38 when it
-// updated no cell, or when x0 lies past the grid).
-// EDGE false: the caller guarantees a strip 8 cells or more inside the borders and their
-// sponges, not periodic (no clamping, border faces, first-order band or sponge).
-template <typename T, bool EDGE = true>
-__device__ __forceinline__ float sweep_strip(const StepArgs<T> &a, const BlockCtl<T> &bc, const int x0,
-                                             const int y0, const int rows) {
+// ---------------------------------------------------------------------------
+// General tiles: one workgroup per tile of 56 output columns and up to kTileRows rows.
+//
+// A shallow face costs several times a deep-water one (square roots, divisions,
+// exponentials, three limiters), and along a coast only one lane in four to one in twenty
+// of a wavefront's row holds one, so evaluating a row's faces in place runs the long code
+// mostly for idle lanes, row after row.  Here the rows of the tile and its halo lie in
+// LDS, every wavefront evaluates the deep-water forms of its rows in place, and the faces
+// that take any other branch are put on a work list (ballots of the depth tests combined
+// with scalar mask arithmetic, so the classification costs little vector work) that the
+// workgroup then evaluates with every lane busy, x and y faces together.  Once for the
+// mass pass, once for the momentum pass:
+//   load the rows, classify                        | barrier
+//   deep mass faces in place, list the others      | barrier
+//   listed mass faces                              | barrier
+//   h* (as e*) of rows y0-2 .. y0+m+1, classify    | barrier
+//   list the other momentum faces                  | barrier
+//   listed momentum faces                          | barrier
+//   deep momentum faces in place, cell updates
+// Which lane evaluates a face does not change its value, and per cell the accumulation
+// order is x faces, lower y face, upper y face in every tile and strip.
+// Everything a tile reads from memory (rows, row tables, metrics) is requested at once:
+// its time is a chain of latencies, and each later read would add one.
+// ---------------------------------------------------------------------------
+// 8 rows: taller tiles would have less halo (4 of 12 rows in the mass pass), but at 8 the
+// tile's LDS (31 KB in FP32) lets five workgroups share a CU, as their registers do.
+constexpr int kTileRows = 8;
+constexpr int kTileHalf = 3;  // rows whose momentum faces always fit the result table
+
+using mask64 = unsigned long long;
+
+template <typename T> struct alignas(16) FaceOut {
+    T mn, pn, mt, w;  // (pt = -mt)
+};
+
+template <typename T> struct TileLds {
+    static constexpr int G = kTileRows;
+    static constexpr int kFluxes = 2 * (G + 5) * 64;
+    static constexpr int kResults = kFluxes / 4;  // listed momentum faces at a time
+    static_assert(kResults >= kTileHalf * 57 + (kTileHalf + 1) * 56, "a round of kTileHalf rows fits");
+    T in[4][(G + 8) * 64];   // e, D, qx, qy of rows y0-4 .. y0+m+3
+    T es[(G + 4) * 64];      // e* of rows y0-2 .. y0+m+1
+    union {
+        T F[2][(G + 5) * 64];     // mass fluxes of the x faces (row, lane) and y faces
+        FaceOut<T> R[kResults];   // results of the listed momentum faces
+    };
+    RowGeo<T> row[G + 4];    // of rows y0-2 ..
+    FaceGeoY<T> fy[G + 5];   // of faces y0-2 ..
+    mask64 deep[G + 8], dry[G + 8];    // lanes deeper than hpos / dry (h <= eps), by row
+    mask64 sdeep[G + 4], sdry[G + 4];  // the same of h*
+    mask64 w[2][G + 1];                // listed momentum faces of an x row / a y face row
+    int base[2][G + 1];                //   and the place of the first of them
+    int count[2];                      // listed faces: mass, momentum
+    unsigned short list[(G + 4) * 61 + (G + 5) * 60];  // direction << 15 | row << 6 | lane
+};
+
+__device__ __forceinline__ bool lane_of(const mask64 m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+__device__ __forceinline__ int rank_of(const mask64 m) {  // set bits below this lane
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+__device__ __forceinline__ mask64 uniform_mask(const mask64 m) {
+    return ((mask64)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m);
+}
+// x faces (lane = the face's high cell) whose four cells / two cells are all in m
+__device__ __forceinline__ mask64 all4(const mask64 m) { return m & (m << 1) & (m << 2) & (m >> 1); }
+__device__ __forceinline__ mask64 both(const mask64 m) { return m & (m << 1); }
+
+// Columns x0 .. x0+55, rows y0 .. y0+m-1 (m <= kTileRows), with bc filled by begin_step for
+// this launch; every thread of the workgroup calls it.  Returns this lane's minimum of the
+// per-cell dt of the next step (3e38 when it updated no cell).
+template <typename T>
+__device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockCtl<T> &bc, const int x0, const int y0,
+                                              const int m, TileLds<T> &s) {
+    constexpr int G = kTileRows, W = SW_WAVES;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    // (selects rather than indexing, so that a copy of the arguments stays in registers)
-    const bool c1 = bc.cur != 0;
-    const T *__restrict__ ge = c1 ? a.e[1] : a.e[0];
-    const T *__restrict__ gqx = c1 ? a.qx[1] : a.qx[0];
-    const T *__restrict__ gqy = c1 ? a.qy[1] : a.qy[0];
-    const T *__restrict__ gD = a.D;
-    T *__restrict__ oe = c1 ? a.e[0] : a.e[1];
-    T *__restrict__ oqx = c1 ? a.qx[0] : a.qx[1];
-    T *__restrict__ oqy = c1 ? a.qy[0] : a.qy[1];
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T dt = (T)bc.dt;
-    const T tnow = (T)bc.t;
-    const int nx = a.nx, ny = a.ny, P = a.pitch;
-    const bool per = EDGE && a.periodic != 0;
-    const int y1 = min(y0 + rows, ny);
+    int nx, ny;
+    bool per;
     float dtmin = 3.0e38f;
     bool bad = false;
 
-    if (x0 < nx) {
-        const int gx = x0 - SW_HALO + lane;
-        // column loaded by this lane: wrapped (periodic) or clamped onto the grid
-        const int cx = !EDGE ? gx : (per ? ((gx % nx) + nx) % nx : (gx < 0 ? 0 : (gx >= nx ? nx - 1 : gx)));
-        // lanes outside the grid take the e* of the clamped column (clamped stencils)
-        const bool xedge = EDGE && !per && (x0 - SW_HALO < 0 || x0 + SW_OUT + SW_HALO > nx);
-        const int src = cx - (x0 - SW_HALO);
-        // this lane's x face is the left face of its cell: g = gx
-        const int xb = (!EDGE || per) ? 0 : (gx == 0 ? 1 : (gx == nx ? 2 : 0));
-        const int gw = per ? cx : gx;
-        const bool xac = EDGE && ((gw < 2) || (gw > nx - 2));
-        const bool out_col = lane >= SW_HALO && lane < SW_HALO + SW_OUT && (!EDGE || gx < nx);
-        const bool any_sponge = EDGE && (a.sp_izq | a.sp_der | a.sp_sup | a.sp_inf) != 0;
-        const int isp = per ? cx : gx;
-
-        Prm<T> px, py;
-        px.eps_h = py.eps_h = a.eps_h;
-        px.hpos = py.hpos = a.hpos;
-        px.cvis = py.cvis = a.cvis;
-        px.bl = a.bizq; px.bh = a.bder;
-        py.bl = a.bsup; py.bh = a.binf;
-
-        auto clamp_row = [&](int r) { return !EDGE ? r : (r < 0 ? 0 : (r >= ny ? ny - 1 : r)); };
-        auto clamp_face = [&](int g) { return !EDGE ? g : (g < 0 ? 0 : (g > ny ? ny : g)); };
-        // buffer loads: the row (clamped onto the grid) in the scalar offset, the lane's
-        // column in the vector offset; never predicated, so the compiler can keep the
-        // prefetches in flight across iterations
-        const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
-        const StateOffsets<T> o(a, ge, gD, gqx, gqy, oe, oqx, oqy);
-        // the loads carry each array's offset in the vector offset (one register per array,
-        // set once) and only the row in the scalar offset: this loop is short of scalar
-        // registers, not of vector ones
-        const int vcx = cx * (int)sizeof(T);
-        const int ve = vcx + o.e, vD = vcx + o.D, vqx = vcx + o.qx, vqy = vcx + o.qy;
-        auto load_row = [&](int r) {
-            const int so = clamp_row(r) * P * (int)sizeof(T);
-            RowCell<T> c;
-            c.e = buf_load<T>(rs, ve, so);
-            c.D = buf_load<T>(rs, vD, so);
-            c.qx = buf_load<T>(rs, vqx, so);
-            c.qy = buf_load<T>(rs, vqy, so);
-            return c;
-        };
-        const int vgx = (EDGE ? (gx < 0 ? 0 : (gx >= nx ? nx - 1 : gx)) : gx) * (int)sizeof(T);
-        const int vm = vgx + o.emax, va = vgx + o.arr;
-        auto load_metrics = [&](int jn, T &m, T &t) {
-            const int so = (jn < y0 ? y0 : (jn >= y1 ? y1 - 1 : jn)) * P * (int)sizeof(T);
-            m = buf_load<T>(rs, vm, so);
-            t = buf_load<T>(rs, va, so);
-        };
-
-        // the segment touches the first-order band of the x borders: no x face of it
-        // takes the deep form
-        const bool seg_ac = EDGE && __any(xac) != 0;
+    const int gx = x0 - SW_HALO + lane;
+    int cx;  // column loaded by this lane: wrapped (periodic) or clamped onto the grid
+    // ---- rows y0-4 .. y0+m+3, the row tables and the metrics of this wavefront's output
+    // rows ra .. rb-1 ----
+    constexpr int KR = (G + W - 1) / W, KL = (G + 8 + W - 1) / W;
+    const int kr = (m + W - 1) / W, ra = wv * kr, rb = min(ra + kr, m);
+    T pm[KR], pt[KR];
+    bool still;
+    {
+        const StepArgs<T> &a = again<T>(args);
+        nx = a.nx;
+        ny = a.ny;
+        per = a.periodic != 0;
         const T hpos = a.hpos;
-
-        // pipeline registers: input rows r-5..r, e* rows r-5..r-2 (with sqrt(h*) and
-        // qy/h* of rows r-4..r-2 for the deep y faces), mass accumulators rows
-        // r-2..r-1, momentum accumulators rows r-4..r-3, and per-row wavefront votes
-        // "every lane deeper than hpos" for the inputs (rows r-3..r) and h* (r-5..r-2)
-        // and "every lane dry" (h <= eps) for the inputs (rows r-2..r) and h* (r-4..r-2)
-        RowCell<T> i5, i4, i3, i2, i1, i0;
-        i5 = i4 = i3 = i2 = i1 = i0 = RowCell<T>{T(0), T(0), T(0), T(0)};
-        T s5 = T(0), s4 = T(0), s3 = T(0);
-        T sq4 = T(0), sq3 = T(0), v4 = T(0), v3 = T(0);
-        T m2 = T(0), m1 = T(0);
-        T X4 = T(0), Y4 = T(0), W4 = T(0), X3 = T(0), Y3 = T(0), W3 = T(0);
-        // the wavefront votes of the rows in the pipeline, one bit each in one word (one
-        // scalar register instead of one per vote): bit k of each byte is the vote of the
-        // k-th row back; byte 0 "deeper than hpos" (inputs, rows r..r-3), byte 1 "dry"
-        // (inputs, rows r..r-2), byte 2 "deeper than hpos" (h*, rows r-2..r-5), byte 3 "dry"
-        // (h*, rows r-2..r-4)
-        unsigned int votes = 0u;
-        // A face both of whose cells are dry (h <= eps) gets a zero flux from the face
-        // functions (src/GPU/Arista_kernel.cu:140,298); where every face of a stage is such
-        // a face (land), the stage uses those zeros without evaluating the faces.
-        constexpr T kZero = T(0);
-        const MF<T> kDryMF{kZero, kZero, kZero, kZero, kZero};
-        // One pipeline iteration for row r.  buf holds row r on entry and receives row
-        // r+1; (pm, pt) hold the metrics inputs of row r-4 on entry and receive those of
-        // row r-3: every load has one iteration of work behind it.  (Keeping loads two
-        // iterations ahead needs a two-way unrolled loop, whose register use costs more
-        // occupancy than the extra latency cover gains.)
-        auto iteration = [&](const int r, RowCell<T> &buf, T &pm, T &pt) {
-            i0 = buf;
-            buf = load_row(r + 1);
-            const int ju = r - 4;  // row updated in this iteration
-            const T cmax = pm, carr = pt;
-            load_metrics(ju + 1, pm, pt);
-            const T h0 = i0.e + i0.D;
-            const bool din0 = __all(h0 > hpos) != 0;
-            const bool dry0 = __all(!(h0 > Num<T>::eps)) != 0;
-            votes |= (din0 ? 0x1u : 0u) | (dry0 ? 0x100u : 0u);
-
-            // Stages run only for the rows and faces that some output row of the strip
-            // depends on (h* rows y0-2 .. y1+1, momentum faces of rows y0 .. y1-1 and
-            // y faces y0 .. y1); the halo iterations skip the rest.
-            // ---- mass x-faces of row r ----
-            T m0 = T(0);
-            if (r >= y0 - 2 && r <= y1 + 1) {
-                const RowGeo<T> rg = uniform_load(a.row + clamp_row(r));
-                if (din0 && !seg_ac) {
-                    const T F = fast_mass_x(dpp_left(i0.qx), dpp_left(h0), h0, rg.ilx, rg.kA, dt);
-                    m0 = F - dpp_right(F);
-                } else if (dry0) {
-                    m0 = ((xb == 1) ? -kZero : kZero) - kZero;
-                } else {
-                    const T eL = dpp_left(i0.e), DL = dpp_left(i0.D), qL = dpp_left(i0.qx);
-                    const T eLL = dpp_left2(i0.e), DLL = dpp_left2(i0.D);
-                    const T eR = dpp_right(i0.e), DR = dpp_right(i0.D);
-                    const T f0 = desing(h0, px.eps_h);  // the lane's cell, moved to its right neighbour
-                    const SC<T> M = sc_of(eLL, DLL, T(0), T(0), T(0)), A = sc_of(eL, DL, qL, T(0), dpp_left(f0));
-                    const SC<T> B = sc_of(i0.e, i0.D, i0.qx, T(0), f0), Q = sc_of(eR, DR, T(0), T(0), T(0));
-                    const T F = mass_flux<T, false>(M, A, B, Q, xb, xac, rg.ilx, T(1), T(1), rg.kA, rg.kA, rg.valx, dt, px);
-                    m0 = ((xb == 1) ? -F : F) - dpp_right(F);
+        cx = gx < 0 ? 0 : (gx >= nx ? nx - 1 : gx);
+        const int vgx = cx * (int)sizeof(T);
+        if (per) cx = ((gx % nx) + nx) % nx;
+        const int P = a.pitch;
+        const bool c1b = __builtin_amdgcn_readfirstlane(bc.cur) != 0;
+        const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
+        const StateOffsets<T> o(a, c1b ? a.e[1] : a.e[0], a.D, c1b ? a.qx[1] : a.qx[0], c1b ? a.qy[1] : a.qy[0], a.e[0],
+                                a.qx[0], a.qy[0]);
+        const int vcx = cx * (int)sizeof(T);
+        T v[KL][4];
+#pragma unroll
+        for (int t = 0; t < KL; t++) {
+            const int y = y0 - 4 + min(wv + t * W, m + 7), r = y < 0 ? 0 : (y >= ny ? ny - 1 : y);
+            const int so = r * P * (int)sizeof(T);
+            v[t][0] = buf_load<T>(rs, vcx + o.e, so);
+            v[t][1] = buf_load<T>(rs, vcx + o.D, so);
+            v[t][2] = buf_load<T>(rs, vcx + o.qx, so);
+            v[t][3] = buf_load<T>(rs, vcx + o.qy, so);
+        }
+        constexpr int NR = sizeof(RowGeo<T>) / sizeof(T), NF = sizeof(FaceGeoY<T>) / sizeof(T);
+        static_assert(NR * (G + 4) <= 64 * W && NF * (G + 5) <= 64 * W, "one table word per thread");
+        T tr = T(0), tf = T(0);
+        if (tid < NR * (G + 4)) {
+            const int y = y0 - 2 + tid / NR;
+            tr = ((const T *)a.row)[(y < 0 ? 0 : (y >= ny ? ny - 1 : y)) * NR + tid % NR];
+        }
+        if (tid < NF * (G + 5)) {
+            const int y = y0 - 2 + tid / NF;
+            tf = ((const T *)a.fy)[(y < 0 ? 0 : (y > ny ? ny : y)) * NF + tid % NF];
+        }
+#pragma unroll
+        for (int t = 0; t < KR; t++) {
+            const int so = (y0 + min(ra + t, m - 1)) * P * (int)sizeof(T);
+            pm[t] = buf_load<T>(rs, vgx + o.emax, so);
+            pt[t] = buf_load<T>(rs, vgx + o.arr, so);
+        }
+        // (rows beyond the tile's were loaded as its last one: no guard for `still`)
+        still = true;
+#pragma unroll
+        for (int t = 0; t < KL; t++) {
+            const int i = wv + t * W;
+            const T h = v[t][0] + v[t][1];
+            still = still && !(h > Num<T>::eps) && v[t][2] == T(0) && v[t][3] == T(0);
+            if (i < m + 8) {
+                const int p = i * 64 + lane;
+                s.in[0][p] = v[t][0];
+                s.in[1][p] = v[t][1];
+                s.in[2][p] = v[t][2];
+                s.in[3][p] = v[t][3];
+                const mask64 dp = __ballot(h > hpos), dr = __ballot(!(h > Num<T>::eps));
+                if (lane == 0) {
+                    s.deep[i] = dp;
+                    s.dry[i] = dr;
                 }
             }
-            // ---- mass y-face g = r-1 (rows r-3..r) ----
-            if (r - 1 >= y0 - 2 && r - 1 <= y1 + 2) {
-                const int g = r - 1;
-                const FaceGeoY<T> fg = uniform_load(a.fy + clamp_face(g));
-                const int yb = !EDGE ? 0 : (g == 0 ? 1 : (g == ny ? 2 : 0));
-                const bool yac = EDGE && ((g < 2) || (g > ny - 2));
-                T F;
-                if ((votes & 0xfu) == 0xfu && !yac) {
-                    F = fast_mass_y(i2.qy, i2.e + i2.D, i1.e + i1.D, fg, dt);
-                } else if ((votes & 0x600u) == 0x600u) {
-                    F = kZero;
-                } else {
-                    const SC<T> M = sc_of(i3.e, i3.D, T(0), T(0), T(0)), A = sc_of(i2.e, i2.D, i2.qy, T(0), py);
-                    const SC<T> B = sc_of(i1.e, i1.D, i1.qy, T(0), py), Q = sc_of(i0.e, i0.D, T(0), T(0), T(0));
-                    F = mass_flux<T, true>(M, A, B, Q, yb, yac, fg.len, fg.cos0, fg.cos1, fg.k0, fg.k1, fg.valy, dt, py);
-                }
-                m2 = Num<T>::mad(-F, fg.ic0, m2);
-                m1 = Num<T>::mad((yb == 1) ? -F : F, fg.ic1, m1);
-            }
-            // ---- h* (as e*) of row r-2, with the sponge ----
-            T s2;
-            const RowGeo<T> rg2 = uniform_load(a.row + clamp_row(r - 2));
-            const bool hrow = r - 2 >= y0 - 2 && r - 2 <= y1 + 1;  // h* of row r-2 is needed
-            if (hrow) {
-                T es = Num<T>::mad(dt * rg2.invA, m2, i2.e);
-                if (!(es + i2.D > T(0))) es = -i2.D;
-                if (any_sponge) es = sponge_eta(a, es, i2.D, isp, r - 2, rg2.dxs, rg2.dys);
-                if (xedge) es = __shfl(es, src, 64);
-                s2 = es;
-            } else {
-                s2 = i2.e;
-            }
-            const T hs2 = s2 + i2.D;
-            const bool ds2 = hrow && __all(hs2 > hpos) != 0;
-            const bool dsd2 = __all(!(hs2 > Num<T>::eps)) != 0;
-            votes |= (ds2 ? 0x10000u : 0u) | (dsd2 ? 0x1000000u : 0u);
-            T sq2 = T(0), u2 = T(0), v2 = T(0);
-            if (ds2) {
-                sq2 = Num<T>::sqrt(hs2);
-                const T ih = Num<T>::rcp(hs2);
-                u2 = i2.qx * ih;
-                v2 = i2.qy * ih;
-            }
-            // ---- momentum x-faces of row r-2 ----
-            T X2 = T(0), Y2 = T(0), W2 = T(0);
-            if (r - 2 < y0 || r - 2 >= y1) {
-                // halo row: no output row uses its x faces
-            } else if (ds2 && !seg_ac) {
-                DC<T> A, B;
-                A.h = dpp_left(hs2); A.e = dpp_left(s2); A.D = dpp_left(i2.D);
-                A.qn = dpp_left(i2.qx); A.qt = dpp_left(i2.qy); A.s = dpp_left(sq2); A.un = dpp_left(u2);
-                B.h = hs2; B.e = s2; B.D = i2.D; B.qn = i2.qx; B.qt = i2.qy; B.s = sq2; B.un = u2;
-                const MF<T> f = fast_mom_x(A, B, rg2.ilx, rg2.kdx, dt);
-                X2 = -f.pn - dpp_right(f.mn);
-                Y2 = -f.pt - dpp_right(f.mt);
-                W2 = f.w + dpp_right(f.w);
-            } else if (dsd2) {
-                const MF<T> &f = kDryMF;
-                X2 = -((xb == 1) ? f.mn : f.pn) - f.mn;
-                Y2 = -((xb == 1) ? f.mt : f.pt) - f.mt;
-                W2 = f.w + f.w;
-            } else {
-                const T eL = dpp_left(s2), DL = dpp_left(i2.D), qxL = dpp_left(i2.qx), qyL = dpp_left(i2.qy);
-                const T eLL = dpp_left2(s2), DLL = dpp_left2(i2.D), qyLL = dpp_left2(i2.qy);
-                const T eR = dpp_right(s2), DR = dpp_right(i2.D), qyR = dpp_right(i2.qy);
-                const T fs = desing(hs2, px.eps_h);  // the lane's cell, moved to its neighbours
-                const SC<T> M = sc_of(eLL, DLL, T(0), qyLL, dpp_left2(fs)), A = sc_of(eL, DL, qxL, qyL, dpp_left(fs));
-                const SC<T> B = sc_of(s2, i2.D, i2.qx, i2.qy, fs), Q = sc_of(eR, DR, T(0), qyR, dpp_right(fs));
-                const MF<T> f = mom_flux<T, false>(M, A, B, Q, xb, xac, rg2.ilx, T(1), T(1), T(1), T(1),
-                                                   rg2.valx, rg2.kdx, dt, px);
-                X2 = -((xb == 1) ? f.mn : f.pn) - dpp_right(f.mn);
-                Y2 = -((xb == 1) ? f.mt : f.pt) - dpp_right(f.mt);
-                W2 = f.w + dpp_right(f.w);
-            }
-            // ---- momentum y-face g = r-3 (rows r-5..r-2) ----
-            if (r - 3 >= y0 && r - 3 <= y1) {
-                const int g = r - 3;
-                const FaceGeoY<T> fg = uniform_load(a.fy + clamp_face(g));
-                const int yb = !EDGE ? 0 : (g == 0 ? 1 : (g == ny ? 2 : 0));
-                const bool yac = EDGE && ((g < 2) || (g > ny - 2));
-                MF<T> f;
-                if ((votes & 0xf0000u) == 0xf0000u && !yac) {
-                    DC<T> A, B;
-                    A.h = s4 + i4.D; A.e = s4; A.D = i4.D; A.qn = i4.qy; A.qt = i4.qx; A.s = sq4; A.un = v4;
-                    B.h = s3 + i3.D; B.e = s3; B.D = i3.D; B.qn = i3.qy; B.qt = i3.qx; B.s = sq3; B.un = v3;
-                    f = fast_mom_y(A, B, fg, dt);
-                } else if ((votes & 0x6000000u) == 0x6000000u && (!EDGE || (g - 1 >= 0 && g < ny))) {
-                    f = kDryMF;  // the face's cells are rows r-4 and r-3 (no clamping here)
-                } else {
-                    SC<T> M = sc_of(s5, i5.D, i5.qy, i5.qx, py), A = sc_of(s4, i4.D, i4.qy, i4.qx, py);
-                    SC<T> B = sc_of(s3, i3.D, i3.qy, i3.qx, py), Q = sc_of(s2, i2.D, i2.qy, i2.qx, py);
-                    // rows outside the grid take the e* of the edge row (clamped stencil)
-                    if (EDGE) {
-                        if (g - 2 < 0) M = (g - 1 < 0) ? B : A;
-                        if (g - 1 < 0) A = B;
-                        if (g >= ny) B = A;
-                        if (g + 1 >= ny) Q = (g >= ny) ? A : B;
-                    }
-                    f = mom_flux<T, true>(M, A, B, Q, yb, yac, fg.len, fg.cos0, fg.cos1, fg.ic0, fg.ic1, fg.valy,
-                                          fg.kdy, dt, py);
-                }
-                Y4 -= f.mn;
-                X4 -= f.mt;
-                W4 += f.w;
-                if (yb == 1) { Y3 -= f.mn; X3 -= f.mt; }
-                else { Y3 -= f.pn; X3 -= f.pt; }
-                W3 += f.w;
-            }
-            // ---- cell update of row r-4 (src/GPU/Volumen_kernel.cu:160-221) ----
-            // The arithmetic runs for output rows only; the five stores are issued in
-            // every iteration and dropped where they do not apply.
-            {
-                const bool row_on = ju >= y0 && ju < y1;
-                const bool on = row_on && out_col;
-                const int soff = (row_on ? ju : y0) * P * (int)sizeof(T);
-                const int voff = on ? gx * (int)sizeof(T) : kDropOffset;
-                const T eo = i4.e;
-                bool max_on = false, arr_on = false;
-                T qx = T(0), qy = T(0);
-                if (row_on) {
-                    const RowGeo<T> rg = uniform_load(a.row + ju);
-                    const T D = i4.D;
-                    // metrics from the state before the step (src/GPU/Metrics.cu:23-42,57-77)
-                    max_on = on && eo > cmax && eo + D > a.eps_h;
-                    arr_on = on && a.track_arrival && !Arrival<T>::arrived(carr) && tabs(eo - carr) > a.dif_at;
-                    const T dtc = (W4 < Num<T>::eps) ? Num<T>::big : Num<T>::div(T(2) * a.cfl * rg.A, W4);
-                    dtmin = fminf(dtmin, (float)dtc);  // halo lanes are dropped after the loop
-                    const T val = dt * rg.invA;
-                    qx = Num<T>::mad(val, X4, i4.qx);
-                    qy = Num<T>::mad(val, Y4, i4.qy);
-                    if (any_sponge) sponge_q(a, gx, ju, qx, qy);
-                    const T hs = s4 + D;
-                    if (hs <= hpos) near_dry(hs, i4.qx, i4.qy, qx, qy, dt, a.mf0, a.vmax, a.eps_h);
-                    bad = bad || (on && bad_cell(s4, qx, qy));
-                }
-                buf_store<T>(eo, rs, voff, o.emax + soff, max_on);
+        }
+        if (tid < NR * (G + 4)) ((T *)s.row)[tid] = tr;
+        if (tid < NF * (G + 5)) ((T *)s.fy)[tid] = tf;
+        if (tid < 2) s.count[tid] = 0;
+    }
+    // lanes outside the grid take the e* of the clamped column (clamped stencils)
+    const bool xedge = !per && (x0 - SW_HALO < 0 || x0 + SW_OUT + SW_HALO > nx);
+    // this lane's x face is the left face of its cell: g = gx
+    const bool low_border = !per && gx == 0;
+    const bool out_col = lane >= SW_HALO && lane < SW_HALO + SW_OUT && gx < nx;
+    // lanes whose x face / cell lies on the grid, and x faces of the first-order band
+    const mask64 on_face = __ballot(per || (gx >= 0 && gx <= nx)), on_cell = __ballot(per || (gx >= 0 && gx < nx));
+    const int gw = per ? cx : gx;
+    const mask64 first = __ballot(gw < 2 || gw > nx - 2);
+    const T *const e_ = s.in[0], *const D_ = s.in[1], *const qx_ = s.in[2], *const qy_ = s.in[3];
+    // Land: every cell of the tile and its halo dry and without discharge, clear of the
+    // sponges.  Every face is then zero and the update leaves e (its depth stays 0) and
+    // zero discharges; the arrival rule may still record the start (a dry cell's eta_ini
+    // is a marker).
+    if (__syncthreads_and(still)) {
+        const StepArgs<T> &a = again<T>(args);
+        if (a.eps_h >= Num<T>::eps && x0 - SW_HALO >= a.sp_izq && x0 + SW_OUT + SW_HALO <= nx - a.sp_der && y0 - 2 >= a.sp_sup &&
+            y0 + m + 2 <= ny - a.sp_inf) {
+            const T tnow = (T)bc.t;
+            const int P = a.pitch;
+            const bool c1b = __builtin_amdgcn_readfirstlane(bc.cur) != 0;
+            const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
+            const StateOffsets<T> o(a, a.e[0], a.D, a.qx[0], a.qy[0], c1b ? a.e[0] : a.e[1], c1b ? a.qx[0] : a.qx[1],
+                                    c1b ? a.qy[0] : a.qy[1]);
+            const int voff = out_col ? gx * (int)sizeof(T) : kDropOffset;
+            for (int f = ra; f < rb; f++) {
+                const int p = (f + 4) * 64 + lane, soff = (y0 + f) * P * (int)sizeof(T);
+                const T eo = e_[p], D = D_[p];
+                T carr = pt[0];
+#pragma unroll
+                for (int t = 1; t < KR; t++) carr = f - ra == t ? pt[t] : carr;
+                const bool arr_on = out_col && a.track_arrival && !Arrival<T>::arrived(carr) && tabs(eo - carr) > a.dif_at;
                 buf_store<T>(Arrival<T>::enc(tnow), rs, voff, o.arr + soff, arr_on);
-                buf_store<T>(s4, rs, voff, o.oe + soff, on);
-                buf_store<T>(qx, rs, voff, o.oqx + soff, on);
-                buf_store<T>(qy, rs, voff, o.oqy + soff, on);
+                buf_store<T>(eo + D > T(0) ? eo : -D, rs, voff, o.oe + soff, out_col);
+                buf_store<T>(T(0), rs, voff, o.oqx + soff, out_col);
+                buf_store<T>(T(0), rs, voff, o.oqy + soff, out_col);
             }
-            // ---- advance the pipeline ----
-            i5 = i4; i4 = i3; i3 = i2; i2 = i1; i1 = i0;
-            s5 = s4; s4 = s3; s3 = s2;
-            sq4 = sq3; sq3 = sq2; v4 = v3; v3 = v2;
-            m2 = m1; m1 = m0;
-            X4 = X3; Y4 = Y3; W4 = W3;
-            X3 = X2; Y3 = Y2; W3 = W2;
-            votes = (votes << 1) & 0x060e060eu;  // the bits of rows that stay in the pipeline
-        };
-
-        // rows y0-4 .. y1+3
-        const int rbeg = y0 - 4, rend = y1 + 3;
-        RowCell<T> buf = load_row(rbeg);
-        T pm, pt;
-        load_metrics(rbeg - 4, pm, pt);
-        // enter the loop with nothing outstanding, so that the wait at its head only
-        // accounts for the previous iteration (see kDropOffset)
-        __builtin_amdgcn_s_waitcnt(0);
-        for (int r = rbeg; r <= rend; r++) iteration(r, buf, pm, pt);
-        dtmin = out_col ? dtmin : 3.0e38f;
+            return out_col ? (float)Num<T>::big : 3.0e38f;
+        }
     }
-    raise_health(a, bad);
-    return dtmin;
-}
-
-// The workgroup's four wavefronts on strip block `tile` (side by side in x).
-template <typename T>
-__device__ __forceinline__ float sweep_block(const StepArgs<T> &a, const BlockCtl<T> &bc, const int tile,
-                                             const bool gauges) {
-    if (gauges) {
-        const bool c1 = bc.cur != 0;
-        gather_gauges(a, bc, c1 ? a.e[1] : a.e[0], c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], threadIdx.x,
-                      64 * SW_WAVES);
+    // ---- mass pass: x faces of rows y0-2+j, y faces g = y0-2+j ----
+    for (int j = wv; j < m + 5; j += W) {
+        const int y = y0 - 2 + j;
+        const int p = (j + 2) * 64 + lane;
+        const T h = e_[p] + D_[p];
+        mask64 wx = 0, wy = 0;
+        if (j < m + 4 && y >= 0 && y < ny) {
+            const mask64 dp = all4(uniform_mask(s.deep[j + 2])) & ~first;
+            T F = T(0);
+            if (dp) {
+                F = fast_mass_x(qx_[p - 1], e_[p - 1] + D_[p - 1], h, s.row[j].ilx, s.row[j].kA, dt);
+                F = lane_of(dp) ? F : T(0);
+            }
+            s.F[0][j * 64 + lane] = F;
+            wx = ~dp & ~both(uniform_mask(s.dry[j + 2])) & on_face & 0x7ffffffffffffffcull;  // lanes 2 .. 62
+        }
+        if (y >= 0 && y <= ny) {
+            const bool yac = y < 2 || y > ny - 2;
+            const mask64 dp = yac ? 0ull : uniform_mask(s.deep[j] & s.deep[j + 1] & s.deep[j + 2] & s.deep[j + 3]);
+            T F = T(0);
+            if (dp) {
+                F = fast_mass_y(qy_[p - 64], e_[p - 64] + D_[p - 64], h, s.fy[j], dt);
+                F = lane_of(dp) ? F : T(0);
+            }
+            s.F[1][j * 64 + lane] = F;
+            wy = ~dp & ~uniform_mask(s.dry[j + 1] & s.dry[j + 2]) & on_cell & 0x3ffffffffffffffcull;  // lanes 2 .. 61
+        }
+        const int cw = __popcll(wx), c = cw + __popcll(wy);
+        if (c) {
+            int b = 0;
+            if (lane == 0) b = atomicAdd(&s.count[0], c);
+            b = __builtin_amdgcn_readfirstlane(b);
+            if (lane_of(wx)) s.list[b + rank_of(wx)] = (unsigned short)(j << 6 | lane);
+            if (lane_of(wy)) s.list[b + cw + rank_of(wy)] = (unsigned short)(0x8000 | j << 6 | lane);
+        }
     }
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tyi = tile / a.tiles_x, txi = tile - tyi * a.tiles_x;
-    return sweep_strip(a, bc, (txi * SW_WAVES + wv) * SW_OUT, tyi * a.srows, a.srows);
+    __syncthreads();
+    // the constants of a listed face
+    struct Listed {
+        Prm<T> p;
+        T L, g0, g1, k0, k1, val, ic0, ic1;
+        int border;
+        bool yf, band;
+    };
+    auto listed = [&](const StepArgs<T> &a, const int code, const int j) {  // j: row of the tables
+        Listed f;
+        f.yf = (code & 0x8000) != 0;
+        const int l = code & 63;
+        const int g = f.yf ? y0 - 2 + j : x0 - SW_HALO + l, ng = f.yf ? ny : nx;
+        int gp = g;
+        if (per && !f.yf) gp = ((g % nx) + nx) % nx;
+        f.border = (per && !f.yf) ? 0 : (g == 0 ? 1 : (g == ng ? 2 : 0));
+        f.band = gp < 2 || gp > ng - 2;
+        f.p.eps_h = a.eps_h;
+        f.p.hpos = a.hpos;
+        f.p.cvis = a.cvis;
+        f.p.bl = f.yf ? a.bsup : a.bizq;
+        f.p.bh = f.yf ? a.binf : a.bder;
+        if (f.yf) {
+            const FaceGeoY<T> &q = s.fy[j];
+            f.L = q.len; f.g0 = q.cos0; f.g1 = q.cos1; f.k0 = q.k0; f.k1 = q.k1; f.val = q.valy; f.ic0 = q.ic0; f.ic1 = q.ic1;
+        } else {
+            const RowGeo<T> &q = s.row[j];
+            f.L = q.ilx; f.k0 = f.k1 = q.kA; f.val = q.valx;
+            f.g0 = f.g1 = f.ic0 = f.ic1 = T(1);
+        }
+        return f;
+    };
+    // ---- listed mass faces ----
+    const int nm = __builtin_amdgcn_readfirstlane(s.count[0]);
+    if (nm) {
+        const StepArgs<T> &a = again<T>(args);
+        for (int k = tid; k < nm; k += 64 * W) {
+            const int code = s.list[k], l = code & 63, j = (code >> 6) & 31;
+            const Listed f = listed(a, code, j);
+            const int p = (j + 2) * 64 + l, st = f.yf ? 64 : 1;
+            const T *const qn = f.yf ? qy_ : qx_;
+            const SC<T> M = sc_of(e_[p - 2 * st], D_[p - 2 * st], T(0), T(0), T(0));
+            const SC<T> A = sc_of(e_[p - st], D_[p - st], qn[p - st], T(0), f.p), B = sc_of(e_[p], D_[p], qn[p], T(0), f.p);
+            const SC<T> Q = sc_of(e_[p + st], D_[p + st], T(0), T(0), T(0));
+            s.F[f.yf ? 1 : 0][j * 64 + l] = mass_waf<T>(f.yf, M, A, B, Q, f.border, f.band, f.L, f.g0, f.g1, f.k0, f.k1,
+                                                        f.val, dt, f.p);
+        }
+        __syncthreads();
+    }
+    // ---- h* (as e*) of rows y0-2 .. y0+m+1, with the sponge ----
+    const StepArgs<T> &ah = again<T>(args);
+    for (int j = wv; j < m + 4; j += W) {
+        const int y = y0 - 2 + j;
+        if (y < 0 || y >= ny) continue;
+        const int q = j * 64 + lane, p = q + 128;
+        const T FL = s.F[0][q], FR = s.F[0][j * 64 + min(lane + 1, 63)], FB = s.F[1][q], FT = s.F[1][q + 64];
+        const T D = D_[p];
+        T acc = (low_border ? -FL : FL) - FR;
+        acc = Num<T>::mad(y == 0 ? -FB : FB, s.fy[j].ic1, acc);
+        acc = Num<T>::mad(-FT, s.fy[j + 1].ic0, acc);
+        T es = Num<T>::mad(dt * s.row[j].invA, acc, e_[p]);
+        if (!(es + D > T(0))) es = -D;
+        if (x0 - SW_HALO < ah.sp_izq || x0 + SW_OUT + SW_HALO > nx - ah.sp_der || y < ah.sp_sup || y >= ny - ah.sp_inf)
+            es = sponge_eta(ah, es, D, per ? cx : gx, y, s.row[j].dxs, s.row[j].dys);
+        if (xedge) es = __shfl(es, cx - (x0 - SW_HALO), 64);
+        s.es[q] = es;
+        const T h = es + D;
+        const mask64 dp = __ballot(h > ah.hpos), dr = __ballot(!(h > Num<T>::eps));
+        if (lane == 0) {
+            s.sdeep[j] = dp;
+            s.sdry[j] = dr;
+        }
+    }
+    __syncthreads();
+    // rows outside the grid stand for the edge row (clamped stencils)
+    const int jlo = max(0, 2 - y0), jhi = min(m + 3, ny + 1 - y0);
+    auto row_j = [&](const int j) { return min(max(j, jlo), jhi); };
+    // ---- momentum pass, rows y0+r0 .. y0+r1-1 at a time: the whole tile, or kTileHalf rows
+    // when its listed faces do not fit the result table ----
+    for (int r0 = 0, r1 = m; r0 < m;) {
+        // list the faces that do not take the deep form: x faces of rows y0+f, y faces g = y0+f
+        for (int f = r0 + wv; f <= r1; f += W) {
+            const int g = y0 + f;
+            mask64 wx = 0;
+            if (f < r1) {
+                const mask64 dp = all4(uniform_mask(s.sdeep[f + 2])) & ~first;
+                wx = ~dp & ~both(uniform_mask(s.sdry[f + 2])) & on_face & 0x1ffffffffffffff0ull;  // lanes 4 .. 60
+            }
+            const bool yac = g < 2 || g > ny - 2;
+            const mask64 dp = yac ? 0ull : uniform_mask(s.sdeep[f] & s.sdeep[f + 1] & s.sdeep[f + 2] & s.sdeep[f + 3]);
+            const mask64 wy = ~dp & ~uniform_mask(s.sdry[row_j(f + 1)] & s.sdry[row_j(f + 2)]) & on_cell &
+                              0x0ffffffffffffff0ull;  // lanes 4 .. 59
+            const int cw = __popcll(wx), c = cw + __popcll(wy);
+            int b = 0;
+            if (c) {
+                if (lane == 0) b = atomicAdd(&s.count[1], c);
+                b = __builtin_amdgcn_readfirstlane(b);
+                if (lane_of(wx)) s.list[b + rank_of(wx)] = (unsigned short)(f << 6 | lane);
+                if (lane_of(wy)) s.list[b + cw + rank_of(wy)] = (unsigned short)(0x8000 | f << 6 | lane);
+            }
+            if (lane == 0) {
+                s.w[0][f] = wx;
+                s.w[1][f] = wy;
+                s.base[0][f] = b;
+                s.base[1][f] = b + cw;
+            }
+        }
+        __syncthreads();
+        const int nq = __builtin_amdgcn_readfirstlane(s.count[1]);
+        if (nq > TileLds<T>::kResults) {
+            __syncthreads();
+            if (tid == 0) s.count[1] = 0;
+            r1 = r0 + kTileHalf;
+            __syncthreads();
+            continue;
+        }
+        if (nq) {
+            const StepArgs<T> &a = again<T>(args);
+            for (int k = tid; k < nq; k += 64 * W) {
+                const int code = s.list[k], l = code & 63, fr = (code >> 6) & 31;
+                const Listed f = listed(a, code, fr + 2);
+                const T *const qn = f.yf ? qy_ : qx_, *const qt = f.yf ? qx_ : qy_;
+                // the four cells: rows fr .. fr+3 of a y face, lanes l-2 .. l+1 of an x face
+                auto cell = [&](const int d) {
+                    const int p = f.yf ? row_j(fr + 2 + d) * 64 + l : (fr + 2) * 64 + l + d;
+                    return sc_of(s.es[p], D_[p + 128], qn[p + 128], qt[p + 128], f.p);
+                };
+                const MF<T> r = mom_waf<T>(f.yf, cell(-2), cell(-1), cell(0), cell(1), f.border, f.band, f.L, f.g0, f.g1,
+                                           f.ic0, f.ic1, f.val, dt, f.p);
+                s.R[k] = FaceOut<T>{r.mn, r.pn, r.mt, r.w};
+            }
+            __syncthreads();
+        }
+        // ---- deep momentum faces and the update of this wavefront's rows ----
+        const int fa = max(ra, r0), fb = min(rb, r1);
+        if (fa < fb) {
+            const StepArgs<T> &a = again<T>(args);
+            const T hpos = a.hpos;
+            const T tnow = (T)bc.t;
+            const int P = a.pitch;
+            const bool c1b = __builtin_amdgcn_readfirstlane(bc.cur) != 0;
+            const bool spx = x0 - SW_HALO < a.sp_izq || x0 + SW_OUT + SW_HALO > nx - a.sp_der;
+            const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
+            const StateOffsets<T> o(a, a.e[0], a.D, a.qx[0], a.qy[0], c1b ? a.e[0] : a.e[1], c1b ? a.qx[0] : a.qx[1],
+                                    c1b ? a.qy[0] : a.qy[1]);
+            // e*, D, sqrt(h*), qy/h*, qx, qy of row g-1 for the y faces
+            T s2, D2, sq2, v2, qx2, qy2;
+            auto star = [&](const int j, T &es, T &D, T &qx, T &qy) {
+                const int q = row_j(j) * 64 + lane;
+                es = s.es[q];
+                D = D_[q + 128];
+                qx = qx_[q + 128];
+                qy = qy_[q + 128];
+            };
+            star(fa + 1, s2, D2, qx2, qy2);
+            {
+                const T h = s2 + D2;
+                sq2 = Num<T>::sqrt(h);
+                v2 = qy2 * Num<T>::rcp(h);
+            }
+            T X2 = T(0), Y2 = T(0), W2 = T(0);  // accumulators of row g-1
+#pragma unroll 1
+            for (int f = fa; f <= fb; f++) {
+                const int g = y0 + f;
+                T s1, D1, qx1, qy1;
+                star(f + 2, s1, D1, qx1, qy1);
+                const T h1 = s1 + D1;
+                const T sq1 = Num<T>::sqrt(h1), ih = Num<T>::rcp(h1);
+                const T u1 = qx1 * ih, v1 = qy1 * ih;
+                T X1 = T(0), Y1 = T(0), W1 = T(0);
+                if (f < fb) {
+                    // x faces of row g
+                    const mask64 dp = all4(uniform_mask(s.sdeep[f + 2])) & ~first, wx = uniform_mask(s.w[0][f]);
+                    MF<T> r{T(0), T(0), T(0), T(0), T(0)};
+                    if (dp) {
+                        const int q = (f + 2) * 64 + lane - 1;
+                        DC<T> A, B;
+                        A.e = s.es[q]; A.D = D_[q + 128]; A.h = A.e + A.D; A.qn = qx_[q + 128]; A.qt = qy_[q + 128];
+                        A.s = dpp_left(sq1); A.un = dpp_left(u1);
+                        B.h = h1; B.e = s1; B.D = D1; B.qn = qx1; B.qt = qy1; B.s = sq1; B.un = u1;
+                        const MF<T> t = fast_mom_x(A, B, s.row[f + 2].ilx, s.row[f + 2].kdx, dt);
+                        if (lane_of(dp)) r = t;
+                    }
+                    if (lane_of(wx)) {
+                        const FaceOut<T> t = s.R[__builtin_amdgcn_readfirstlane(s.base[0][f]) + rank_of(wx)];
+                        r = MF<T>{t.mn, t.mt, t.pn, -t.mt, t.w};
+                    }
+                    X1 = -(low_border ? r.mn : r.pn) - dpp_right(r.mn);
+                    Y1 = -(low_border ? r.mt : r.pt) - dpp_right(r.mt);
+                    W1 = r.w + dpp_right(r.w);
+                }
+                {
+                    // y face between rows g-1 and g
+                    const bool yac = g < 2 || g > ny - 2;
+                    const mask64 dp = yac ? 0ull : uniform_mask(s.sdeep[f] & s.sdeep[f + 1] & s.sdeep[f + 2] & s.sdeep[f + 3]);
+                    const mask64 wy = uniform_mask(s.w[1][f]);
+                    MF<T> r{T(0), T(0), T(0), T(0), T(0)};
+                    if (dp) {
+                        DC<T> A, B;
+                        A.h = s2 + D2; A.e = s2; A.D = D2; A.qn = qy2; A.qt = qx2; A.s = sq2; A.un = v2;
+                        B.h = h1; B.e = s1; B.D = D1; B.qn = qy1; B.qt = qx1; B.s = sq1; B.un = v1;
+                        const MF<T> t = fast_mom_y(A, B, s.fy[f + 2], dt);
+                        if (lane_of(dp)) r = t;
+                    }
+                    if (lane_of(wy)) {
+                        const FaceOut<T> t = s.R[__builtin_amdgcn_readfirstlane(s.base[1][f]) + rank_of(wy)];
+                        r = MF<T>{t.mn, t.mt, t.pn, -t.mt, t.w};
+                    }
+                    Y2 -= r.mn;
+                    X2 -= r.mt;
+                    W2 += r.w;
+                    if (g == 0) { Y1 -= r.mn; X1 -= r.mt; }
+                    else { Y1 -= r.pn; X1 -= r.pt; }
+                    W1 += r.w;
+                }
+                // cell update of row g-1 (src/GPU/Volumen_kernel.cu:160-221)
+                if (f > fa) {
+                    const int ju = g - 1;
+                    const RowGeo<T> &rg = s.row[f + 1];
+                    const int soff = ju * P * (int)sizeof(T);
+                    const int voff = out_col ? gx * (int)sizeof(T) : kDropOffset;
+                    const T eo = e_[(f + 3) * 64 + lane];
+                    T cmax = pm[0], carr = pt[0];
+#pragma unroll
+                    for (int t = 1; t < KR; t++)
+                        if (f - 1 - ra == t) { cmax = pm[t]; carr = pt[t]; }
+                    // metrics from the state before the step (src/GPU/Metrics.cu:23-42,57-77)
+                    const bool max_on = out_col && eo > cmax && eo + D2 > a.eps_h;
+                    const bool arr_on = out_col && a.track_arrival && !Arrival<T>::arrived(carr) && tabs(eo - carr) > a.dif_at;
+                    const T dtc = (W2 < Num<T>::eps) ? Num<T>::big : Num<T>::div(T(2) * a.cfl * rg.A, W2);
+                    dtmin = fminf(dtmin, (float)dtc);  // halo lanes are dropped at the end
+                    const T val = dt * rg.invA;
+                    T qx = Num<T>::mad(val, X2, qx2), qy = Num<T>::mad(val, Y2, qy2);
+                    if (spx || ju < a.sp_sup || ju >= ny - a.sp_inf) sponge_q(a, gx, ju, qx, qy);
+                    const T hs = s2 + D2;
+                    if (hs <= hpos) near_dry(hs, qx2, qy2, qx, qy, dt, a.mf0, a.vmax, a.eps_h);
+                    bad = bad || (out_col && bad_cell(s2, qx, qy));
+                    buf_store<T>(eo, rs, voff, o.emax + soff, max_on);
+                    buf_store<T>(Arrival<T>::enc(tnow), rs, voff, o.arr + soff, arr_on);
+                    buf_store<T>(s2, rs, voff, o.oe + soff, out_col);
+                    buf_store<T>(qx, rs, voff, o.oqx + soff, out_col);
+                    buf_store<T>(qy, rs, voff, o.oqy + soff, out_col);
+                }
+                X2 = X1; Y2 = Y1; W2 = W1;
+                s2 = s1; D2 = D1; sq2 = sq1; v2 = v1; qx2 = qx1; qy2 = qy1;
+            }
+        }
+        r0 = r1;
+        r1 = min(r0 + kTileHalf, m);
+        if (r0 < m) {
+            __syncthreads();  // the results of this round are still being read
+            if (tid == 0) s.count[1] = 0;
+            __syncthreads();
+        }
+    }
+    raise_health(again<T>(args), bad);
+    return out_col ? dtmin : 3.0e38f;
 }
 
-// wavefront work items of the split launches: strip row * nseg + segment (-1: idle),
-// strip rows in units of `rows`, shifted up by a.yoff rows so that the strip rows along
-// the top and bottom borders are thin (the first one is cut at row 0).  n: the strip's
-// rows inside the grid.
+// workgroup minimum of the lanes' dt, folded into partial `part` of the launch's dt slot
 template <typename T>
-__device__ __forceinline__ void item_origin(const StepArgs<T> &a, const int item, const int rows, int &x0, int &y0,
-                                            int &n) {
-    const int strip = item / a.nseg;
-    x0 = (item - strip * a.nseg) * SW_OUT;
-    const int y = strip * rows - a.yoff;
-    y0 = max(y, 0);
-    n = min(y + rows, a.ny) - y0;
-}
-
-// origin of a deep-water strip (never cut at row 0: it lies clear of the top border band)
-template <typename T>
-__device__ __forceinline__ void deep_origin(const StepArgs<T> &a, const int item, int &x0, int &y0) {
-    const int strip = item / a.nseg;
-    x0 = (item - strip * a.nseg) * SW_OUT;
-    y0 = strip * a.srows - a.yoff;
-}
-
-// workgroup minimum of the lanes' dt, folded into the launch's dt slot of the grid
-template <typename T>
-__device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slot, float dtmin, float *s_red) {
+__device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slot, float dtmin, float *s_red,
+                                             const int part) {
     const int tid = threadIdx.x;
     dtmin = wave_min(dtmin);
     if ((tid & 63) == 0) s_red[tid >> 6] = dtmin;
@@ -574,83 +723,19 @@ __device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slo
         float m = s_red[0];
 #pragma unroll
         for (int w = 1; w < SW_WAVES; w++) m = fminf(m, s_red[w]);
-        atomicMin(&a.dtmin[dt_at(slot, 0)], __float_as_uint(m));
+        atomicMin(&a.dtmin[dt_at(slot, part)], __float_as_uint(m));
     }
-}
-
-// One step of one grid, general faces.  mode 0: one workgroup per strip block, every
-// block (the table's order, costliest first, or without a table the chunked XCD
-// order).  With a deep-water launch in the step, one wavefront per strip: mode 1 takes
-// the general strips (costliest first, cut into strips of a.gsrows rows so that the
-// few, slow coastal and border strips do not set the step's critical path), mode 2 the
-// strips the deep-water launch of this step handed back (the grid has room for all of
-// them; workgroups beyond the hand-backs return before the prologue).
-template <typename T>
-__global__ void __launch_bounds__(64 * SW_WAVES) k_sweep(const StepArgs<T> a, const int slot, const int mode) {
-    __shared__ BlockCtl<T> bc;
-    __shared__ float s_red[SW_WAVES];
-    const int tid = threadIdx.x;
-    const int bid = blockIdx.x;
-    // the step's writer is the deep-water launch when there is one, else workgroup 0
-    const bool writer = bid == 0 && mode == 0;
-    int n_fb = 0;
-    if (mode == 2) {  // hand-backs: workgroups beyond them return before the prologue
-        n_fb = min((int)__builtin_amdgcn_readfirstlane(a.fb_count[slot]), a.n_deep);
-        if (bid * SW_WAVES >= n_fb) return;
-    }
-    if (tid == 0) begin_step(a, slot, writer, bc);
-    __syncthreads();
-    if (!bc.run) return;
-    float dtmin;
-    if (mode == 0) {
-        int tile;
-        if (!a.order) {
-            const int loc = bid >> 3, ch = loc / a.chunk;
-            tile = ((ch << 3) + (bid & 7)) * a.chunk + (loc - ch * a.chunk);
-            if (tile >= a.n_tiles) return;
-        } else {
-            if (bid >= a.n_order) return;
-            tile = a.order[bid];
-        }
-        dtmin = sweep_block(a, bc, __builtin_amdgcn_readfirstlane(tile), writer);
-    } else {
-        const int k = bid * SW_WAVES + __builtin_amdgcn_readfirstlane(tid >> 6);
-        int item = -1;
-        if (mode == 1) {
-            if (k < a.n_gen) item = a.gen[k];
-        } else {
-            if (k < n_fb) item = a.fb_list[slot * a.n_deep + k];
-        }
-        item = __builtin_amdgcn_readfirstlane(item);
-        const int rows = mode == 1 ? a.gsrows : a.srows;
-        dtmin = 3.0e38f;
-        if (item >= 0) {
-            int x0, y0, n;
-            item_origin(a, item, rows, x0, y0, n);
-            // strips whose rows and 64 columns lie 8 cells or more inside the borders and
-            // their sponges (no clamped rows or columns, no first-order band, no border
-            // faces, no sponge) take the strip compiled without the edge cases
-            constexpr int m = 8;
-            const bool interior = !a.periodic && x0 - SW_HALO - m >= a.sp_izq &&
-                                  x0 + SW_OUT + SW_HALO + m <= a.nx - a.sp_der && y0 - m >= a.sp_sup &&
-                                  y0 + n + m <= a.ny - a.sp_inf;
-            if (n > 0) dtmin = interior ? sweep_strip<T, false>(a, bc, x0, y0, n) : sweep_strip<T, true>(a, bc, x0, y0, n);
-        }
-    }
-    block_dt_min(a, slot, dtmin, s_red);
 }
 
 // ---------------------------------------------------------------------------
-// Deep-water sweep.  Blocks whose strips and halos lie clear of the borders, the
-// first-order bands and the sponges, and whose still-water depth exceeds 3 hpos, run
-// this lean form of the pipeline: only the 2s faces, no sponge and no near-dry update,
-// no clamped columns or rows, and fewer pipeline registers.  Every wavefront checks at
-// run time the conditions under which the general faces take the 2s branch (every
-// loaded row deeper than hpos; every h* row that a face's stencil reaches deeper than
-// hpos).  A workgroup where a check fails commits no dt and hands its block to the
-// general launch of the same step, which recomputes and rewrites all of it; the two
-// launches evaluate the deep faces with the same functions, so the split changes no
-// result.
+// Deep-water strips.  Strips that with their halos lie clear of the borders, the
+// first-order bands and the sponges, and whose still-water depth exceeds 3 hpos, take only
+// the 2s faces: no sponge and no near-dry update, no clamped columns or rows.  Every
+// wavefront checks at run time the conditions under which the general faces take the 2s
+// branch (every loaded row deeper than hpos; every h* row that a face's stencil reaches
+// deeper than hpos).  A strip whose check fails commits no dt and is redone as general
+// tiles by its workgroup in the same launch (tile_or_strips); both evaluate the deep faces
+// with the same functions, so the split changes no result.
 // ---------------------------------------------------------------------------
 
 
@@ -658,15 +743,15 @@ __global__ void __launch_bounds__(64 * SW_WAVES) k_sweep(const StepArgs<T> a, co
 // column, so the pipeline lags two rows: iteration r loads row r, evaluates the mass
 // faces of row r and the y face between rows r-1 and r, h* of row r-1, the momentum
 // faces of row r-1 and the y face between rows r-2 and r-1, and updates row r-2.  Per
-// cell the accumulation order is that of the general pipeline (x faces, lower y face,
-// upper y face), so the values are the same.  The conditions under which the general
+// cell the accumulation order is that of the general tiles (x faces, lower y face, upper y
+// face), so the values are the same.  The conditions under which the general
 // faces take the 2s branch are checked for the whole strip and combined: every row
 // y0-4 .. y1+3 and every h* row y0-2 .. y1+1 deeper than hpos on every lane.  Returns
-// whether they held; if not, the caller hands the strip back (its writes are then
-// rewritten by the general launch and its dt is dropped).
+// whether they held; if not, the caller redoes the strip (its writes are then rewritten
+// and its dt is dropped).
 template <typename T>
 __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<T> &bc, const int x0, const int y0,
-                                           float &dtmin_out) {
+                                           const int rows, float &dtmin_out) {
     const int lane = threadIdx.x & 63;
     const bool c1 = bc.cur != 0;
     T *__restrict__ oe = c1 ? a.e[0] : a.e[1];
@@ -675,7 +760,7 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
     const T dt = (T)bc.dt;
     const T tnow = (T)bc.t;
     const int P = a.pitch;
-    const int y1 = min(y0 + a.srows, a.ny);
+    const int y1 = y0 + rows;
     float dtmin = 3.0e38f;
     bool valid = true, bad = false;
     if (x0 < a.nx) {
@@ -834,152 +919,138 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
         for (; r <= y1 + 2; r++) row(r, Edge{});
         dtmin = out_col ? dtmin : 3.0e38f;
     }
-    // a strip handed back is redone (and checked) by the general launch
+    // a strip whose check failed is redone, and checked, as general tiles
     if (valid) raise_health(a, bad);
     dtmin_out = dtmin;
     return valid;
 }
 
+// One workgroup's share of a step.  A tile item: the general tile (x0, y0, rows).  A deep
+// item: the strip (x0, y0, rows) of each wavefront; a strip whose check fails is redone
+// here, tile by tile, by the whole workgroup (the values it has stored are overwritten;
+// its metric updates used the state before the step and stand).
 template <typename T>
-__global__ void __launch_bounds__(64 * SW_WAVES) k_sweep_deep(const StepArgs<T> a, const int slot) {
+__device__ __forceinline__ float tile_or_strips(const ArgsAt<T> args, const BlockCtl<T> &bc, const bool tile, int x0, int y0,
+                                                int rows, TileLds<T> &s, int *s_fail) {
+    float dtmin = 3.0e38f;
+    int n_tiles = 1, per = 1;
+    if (!tile) {
+        const int wv = threadIdx.x >> 6;
+        bool ok = true;
+        if (x0 >= 0) ok = deep_strip(again<T>(args), bc, x0, y0, rows, dtmin);
+        if (!ok) {
+            dtmin = 3.0e38f;
+            __threadfence();  // its stores land before those that replace them
+        }
+        if ((threadIdx.x & 63) == 0) {
+            s_fail[3 * wv] = ok ? -1 : x0;
+            s_fail[3 * wv + 1] = y0;
+            s_fail[3 * wv + 2] = ok ? 0 : rows;
+        }
+        __syncthreads();
+        int most = 0;
+        for (int w = 0; w < SW_WAVES; w++) most = max(most, __builtin_amdgcn_readfirstlane(s_fail[3 * w + 2]));
+        if (most == 0) return dtmin;
+        per = (most + kTileRows - 1) / kTileRows;
+        n_tiles = SW_WAVES * per;
+    }
+    for (int t = 0; t < n_tiles; t++) {
+        if (!tile) {  // tile t - w * per of the strip of wavefront w
+            const int w = t / per, d = (t - w * per) * kTileRows;
+            x0 = __builtin_amdgcn_readfirstlane(s_fail[3 * w]);
+            y0 = __builtin_amdgcn_readfirstlane(s_fail[3 * w + 1]) + d;
+            rows = min(kTileRows, __builtin_amdgcn_readfirstlane(s_fail[3 * w + 2]) - d);
+            if (x0 < 0 || rows <= 0) continue;
+            __syncthreads();  // the tile before still uses the rows in LDS
+        }
+        dtmin = fminf(dtmin, general_tile(args, bc, x0, y0, rows, s));
+    }
+    return dtmin;
+}
+
+// Work items, one per workgroup: a general tile (x0, y0 << 4 | rows), or four deep-water
+// strips (index of the first in the strip list, 0).  `strip`: a deep item's strip of this
+// wavefront; x0 < 0: none.
+template <typename T> __device__ __forceinline__ int2 item_origin(const StepArgs<T> &a, const int2 it, bool &tile, int &rows) {
+    rows = it.y & 15;
+    tile = rows != 0;
+    if (tile) return make_int2(it.x, it.y >> 4);
+    const int2 strip = uniform_load(a.deep + it.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    rows = strip.y & 2047;
+    return make_int2(strip.x, strip.y >> 11);
+}
+
+// One step of one grid in one launch, a workgroup per work item.  Workgroup 0 is the
+// step's writer.
+template <typename T>
+__global__ void __launch_bounds__(64 * SW_WAVES, sizeof(T) == 4 ? 5 : 2) k_sweep(const StepArgs<T> args_, const int slot) {
+    __shared__ TileLds<T> s;
     __shared__ BlockCtl<T> bc;
     __shared__ float s_red[SW_WAVES];
+    __shared__ int s_fail[3 * SW_WAVES];
+    (void)args_;  // the first kernel argument, read through its address
+    const ArgsAt<T> args = (ArgsAt<T>)__builtin_amdgcn_kernarg_segment_ptr();
+    const StepArgs<T> &a = again<T>(args);
     const int tid = threadIdx.x, bid = blockIdx.x;
-    if (tid == 0) {
-        begin_step(a, slot, bid == 0, bc);  // this launch is the step's writer
-        if (bid == 0) a.fb_count[(slot + 1) % 3] = 0u;  // the next launch's hand-back list
-    }
+    const int2 w = uniform_load(a.items + bid);
+    if (tid == 0) begin_step(a, slot, bid == 0, bc, kDtParts);
+    bool tile;
+    int rows;
+    const int2 o = item_origin(a, w, tile, rows);
     __syncthreads();
     if (!bc.run) return;
     if (bid == 0) {
         const bool c1 = bc.cur != 0;
-        gather_gauges(a, bc, c1 ? a.e[1] : a.e[0], c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], tid,
-                      64 * SW_WAVES);
+        gather_gauges(a, bc, c1 ? a.e[1] : a.e[0], c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], tid, 64 * SW_WAVES);
     }
-    const int k = bid * SW_WAVES + __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int item = __builtin_amdgcn_readfirstlane(k < a.n_deep ? a.deep[k] : -1);
-    float dtmin = 3.0e38f;
-    if (item >= 0) {
-        int x0, y0;
-        deep_origin(a, item, x0, y0);
-        if (!deep_strip(a, bc, x0, y0, dtmin)) {
-            // hand the strip back; its dt comes from the general launch that redoes it
-            dtmin = 3.0e38f;
-            if ((tid & 63) == 0) {
-                const unsigned n = atomicAdd(&a.fb_count[slot], 1u);
-                if (n < (unsigned)a.n_deep) a.fb_list[slot * a.n_deep + n] = item;
-            }
-        }
-    }
-    block_dt_min(a, slot, dtmin, s_red);
+    const float dtmin = tile_or_strips<T>(args, bc, tile, o.x, o.y, rows, s, s_fail);
+    block_dt_min(again<T>(args), slot, dtmin, s_red, bid);
 }
 
-}  // namespace thy
-
-namespace thy {
-
 // ---------------------------------------------------------------------------
-// Many grids per launch.  Each scenario keeps its own state, control block and dt
-// slots; a step of the batch advances every running scenario by one of its own steps
-// in three launches, as for one grid: the deep-water strips of all scenarios, beside
-// them (on a second stream) the general strips of all scenarios, costliest first, and
-// after both the strips that the deep-water launch handed back.  Every wavefront takes
-// one item (scenario, strip) and runs the step prologue of its scenario itself; the
-// item flagged as its scenario's writer publishes the next control block.  Item
-// counts are read on the device, so one captured launch sequence serves a changing
-// item list up to the captured grid sizes.
+// Many grids per launch.  Each scenario keeps its own state, control block and dt slots; a
+// step of the batch advances every running scenario by one of its own steps in one launch:
+// the general tiles of all scenarios, costliest first, then their deep-water strips, four
+// of one scenario to a workgroup.  The item flagged as its scenario's writer publishes the
+// next control block.  Item counts are read on the device, so one captured launch sequence
+// serves a changing item list up to the captured grid size.
 // ---------------------------------------------------------------------------
-struct BatchArgs {
-    const StepArgs<float> *args;  // per scenario slot (zeroed while the slot is free)
-    const int2 *deep;             // (scenario slot, strip << 1 | writer): deep-water strips
-    const int *n_deep;
-    const int2 *gen;              // (scenario slot, strip << 1 | writer): general strips
-    const int *n_gen;
-    int2 *fb_list;                // 3 slots of fb_cap hand-backs (scenario slot, strip)
-    unsigned int *fb_count;       // 3 slots: launch n appends to slot n mod 3
-    int fb_cap;
-    int gen_sub;                  // general items are strips of gsrows rows (else srows)
+struct BatchItem {
+    int slot;    // scenario slot (-1: padding)
+    int writer;
+    int2 it;     // the work item, as in the scenario's own list
 };
 
-// the step prologue of one wavefront's scenario (every lane computes the same values;
-// lane 0 of the writer item publishes the next control block and samples the gauges)
-__device__ __forceinline__ BlockCtl<float> wave_begin(const StepArgs<float> &a, const int slot, const bool writer) {
-    const int lane = threadIdx.x & 63;
-    BlockCtl<float> bc;
-    begin_step(a, slot, writer && lane == 0, bc, kDtParts);
-    if (writer && bc.run) {
+struct BatchArgs {
+    const StepArgs<float> *args;  // per scenario slot (zeroed while the slot is free)
+    const BatchItem *items;
+    const int *n_items;
+};
+
+__global__ void __launch_bounds__(64 * SW_WAVES, 5) k_batch(const BatchArgs q, const int slot) {
+    __shared__ TileLds<float> s;
+    __shared__ BlockCtl<float> bc;
+    __shared__ float s_red[SW_WAVES];
+    __shared__ int s_fail[3 * SW_WAVES];
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(*q.n_items)) return;
+    const BatchItem w = uniform_load(q.items + blockIdx.x);
+    if (w.slot < 0) return;
+    const ArgsAt<float> args = (ArgsAt<float>)(q.args + w.slot);
+    const StepArgs<float> &a = again<float>(args);
+    if (!a.ctrl) return;
+    if (tid == 0) begin_step(a, slot, w.writer != 0, bc, kDtParts);
+    bool tile;
+    int rows;
+    const int2 o = item_origin(a, w.it, tile, rows);
+    __syncthreads();
+    if (!bc.run) return;
+    if (w.writer) {
         const bool c1 = bc.cur != 0;
-        gather_gauges(a, bc, c1 ? a.e[1] : a.e[0], c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], lane, 64);
+        gather_gauges(a, bc, c1 ? a.e[1] : a.e[0], c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], tid, 64 * SW_WAVES);
     }
-    return bc;
-}
-
-__device__ __forceinline__ void wave_dt_min(const StepArgs<float> &a, const int slot, const float dtmin) {
-    const float m = wave_min(dtmin);
-    if ((threadIdx.x & 63) == 0)
-        atomicMin(&a.dtmin[dt_at(slot, blockIdx.x * SW_WAVES + (threadIdx.x >> 6))], __float_as_uint(m));
-}
-
-__global__ void __launch_bounds__(64 * SW_WAVES) k_batch_deep(const BatchArgs q, const int slot) {
-    const int lane = threadIdx.x & 63;
-    const int k = blockIdx.x * SW_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (k == 0 && lane == 0) q.fb_count[(slot + 1) % 3] = 0u;  // the next launch's hand-back list
-    const int n = __builtin_amdgcn_readfirstlane(*q.n_deep);
-    if (k >= n) return;
-    const int2 w = q.deep[k];
-    const int sc = __builtin_amdgcn_readfirstlane(w.x), code = __builtin_amdgcn_readfirstlane(w.y);
-    if (sc < 0) return;  // padding of an XCD run
-    const StepArgs<float> a = uniform_load(q.args + sc);
-    if (!a.ctrl) return;
-    const BlockCtl<float> bc = wave_begin(a, slot, (code & 1) != 0);
-    if (!bc.run) return;
-    int x0, y0;
-    deep_origin(a, code >> 1, x0, y0);
-    float dtmin;
-    if (!deep_strip(a, bc, x0, y0, dtmin)) {
-        // hand the strip back; its dt comes from the launch that redoes it
-        dtmin = 3.0e38f;
-        if (lane == 0) {
-            const unsigned m = atomicAdd(&q.fb_count[slot], 1u);
-            if (m < (unsigned)q.fb_cap) q.fb_list[slot * q.fb_cap + m] = make_int2(sc, code >> 1);
-        }
-    }
-    wave_dt_min(a, slot, dtmin);
-}
-
-// one wavefront's general strip of the batch (item code: strip << 1 | writer; strips
-// of gsrows rows when sub, else of srows rows)
-__device__ __forceinline__ void batch_general_item(const BatchArgs &q, const int slot, const int sc, const int code,
-                                                   const bool sub) {
-    const StepArgs<float> a = uniform_load(q.args + sc);
-    if (!a.ctrl) return;
-    const BlockCtl<float> bc = wave_begin(a, slot, (code & 1) != 0);
-    if (!bc.run) return;
-    const int rows = sub ? a.gsrows : a.srows;
-    int x0, y0, n;
-    item_origin(a, code >> 1, rows, x0, y0, n);
-    wave_dt_min(a, slot, n > 0 ? sweep_strip(a, bc, x0, y0, n) : 3.0e38f);
-}
-
-// HANDBACK false: the general strips, one wavefront each.  HANDBACK true: the strips
-// that this step's deep-water launch handed back; a small grid strides over them.
-template <bool HANDBACK>
-__global__ void __launch_bounds__(64 * SW_WAVES) k_batch_general(const BatchArgs q, const int slot) {
-    const int k0 = blockIdx.x * SW_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (!HANDBACK) {
-        const int n = __builtin_amdgcn_readfirstlane(*q.n_gen);
-        if (k0 >= n) return;
-        const int2 w = q.gen[k0];
-        batch_general_item(q, slot, __builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y),
-                           q.gen_sub != 0);
-    } else {
-        const int n = __builtin_amdgcn_readfirstlane((int)min(q.fb_count[slot], (unsigned)q.fb_cap));
-        for (int k = k0; k < n; k += gridDim.x * SW_WAVES) {
-            const int2 w = q.fb_list[slot * q.fb_cap + k];
-            batch_general_item(q, slot, __builtin_amdgcn_readfirstlane(w.x),
-                               __builtin_amdgcn_readfirstlane(w.y) << 1, false);
-        }
-    }
+    const float dtmin = tile_or_strips<float>(args, bc, tile, o.x, o.y, rows, s, s_fail);
+    block_dt_min(again<float>(args), slot, dtmin, s_red, blockIdx.x);
 }
 
 // control blocks of the scenarios at launch slot `slot`, gathered for one copy (a free

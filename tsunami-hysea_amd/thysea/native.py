@@ -287,9 +287,9 @@ class Solver:
         return v.value
 
     def autotune(self, reps=5):
-        """Pick the fastest strip height and general strip height of the row-sweep
-        kernel (thy_autotune); returns (strip_rows, ms per step) and keeps the general
-        strip height in self.general_rows."""
+        """Pick the fastest strip height and tile height of the row-sweep kernel
+        (thy_autotune); returns (strip_rows, ms per step) and keeps the tile height in
+        self.general_rows."""
         rows = C.c_int()
         grows = C.c_int()
         ms = C.c_double()
