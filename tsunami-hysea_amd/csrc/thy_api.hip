@@ -53,7 +53,7 @@ struct thy_ctx {
     void *D = nullptr, *emax = nullptr, *arr = nullptr;
     void *state = nullptr;   // one allocation holding e, qx, qy (x2), D, emax and arr
     size_t state_bytes = 0;
-    void *row = nullptr, *fy = nullptr;
+    void *row = nullptr, *fy = nullptr, *deep_row = nullptr;
     double *area_d = nullptr;
     Ctrl *ctrl = nullptr;
     unsigned int *dtmin = nullptr;
@@ -230,6 +230,7 @@ StepArgs<T> make_args(thy_ctx *c, const bool batch = false) {
     a.block_bytes = (int)std::min(c->state_bytes, (size_t)INT32_MAX);  // kernel 0 only when it fits
     a.row = (const RowGeo<T> *)c->row;
     a.fy = (const FaceGeoY<T> *)c->fy;
+    a.deep_row = (const DeepRow<T> *)c->deep_row;
     a.ctrl = c->ctrl;
     a.dtmin = c->dtmin;
     a.ftime = c->ftime;
@@ -329,6 +330,33 @@ void fill_geometry(thy_ctx *c, std::vector<RowGeo<T>> &rows, std::vector<FaceGeo
         f.pad = T(0);
         fys[g] = f;
     }
+}
+
+// the row tables on the device
+template <typename T>
+int upload_geometry(thy_ctx *ctx) {
+    std::vector<RowGeo<T>> rows;
+    std::vector<FaceGeoY<T>> fys;
+    fill_geometry(ctx, rows, fys);
+    const int ny = ctx->ny;
+    std::vector<DeepRow<T>> deep(ny + 1);
+    for (int r = 0; r <= ny; r++) {
+        const RowGeo<T> &r0 = rows[std::min(r, ny - 1)], &r1 = rows[std::max(r - 1, 0)], &r2 = rows[std::max(r - 2, 0)];
+        const FaceGeoY<T> &f0 = fys[r], &f1 = fys[std::max(r - 1, 0)];
+        DeepRow<T> &d = deep[r];
+        memset(&d, 0, sizeof(d));
+        d.ilx = r0.ilx; d.kA = r0.kA; d.lc0 = f0.lc0; d.k0 = f0.k0; d.k1 = f0.k1; d.ic0 = f0.ic0; d.ic1 = f0.ic1;
+        d.p = DeepMom<T>{r1.invA, r1.ilx, r1.kdx, f1.len, f1.cos0, f1.cos1, f1.ic0, f1.ic1, f1.gh, f1.gd, f1.g1ic0, f1.kdy};
+        d.q = DeepUpdate<T>{r2.A, r2.invA};
+    }
+    auto put = [&](void *&dst, const auto &v) -> hipError_t {
+        hipError_t e = dev_alloc(&dst, v.size() * sizeof(v[0]));
+        return e == hipSuccess ? ctx_copy(ctx, dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice) : e;
+    };
+    HIPCHK(put(ctx->row, rows));
+    HIPCHK(put(ctx->fy, fys));
+    HIPCHK(put(ctx->deep_row, deep));
+    return THY_OK;
 }
 
 int pick_tile(thy_ctx *c) {
@@ -1129,23 +1157,7 @@ int thy_create(const thy_grid *g, const thy_params *p, thy_ctx **out) {
         HIPCHK(dev_alloc((void **)&ctx->okada_row, r.size() * sizeof(OkadaRow)));
         HIPCHK(ctx_copy(ctx, ctx->okada_row, r.data(), r.size() * sizeof(OkadaRow), hipMemcpyHostToDevice));
     }
-    if (ctx->prec) {
-        std::vector<RowGeo<double>> rows;
-        std::vector<FaceGeoY<double>> fys;
-        fill_geometry(ctx, rows, fys);
-        HIPCHK(dev_alloc(&ctx->row, rows.size() * sizeof(rows[0])));
-        HIPCHK(dev_alloc(&ctx->fy, fys.size() * sizeof(fys[0])));
-        HIPCHK(ctx_copy(ctx, ctx->row, rows.data(), rows.size() * sizeof(rows[0]), hipMemcpyHostToDevice));
-        HIPCHK(ctx_copy(ctx, ctx->fy, fys.data(), fys.size() * sizeof(fys[0]), hipMemcpyHostToDevice));
-    } else {
-        std::vector<RowGeo<float>> rows;
-        std::vector<FaceGeoY<float>> fys;
-        fill_geometry(ctx, rows, fys);
-        HIPCHK(dev_alloc(&ctx->row, rows.size() * sizeof(rows[0])));
-        HIPCHK(dev_alloc(&ctx->fy, fys.size() * sizeof(fys[0])));
-        HIPCHK(ctx_copy(ctx, ctx->row, rows.data(), rows.size() * sizeof(rows[0]), hipMemcpyHostToDevice));
-        HIPCHK(ctx_copy(ctx, ctx->fy, fys.data(), fys.size() * sizeof(fys[0]), hipMemcpyHostToDevice));
-    }
+    if ((r = ctx->prec ? upload_geometry<double>(ctx) : upload_geometry<float>(ctx)) != THY_OK) return r;
     // zero state so that padding columns hold finite values
     for (int k = 0; k < 2; k++) {
         HIPCHK(ctx_fill(ctx, ctx->e[k], b));
@@ -1167,7 +1179,7 @@ void thy_destroy(thy_ctx *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     drop_graphs(ctx);
-    void *ptrs[] = {ctx->state, ctx->row, ctx->fy, ctx->area_d, ctx->ctrl, ctx->dtmin, ctx->scratch_u,
+    void *ptrs[] = {ctx->state, ctx->row, ctx->fy, ctx->deep_row, ctx->area_d, ctx->ctrl, ctx->dtmin, ctx->scratch_u,
                     ctx->ftime, ctx->gpos, ctx->gbuf, ctx->gtime, ctx->okada_def, ctx->okada_row, ctx->mass_partial, ctx->outbuf,
                     ctx->steplog, ctx->alone.deep, ctx->alone.items, ctx->batched.deep, ctx->batched.items, ctx->health};
     for (void *q : ptrs)

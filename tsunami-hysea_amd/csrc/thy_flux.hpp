@@ -28,6 +28,12 @@ template <> struct Num<float> {
     static __device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
     // a / sqrt(x) with one transcendental (reciprocal square root)
     static __device__ __forceinline__ float div_sqrt(float a, float x) { return a * __builtin_amdgcn_rsqf(x); }
+    // lesser of two numbers that are not signalling NaN (fminf would first quiet them)
+    static __device__ __forceinline__ float min(float a, float b) {
+        float m;
+        asm("v_min_f32 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+        return m;
+    }
     static __device__ __forceinline__ float exp(float x) {
         return __builtin_amdgcn_exp2f(x * 1.4426950408889634f);
     }
@@ -46,6 +52,7 @@ template <> struct Num<double> {
     // FP64 keeps the product and the sum rounded separately, as the oracle rounds them
     static __device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
     static __device__ __forceinline__ double div_sqrt(double a, double x) { return a / ::sqrt(x); }
+    static __device__ __forceinline__ double min(double a, double b) { return a < b ? a : b; }
     static __device__ __forceinline__ double exp(double x) { return ::exp(x); }
     static __device__ __forceinline__ double pow43(double x) { return ::pow(x, 4.0 / 3.0); }
 };
@@ -118,14 +125,16 @@ template <typename T> __device__ __forceinline__ T blend(T hij, T hpos, bool alf
 // from the row tables (the same condition, no division unless the limiter acts).  Every
 // face evaluation (deep-water forms and general faces) goes through this one function,
 // so a face evaluated by two wavefronts has one value.
-template <typename T> __device__ __forceinline__ T positivity(T F, T h0, T h1, T k0, T k1, T dt) {
-    const T lim = (F > T(0)) ? h0 * k0 : h1 * k1;
-    const T den = habs(F) + Num<T>::eps;
+template <typename T> __device__ __forceinline__ T limit_flux(T F, const T lim, const T den, const T dt) {
     if (dt * den > lim) {
         const T dt0 = Num<T>::div(lim, den);
         if (dt > dt0) F *= Num<T>::div(dt0, dt + Num<T>::eps);
     }
     return F;
+}
+template <typename T> __device__ __forceinline__ T positivity(T F, T h0, T h1, T k0, T k1, T dt) {
+    const T lim = (F > T(0)) ? h0 * k0 : h1 * k1;
+    return limit_flux(F, lim, habs(F) + Num<T>::eps, dt);
 }
 
 // wet/dry treatment of the normal discharges: src/GPU/Arista_kernel.cu:70-77

@@ -75,6 +75,22 @@ template <typename T> struct FaceGeoY {
     T gh, gd, g1ic0, k0, k1, lc0, kdy, pad;
 };
 
+// What iteration r of a deep-water strip needs of its rows, in one record (one fetch a row
+// instead of nine): the mass faces of row r and y face r, h* and the momentum faces of row
+// r-1 (with y face r-1), the update of row r-2; the same values as the tables above.
+template <typename T> struct DeepMom {
+    T invA, ilx, kdx, len, cos0, cos1, ic0, ic1, gh, gd, g1ic0, kdy;
+};
+template <typename T> struct DeepUpdate {
+    T A, invA;
+};
+template <typename T> struct alignas(32) DeepRow {
+    T ilx, kA, lc0, k0, k1, ic0, ic1;
+    DeepMom<T> p;     // row r-1
+    DeepUpdate<T> q;  // row r-2
+    T pad[3];
+};
+
 // The dt minimum of a launch is kept as kDtParts partial minima (float bits; for
 // positive floats the unsigned order is the float order), one 64-byte line apart:
 // atomics on one line are applied one after another.  The launches of one grid fold
@@ -112,6 +128,7 @@ template <typename T> struct StepArgs {
     int block_bytes;         //   its size, below 2^31
     const RowGeo<T> *row;
     const FaceGeoY<T> *fy;
+    const DeepRow<T> *deep_row;  // [ny + 1]
     Ctrl *ctrl;
     unsigned int *dtmin;     // 3 launch slots of kDtParts partial minima (dt_at)
     const double *ftime;     // fault times (s), sorted
@@ -276,6 +293,11 @@ __device__ __forceinline__ void raise_health(const StepArgs<T> &a, const bool ba
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+__device__ __forceinline__ double wave_min(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
     return v;
 }
 

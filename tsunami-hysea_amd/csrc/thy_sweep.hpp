@@ -22,33 +22,19 @@ constexpr int SW_HALO = 4;
 constexpr int SW_OUT = 64 - 2 * SW_HALO;  // output columns per wavefront
 constexpr int SW_WAVES = 4;               // wavefronts per workgroup (side by side in x)
 
-// Cross-lane moves: lane l receives the value of lane l-1 / l-2 / l+1 (a lane without
-// a source keeps its own value; lanes 0, 1 and 63 lie outside every output cell's
-// stencil).  These go through ds_bpermute on the LDS pipe, which leaves the VALU (the
-// unit this kernel saturates) to the flux arithmetic; DPP row moves were measured
-// slower here for that reason.
-template <typename T> __device__ __forceinline__ T from_left(T v) { return __shfl_up(v, 1, 64); }
-template <typename T> __device__ __forceinline__ T from_right(T v) { return __shfl_down(v, 1, 64); }
-
-// The same moves as VALU data-parallel-primitive moves across the whole wavefront
-// (wave_shr:1 / wave_shl:1; the lane without a source keeps its own value): a few cycles
-// of latency instead of an LDS round trip.  The general tiles, whose time is a chain of
-// latencies, use these; the deep-water strips keep the LDS moves, which leave the VALU to
-// their flux arithmetic.
-__device__ __forceinline__ int dpp_shr1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false); }
-__device__ __forceinline__ int dpp_shl1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false); }
-__device__ __forceinline__ float dpp_left(float v) { return __int_as_float(dpp_shr1(__float_as_int(v))); }
-__device__ __forceinline__ float dpp_right(float v) { return __int_as_float(dpp_shl1(__float_as_int(v))); }
-__device__ __forceinline__ double dpp_left(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = dpp_shr1((int)(b & 0xffffffffll)), hi = dpp_shr1((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+// Cross-lane moves: lane l receives the value of lane l-1 / l+1 (the lane without a source
+// receives 0 or keeps its own value; it lies outside every output cell's stencil).  FP32
+// moves are data-parallel-primitive moves across the whole wavefront (wave_shr:1,
+// wave_shl:1), which the compiler folds into the instruction that uses the value where
+// there is one; FP64 values move as two words.
+__device__ __forceinline__ float dpp_left(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
 }
-__device__ __forceinline__ double dpp_right(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = dpp_shl1((int)(b & 0xffffffffll)), hi = dpp_shl1((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+__device__ __forceinline__ float dpp_right(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
 }
+__device__ __forceinline__ double dpp_left(double v) { return __shfl_up(v, 1, 64); }
+__device__ __forceinline__ double dpp_right(double v) { return __shfl_down(v, 1, 64); }
 
 // read-only table entry at a wavefront-uniform address (scalar load)
 template <typename S> __device__ __forceinline__ S uniform_load(const S *p) {
@@ -91,20 +77,20 @@ __device__ __forceinline__ T fast_mass_y(T qa, T ha, T hb, const FaceGeoY<T> &f,
     return positivity(F, ha, hb, f.k0, f.k1, dt);
 }
 
-// one cell of a deep momentum face: total depth, eta, depth, normal and tangential
-// discharge, sqrt(h), normal velocity
+// one cell of a deep momentum face: total depth, normal and tangential discharge, sqrt(h),
+// normal velocity
 template <typename T> struct DC {
-    T h, e, D, qn, qt, s, un;
+    T h, qn, qt, s, un;
 };
 
-// x face, 2s momentum flux: src/GPU/Arista_kernel.cu:221-280
+// x face, 2s momentum flux: src/GPU/Arista_kernel.cu:221-280.  deta: eta difference of the
+// face (deta_of; e_b - e_a where both cells' eta clears the shallower bed)
 template <typename T>
-__device__ __forceinline__ MF<T> fast_mom_x(const DC<T> &a, const DC<T> &b, T il, T kd, T dt) {
+__device__ __forceinline__ MF<T> fast_mom_x(const DC<T> &a, const DC<T> &b, T deta, T il, T kd, T dt) {
     MF<T> o;
     const T hij = T(0.5) * (a.h + b.h);
     const T uij = Num<T>::div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
     const T lmax = habs(uij) + Num<T>::sqrt(hij);
-    const T deta = deta_of(a.e, b.e, a.D, b.D);
     const bool up = uij < T(0);
     const T uu = up ? b.un : a.un;
     const T qnn = up ? b.qn : a.qn;
@@ -120,15 +106,15 @@ __device__ __forceinline__ MF<T> fast_mom_x(const DC<T> &a, const DC<T> &b, T il
     return o;
 }
 
-// y face, 2s momentum flux: src/GPU/Arista_kernel.cu:780-843
-template <typename T>
-__device__ __forceinline__ MF<T> fast_mom_y(const DC<T> &a, const DC<T> &b, const FaceGeoY<T> &f, T dt) {
+// y face, 2s momentum flux: src/GPU/Arista_kernel.cu:780-843 (G: FaceGeoY or DeepMom)
+template <typename T, typename G>
+__device__ __forceinline__ MF<T> fast_mom_y(const DC<T> &a, const DC<T> &b, T deta, const G &f, T dt) {
     MF<T> o;
     const T g0 = f.cos0, g1 = f.cos1, ic0 = f.ic0, ic1 = f.ic1, len = f.len;
     const T hij = T(0.5) * (a.h + b.h);
     const T uij = Num<T>::div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
     const T lmax = habs(uij) + Num<T>::sqrt(hij);
-    const T deta = Num<T>::mad(-(uij * uij), f.gd, f.gh * deta_of(a.e, b.e, a.D, b.D));
+    deta = Num<T>::mad(-(uij * uij), f.gd, f.gh * deta);
     const bool up = uij < T(0);
     const T uu = up ? b.un : a.un;
     const T qnn = up ? b.qn : a.qn;
@@ -191,7 +177,7 @@ template <> __device__ __forceinline__ double buf_load<double>(__amdgpu_buffer_r
 constexpr int kDropOffset = (int)0x80000000;
 
 template <typename T>
-__device__ __forceinline__ void buf_store(T v, __amdgpu_buffer_rsrc_t r, int voff, int soff, bool on);
+__device__ __forceinline__ void buf_store(T v, __amdgpu_buffer_rsrc_t r, int voff, int soff, bool on = true);
 template <>
 __device__ __forceinline__ void buf_store<float>(float v, __amdgpu_buffer_rsrc_t r, int voff, int soff, bool on) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, on ? voff : kDropOffset, soff, 0);
@@ -629,10 +615,11 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
                     if (dp) {
                         const int q = (f + 2) * 64 + lane - 1;
                         DC<T> A, B;
-                        A.e = s.es[q]; A.D = D_[q + 128]; A.h = A.e + A.D; A.qn = qx_[q + 128]; A.qt = qy_[q + 128];
+                        const T eL = s.es[q], DL = D_[q + 128];
+                        A.h = eL + DL; A.qn = qx_[q + 128]; A.qt = qy_[q + 128];
                         A.s = dpp_left(sq1); A.un = dpp_left(u1);
-                        B.h = h1; B.e = s1; B.D = D1; B.qn = qx1; B.qt = qy1; B.s = sq1; B.un = u1;
-                        const MF<T> t = fast_mom_x(A, B, s.row[f + 2].ilx, s.row[f + 2].kdx, dt);
+                        B.h = h1; B.qn = qx1; B.qt = qy1; B.s = sq1; B.un = u1;
+                        const MF<T> t = fast_mom_x(A, B, deta_of(eL, s1, DL, D1), s.row[f + 2].ilx, s.row[f + 2].kdx, dt);
                         if (lane_of(dp)) r = t;
                     }
                     if (lane_of(wx)) {
@@ -651,9 +638,9 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
                     MF<T> r{T(0), T(0), T(0), T(0), T(0)};
                     if (dp) {
                         DC<T> A, B;
-                        A.h = s2 + D2; A.e = s2; A.D = D2; A.qn = qy2; A.qt = qx2; A.s = sq2; A.un = v2;
-                        B.h = h1; B.e = s1; B.D = D1; B.qn = qy1; B.qt = qx1; B.s = sq1; B.un = v1;
-                        const MF<T> t = fast_mom_y(A, B, s.fy[f + 2], dt);
+                        A.h = s2 + D2; A.qn = qy2; A.qt = qx2; A.s = sq2; A.un = v2;
+                        B.h = h1; B.qn = qy1; B.qt = qx1; B.s = sq1; B.un = v1;
+                        const MF<T> t = fast_mom_y(A, B, deta_of(s2, s1, D2, D1), s.fy[f + 2], dt);
                         if (lane_of(dp)) r = t;
                     }
                     if (lane_of(wy)) {
@@ -738,190 +725,200 @@ __device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slo
 // with the same functions, so the split changes no result.
 // ---------------------------------------------------------------------------
 
+// Least depth of a deep-water strip whatever hpos is: far below any depth of use, and far
+// enough above zero that the wave speeds of a cell sum to more than the guard of its dt.
+constexpr double kDeepFloor = 1e-12;
 
-// One wavefront's strip on the deep-water path.  The 2s faces reach one row and one
-// column, so the pipeline lags two rows: iteration r loads row r, evaluates the mass
-// faces of row r and the y face between rows r-1 and r, h* of row r-1, the momentum
-// faces of row r-1 and the y face between rows r-2 and r-1, and updates row r-2.  Per
-// cell the accumulation order is that of the general tiles (x faces, lower y face, upper y
-// face), so the values are the same.  The conditions under which the general
-// faces take the 2s branch are checked for the whole strip and combined: every row
-// y0-4 .. y1+3 and every h* row y0-2 .. y1+1 deeper than hpos on every lane.  Returns
-// whether they held; if not, the caller redoes the strip (its writes are then rewritten
-// and its dt is dropped).
+// the value, computed where it is written (a cross-lane move folds into an instruction of
+// its own basic block only)
+__device__ __forceinline__ float here(float v) { asm("" : "+v"(v)); return v; }
+__device__ __forceinline__ double here(double v) { return v; }
+
+// One wavefront's strip on the deep-water path.  The 2s faces reach one row and one column,
+// so the pipeline lags two rows: iteration r loads row r + 1, evaluates the mass faces of
+// row r and the y face between rows r-1 and r, h* of row r-1, the momentum faces of row
+// r-1 and the y face between rows r-2 and r-1, and updates row r-2.  Per cell the
+// accumulation order is that of the general tiles (x faces, lower y face, upper y face), so
+// the values are the same.
+//
+// The conditions under which the general faces take the 2s branch and its eta difference is
+// e1 - e0 (every row y0-4 .. y1+3 and every h* deeper than hpos on every lane, both eta of a
+// face above the shallower bed, no h* clipped at the bed) follow from one: the lowest eta
+// plus the smallest depth of the strip exceeds hpos.  (A rounded sum is monotonic in its
+// terms.)  Two running minima a row take the place of a vote for each.  Returns whether it
+// held; if not, the caller redoes the strip (its writes are then rewritten and its dt is
+// dropped).
+//
+// Bound by memory on a large grid (4000x3000, all deep: 111 us a step, 3.9 TB/s of the nine
+// arrays, whatever the strip height, and no less with two rows of cells in flight), by the
+// latency of a row on a small one.  A steady row takes 132 vector instructions (175 before:
+// a vote and a comparison for each condition, neighbours' values through the LDS pipe, two
+// limiter branches, copies from row to row, which two rows of the loop written out spare;
+// four rows are no faster).  2000x2000: 54.9 us a step before, 49.7 now; 1000x800 20.8 and
+// 18.6; FP64 2000x2000 143.5 and 134.3.
 template <typename T>
 __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<T> &bc, const int x0, const int y0,
                                            const int rows, float &dtmin_out) {
     const int lane = threadIdx.x & 63;
-    const bool c1 = bc.cur != 0;
-    T *__restrict__ oe = c1 ? a.e[0] : a.e[1];
-    T *__restrict__ oqx = c1 ? a.qx[0] : a.qx[1];
-    T *__restrict__ oqy = c1 ? a.qy[0] : a.qy[1];
+    const bool c1 = __builtin_amdgcn_readfirstlane(bc.cur) != 0;
     const T dt = (T)bc.dt;
-    const T tnow = (T)bc.t;
-    const int P = a.pitch;
+    const T tnow = Arrival<T>::enc((T)bc.t);
+    const int P = a.pitch * (int)sizeof(T);  // bytes per row
     const int y1 = y0 + rows;
+    // the strip's columns x0-4 .. x0+59 and rows y0-4 .. y1+3 lie inside the grid: no
+    // clamping.  Buffer accesses: the column and the array in the vector offset, the row in
+    // the scalar offset.
+    const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
+    const StateOffsets<T> o(a, c1 ? a.e[1] : a.e[0], a.D, c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0],
+                            c1 ? a.e[0] : a.e[1], c1 ? a.qx[0] : a.qx[1], c1 ? a.qy[0] : a.qy[1]);
+    const int vx = (x0 - SW_HALO + lane) * (int)sizeof(T);
+    const bool out_col = lane >= SW_HALO && lane < SW_HALO + SW_OUT;
+    const int ve = vx + o.e, vD = vx + o.D, vqx = vx + o.qx, vqy = vx + o.qy, vm = vx + o.emax, va = vx + o.arr;
+    const int vout = out_col ? vx : kDropOffset;
+    const int we = vout + o.oe, wqx = vout + o.oqx, wqy = vout + o.oqy;
+    auto load_row = [&](const int so) {
+        RowCell<T> c;
+        c.e = buf_load<T>(rs, ve, so);
+        c.D = buf_load<T>(rs, vD, so);
+        c.qx = buf_load<T>(rs, vqx, so);
+        c.qy = buf_load<T>(rs, vqy, so);
+        return c;
+    };
+    const T eps_h = a.eps_h, dif_at = a.dif_at, cfl2 = T(2) * a.cfl;
+    const bool track = a.track_arrival != 0;
+    const DeepRow<T> *const geo = a.deep_row;
     float dtmin = 3.0e38f;
-    bool valid = true, bad = false;
-    if (x0 < a.nx) {
-        // the strip classification keeps columns x0-4 .. x0+59 and rows y0-4 .. y1+3
-        // inside the grid: no clamping.  Loads are buffer loads: the lane's column is the
-        // vector offset, the row the scalar offset.
-        const __amdgpu_buffer_rsrc_t rs = whole_array(a.block, a.block_bytes);
-        const StateOffsets<T> o(a, c1 ? a.e[1] : a.e[0], a.D, c1 ? a.qx[1] : a.qx[0], c1 ? a.qy[1] : a.qy[0], oe, oqx,
-                                oqy);
-        const int gx = x0 - SW_HALO + lane;
-        const int voff = gx * (int)sizeof(T);
-        // byte addresses of the left and right neighbour lanes for ds_bpermute (the same
-        // moves as from_left / from_right, computed once per strip; FP64 values move as
-        // two dwords through from_left / from_right)
-        const int adl = (lane > 0 ? lane - 1 : lane) << 2, adr = (lane < 63 ? lane + 1 : lane) << 2;
-        auto left = [&](const T v) -> T {
-            if constexpr (sizeof(T) == 4) return __int_as_float(__builtin_amdgcn_ds_bpermute(adl, __float_as_int(v)));
-            else return from_left(v);
-        };
-        auto right = [&](const T v) -> T {
-            if constexpr (sizeof(T) == 4) return __int_as_float(__builtin_amdgcn_ds_bpermute(adr, __float_as_int(v)));
-            else return from_right(v);
-        };
-        auto ld = [&](const int off, const int row) { return buf_load<T>(rs, voff, off + row * P * (int)sizeof(T)); };
-        auto load_row = [&](const int r) {
-            RowCell<T> c;
-            c.e = ld(o.e, r);
-            c.D = ld(o.D, r);
-            c.qx = ld(o.qx, r);
-            c.qy = ld(o.qy, r);
-            return c;
-        };
-        auto metrics_row = [&](const int j) { return j < y0 ? y0 : (j >= y1 ? y1 - 1 : j); };
-        const bool out_col = lane >= SW_HALO && lane < SW_HALO + SW_OUT;
-        const T hpos = a.hpos;
-        // rows y0-4 and y1+3 enter only the branch conditions of the outermost mass faces
-        valid = __all(ld(o.e, y0 - 4) + ld(o.D, y0 - 4) > hpos) && __all(ld(o.e, y1 + 3) + ld(o.D, y1 + 3) > hpos);
-        // pipeline registers: input rows r-2, r-1; h* row r-2 with sqrt(h*), qy/h*;
-        // mass accumulator of row r-1; momentum accumulators of row r-2
-        RowCell<T> i2 = RowCell<T>{T(0), T(0), T(0), T(0)}, i1 = i2;
-        T s2 = T(0), sq2 = T(0), v2 = T(0), m1 = T(0);
-        T X2 = T(0), Y2 = T(0), W2 = T(0);
-        RowCell<T> buf = load_row(y0 - 3);
-        T pm = ld(o.emax, y0), pt = ld(o.arr, y0);
-        // One row of the pipeline.  In the steady state (rows y0+2 .. y1) every stage
-        // applies, so the stage conditions drop out at compile time; the other rows keep
-        // them.  Both forms evaluate the same expressions.
-        auto row = [&](const int r, auto steady_tag) {
-            constexpr bool kS = decltype(steady_tag)::value;
-            const RowCell<T> i0 = buf;
-            buf = load_row((kS || r < y1 + 2) ? r + 1 : r);
-            const int ju = r - 2;  // row updated in this iteration
-            const T cmax = pm, carr = pt;
-            {
-                const int jn = kS ? ju + 1 : metrics_row(ju + 1);
-                pm = ld(o.emax, jn);
-                pt = ld(o.arr, jn);
+    T nan_acc = T(0);  // turns NaN when a stored value is not finite
+    // rows y0-4 and y1+3 enter only the conditions
+    T smin = Num<T>::big;  // of h* (lanes 0 and 63 lack a face and are left out)
+    T emin = tmin(buf_load<T>(rs, ve, (y0 - 4) * P), buf_load<T>(rs, ve, (y1 + 3) * P));
+    T Dmin = tmin(buf_load<T>(rs, vD, (y0 - 4) * P), buf_load<T>(rs, vD, (y1 + 3) * P));
+    // pipeline registers: rows r-2 and r-1 with their depths, h* of row r-2 with sqrt(h*)
+    // and qy/h*, mass accumulator of row r-1, momentum accumulators of row r-2
+    RowCell<T> i2 = RowCell<T>{T(0), T(0), T(0), T(0)}, i1 = i2;
+    T h2 = T(0), h1 = T(0), s2 = T(0), hs2 = T(0), sq2 = T(0), v2 = T(0), m1 = T(0);
+    T X2 = T(0), Y2 = T(0), W2 = T(0);
+    RowCell<T> buf = load_row((y0 - 3) * P);
+    T pm = buf_load<T>(rs, vm, y0 * P), pt = buf_load<T>(rs, va, y0 * P);
+    // One row of the pipeline.  In the steady state (rows y0+2 .. y1) every stage applies,
+    // so the stage conditions drop out at compile time; the other rows keep them.  Both
+    // forms evaluate the same expressions.
+    auto row = [&](const int r, auto steady_tag) {
+        constexpr bool kS = decltype(steady_tag)::value;
+        const RowCell<T> i0 = buf;
+        const DeepRow<T> g = uniform_load(geo + r);
+        const T cmax = pm, carr = pt;
+        {
+            const int rn = (kS || r < y1 + 2) ? r + 1 : r;
+            buf = load_row(rn * P);
+            const int jn = kS ? r - 1 : min(max(r - 1, y0), y1 - 1);
+            pm = buf_load<T>(rs, vm, jn * P);
+            pt = buf_load<T>(rs, va, jn * P);
+        }
+        const int ju = r - 2, j1 = r - 1;  // the row updated in this iteration, the row of h*
+        const T h0 = i0.e + i0.D;
+        emin = Num<T>::min(emin, i0.e);
+        Dmin = Num<T>::min(Dmin, i0.D);
+        // mass x faces of row r (h* rows y0-2 .. y1+1), y face r between rows r-1 and r
+        // (faces y0-2 .. y1+2).  The limiter rarely acts: one test for both faces.
+        T m0 = T(0);
+        if (kS || r >= y0 - 2) {
+            T Fx = dpp_left(i0.qx) * g.ilx, Fy = i1.qy * g.lc0;
+            const T hL = dpp_left(h0);
+            const T limx = (Fx > T(0) ? hL : h0) * g.kA, limy = Fy > T(0) ? h1 * g.k0 : h0 * g.k1;
+            const T denx = habs(Fx) + Num<T>::eps, deny = habs(Fy) + Num<T>::eps;
+            if (__any(dt * denx > limx || dt * deny > limy)) {
+                Fx = limit_flux(Fx, limx, denx, dt);
+                Fy = limit_flux(Fy, limy, deny, dt);
             }
-            const T h0 = i0.e + i0.D;
-            valid = valid && __all(h0 > hpos);
-            // mass x-faces of row r (h* rows y0-2 .. y1+1)
-            T m0 = T(0);
-            if (kS || (r >= y0 - 2 && r <= y1 + 1)) {
-                const RowGeo<T> rg = uniform_load(a.row + r);
-                const T F = fast_mass_x(left(i0.qx), left(h0), h0, rg.ilx, rg.kA, dt);
-                m0 = F - right(F);
-            }
-            // mass y-face g = r between rows r-1 and r (faces y0-2 .. y1+2)
-            if (kS || r >= y0 - 2) {
-                const FaceGeoY<T> fg = uniform_load(a.fy + r);
-                const T F = fast_mass_y(i1.qy, i1.e + i1.D, h0, fg, dt);
-                m1 = Num<T>::mad(-F, fg.ic0, m1);
-                m0 = Num<T>::mad(F, fg.ic1, m0);
-            }
-            // h* of row r-1 (rows y0-2 .. y1+1)
-            T s1 = T(0), hs1 = T(0), sq1 = T(0), u1 = T(0), v1 = T(0);
-            const int j1 = r - 1;
-            const RowGeo<T> rg1 = uniform_load(a.row + ((kS || j1 >= y0 - 2) ? j1 : y0 - 2));
-            if (kS || (j1 >= y0 - 2 && j1 <= y1 + 1)) {
-                T es = Num<T>::mad(dt * rg1.invA, m1, i1.e);
-                if (!(es + i1.D > T(0))) es = -i1.D;
-                s1 = es;
-                hs1 = es + i1.D;
-                valid = valid && __all(hs1 > hpos);
-                sq1 = Num<T>::sqrt(hs1);
-                const T ih = Num<T>::rcp(hs1);
-                u1 = i1.qx * ih;
-                v1 = i1.qy * ih;
-            }
-            // momentum x-faces of row r-1 (rows y0 .. y1-1)
-            T X1 = T(0), Y1 = T(0), W1 = T(0);
-            if (kS || (j1 >= y0 && j1 < y1)) {
-                DC<T> A, B;
-                A.h = left(hs1); A.e = left(s1); A.D = left(i1.D);
-                A.qn = left(i1.qx); A.qt = left(i1.qy); A.s = left(sq1); A.un = left(u1);
-                B.h = hs1; B.e = s1; B.D = i1.D; B.qn = i1.qx; B.qt = i1.qy; B.s = sq1; B.un = u1;
-                const MF<T> f = fast_mom_x(A, B, rg1.ilx, rg1.kdx, dt);
-                X1 = -f.pn - right(f.mn);
-                Y1 = -f.pt - right(f.mt);
-                W1 = f.w + right(f.w);
-            }
-            // momentum y-face g = r-1 between rows r-2 and r-1 (faces y0 .. y1)
-            if (kS || (j1 >= y0 && j1 <= y1)) {
-                const FaceGeoY<T> fg = uniform_load(a.fy + j1);
-                DC<T> A, B;
-                A.h = s2 + i2.D; A.e = s2; A.D = i2.D; A.qn = i2.qy; A.qt = i2.qx; A.s = sq2; A.un = v2;
-                B.h = hs1; B.e = s1; B.D = i1.D; B.qn = i1.qy; B.qt = i1.qx; B.s = sq1; B.un = v1;
-                const MF<T> f = fast_mom_y(A, B, fg, dt);
-                Y2 -= f.mn;
-                X2 -= f.mt;
-                W2 += f.w;
-                Y1 -= f.pn;
-                X1 -= f.pt;
-                W1 += f.w;
-            }
-            // cell update of row r-2 (src/GPU/Volumen_kernel.cu:160-221; h* > hpos here).
-            // Every iteration issues the five stores; those of halo rows and halo lanes,
-            // and metric stores that do not apply, are dropped.
-            {
-                const bool in_rows = kS || (ju >= y0 && ju < y1);
-                const bool on = in_rows && out_col;
-                const int jr = in_rows ? ju : y0;  // a row inside the arrays
-                const RowGeo<T> rg = uniform_load(a.row + jr);
-                const int soff = jr * P * (int)sizeof(T);
-                const T D = i2.D, eo = i2.e;
-                buf_store<T>(eo, rs, voff, o.emax + soff, on && eo > cmax && eo + D > a.eps_h);
-                buf_store<T>(Arrival<T>::enc(tnow), rs, voff, o.arr + soff,
-                              on && a.track_arrival && !Arrival<T>::arrived(carr) && tabs(eo - carr) > a.dif_at);
-                const T dtc = (W2 < Num<T>::eps) ? Num<T>::big : Num<T>::div(T(2) * a.cfl * rg.A, W2);
-                dtmin = in_rows ? fminf(dtmin, (float)dtc) : dtmin;  // halo lanes are dropped after the loop
-                const T val = dt * rg.invA;
-                const T qx = Num<T>::mad(val, X2, i2.qx), qy = Num<T>::mad(val, Y2, i2.qy);
-                bad = bad || (on && bad_cell(s2, qx, qy));
-                buf_store<T>(s2, rs, voff, o.oe + soff, on);
-                buf_store<T>(qx, rs, voff, o.oqx + soff, on);
-                buf_store<T>(qy, rs, voff, o.oqy + soff, on);
-            }
-            i2 = i1; i1 = i0;
-            s2 = s1; sq2 = sq1; v2 = v1;
-            m1 = m0;
-            X2 = X1; Y2 = Y1; W2 = W1;
-        };
-        using Edge = std::integral_constant<bool, false>;
-        using Steady = std::integral_constant<bool, true>;
-        // Enter the loops with no memory instruction outstanding: the wait before a row
-        // then only has the previous rows to account for (their stores may stay in flight
-        // while the next row loads), instead of a full wait every row.
-        __builtin_amdgcn_s_waitcnt(0);
-        // rows y0-3 .. y1+2: the halo rows at either end with the stage conditions, the
-        // steady state without them
-        const int pe = min(y0 + 1, y1 + 2);
-        int r = y0 - 3;
-        for (; r <= pe; r++) row(r, Edge{});
+            m0 = here(Fx - dpp_right(Fx));
+            m1 = Num<T>::mad(-Fy, g.ic0, m1);
+            m0 = Num<T>::mad(Fy, g.ic1, m0);
+        }
+        // h* of row r-1 (rows y0-2 .. y1+1)
+        T s1 = T(0), hs1 = T(0), sq1 = T(0), u1 = T(0), v1 = T(0);
+        if (kS || (j1 >= y0 - 2 && j1 <= y1 + 1)) {
+            s1 = Num<T>::mad(dt * g.p.invA, m1, i1.e);
+            smin = Num<T>::min(smin, s1);
+            hs1 = s1 + i1.D;
+            sq1 = Num<T>::sqrt(hs1);
+            const T ih = Num<T>::rcp(hs1);
+            u1 = i1.qx * ih;
+            v1 = i1.qy * ih;
+        }
+        // momentum x faces of row r-1 (rows y0 .. y1-1)
+        T X1 = T(0), Y1 = T(0), W1 = T(0);
+        if (kS || (j1 >= y0 && j1 < y1)) {
+            const DC<T> A{dpp_left(hs1), dpp_left(i1.qx), dpp_left(i1.qy), dpp_left(sq1), dpp_left(u1)};
+            const DC<T> B{hs1, i1.qx, i1.qy, sq1, u1};
+            const MF<T> f = fast_mom_x(A, B, s1 - dpp_left(s1), g.p.ilx, g.p.kdx, dt);
+            X1 = here(-f.pn - dpp_right(f.mn));
+            Y1 = here(-f.pt - dpp_right(f.mt));
+            W1 = here(f.w + dpp_right(f.w));
+        }
+        // momentum y face r-1 between rows r-2 and r-1 (faces y0 .. y1)
+        if (kS || (j1 >= y0 && j1 <= y1)) {
+            const DC<T> A{hs2, i2.qy, i2.qx, sq2, v2}, B{hs1, i1.qy, i1.qx, sq1, v1};
+            const MF<T> f = fast_mom_y(A, B, s1 - s2, g.p, dt);
+            Y2 -= f.mn;
+            X2 -= f.mt;
+            W2 += f.w;
+            Y1 -= f.pn;
+            X1 -= f.pt;
+            W1 += f.w;
+        }
+        // cell update of row r-2 (src/GPU/Volumen_kernel.cu:160-221; h* > hpos here).  Every
+        // iteration issues the five stores; those of halo rows and halo lanes, and metric
+        // stores that do not apply, are dropped.
+        {
+            const bool on = kS || (ju >= y0 && ju < y1);
+            const int so = (kS || on ? ju : y0) * P;
+            const T eo = i2.e;
+            const bool max_on = on && eo > cmax && h2 > eps_h;
+            const bool arr_on = on && track && !Arrival<T>::arrived(carr) && habs(eo - carr) > dif_at;
+            buf_store<T>(eo, rs, (max_on ? vout : kDropOffset) + o.emax, so);
+            buf_store<T>(tnow, rs, (arr_on ? vout : kDropOffset) + o.arr, so);
+            if (on) dtmin = Num<float>::min(dtmin, (float)Num<T>::div(cfl2 * g.q.A, W2));  // halo lanes: dropped below
+            const T val = dt * g.q.invA;
+            const T qx = Num<T>::mad(val, X2, i2.qx), qy = Num<T>::mad(val, Y2, i2.qy);
+            if (on) nan_acc = Num<T>::mad(s2, T(0), Num<T>::mad(qx, T(0), Num<T>::mad(qy, T(0), nan_acc)));
+            buf_store<T>(s2, rs, kS || on ? we : kDropOffset, so);
+            buf_store<T>(qx, rs, kS || on ? wqx : kDropOffset, so);
+            buf_store<T>(qy, rs, kS || on ? wqy : kDropOffset, so);
+        }
+        i2 = i1; i1 = i0;
+        h2 = h1; h1 = h0;
+        s2 = s1; hs2 = hs1; sq2 = sq1; v2 = v1;
+        m1 = m0;
+        X2 = X1; Y2 = Y1; W2 = W1;
+        // rows are not mixed: that would hold the registers of several at once
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using Edge = std::integral_constant<bool, false>;
+    using Steady = std::integral_constant<bool, true>;
+    // Enter the loops with no memory instruction outstanding: the wait before a row then
+    // only has the previous rows to account for (their stores may stay in flight while the
+    // next row loads), instead of a full wait every row.
+    __builtin_amdgcn_s_waitcnt(0);
+    // rows y0-3 .. y1+2: the halo rows at either end (and a last row without a partner)
+    // with the stage conditions, the steady state without them
+    int r = y0 - 3;
 #pragma unroll 1
-        for (; r <= y1; r++) row(r, Steady{});
-        for (; r <= y1 + 2; r++) row(r, Edge{});
-        dtmin = out_col ? dtmin : 3.0e38f;
+    for (; r <= y0 + 1; r++) row(r, Edge{});
+#pragma unroll 1
+    for (; r + 1 <= y1; r += 2) {
+        row(r, Steady{});
+        row(r + 1, Steady{});
     }
+#pragma unroll 1
+    for (; r <= y1 + 2; r++) row(r, Edge{});
+    // (the minima are taken over the wavefront first: a face joins the eta of one lane with
+    // the depth of another)
+    const T floor_h = wave_min(lane == 0 || lane == 63 ? emin : Num<T>::min(emin, smin)) + wave_min(Dmin);
+    const bool valid = floor_h > tmax(a.hpos, T(kDeepFloor));
     // a strip whose check failed is redone, and checked, as general tiles
-    if (valid) raise_health(a, bad);
-    dtmin_out = dtmin;
+    if (valid) raise_health(a, out_col && nan_acc != nan_acc);
+    dtmin_out = out_col ? dtmin : 3.0e38f;
     return valid;
 }
 
