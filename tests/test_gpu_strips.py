@@ -46,3 +46,13 @@ def test_failed_strips(spot, precision):
     assert np.all(np.isfinite(a[0])) and np.max(np.abs(a[1])) > 0
     for p, q in zip(a, b):
         assert np.array_equal(p, q)
+
+
+def test_rows_beyond_the_pole():
+    """A grid that runs past the pole has rows of negative area and length, whose wave speeds
+    sum to less than the guard of a cell's dt: such cells set no dt."""
+    pr = make_problem(nx=300, ny=200, seed=9, coast=(), lat0=85.0)
+    a = _run(pr, 7)
+    b = _run(pr, 7, kernel="sweep_general")
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)

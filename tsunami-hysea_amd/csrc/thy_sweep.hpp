@@ -725,10 +725,6 @@ __device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slo
 // with the same functions, so the split changes no result.
 // ---------------------------------------------------------------------------
 
-// Least depth of a deep-water strip whatever hpos is: far below any depth of use, and far
-// enough above zero that the wave speeds of a cell sum to more than the guard of its dt.
-constexpr double kDeepFloor = 1e-12;
-
 // the value, computed where it is written (a cross-lane move folds into an instruction of
 // its own basic block only)
 __device__ __forceinline__ float here(float v) { asm("" : "+v"(v)); return v; }
@@ -751,7 +747,7 @@ __device__ __forceinline__ double here(double v) { return v; }
 //
 // Bound by memory on a large grid (4000x3000, all deep: 111 us a step, 3.9 TB/s of the nine
 // arrays, whatever the strip height, and no less with two rows of cells in flight), by the
-// latency of a row on a small one.  A steady row takes 132 vector instructions (175 before:
+// latency of a row on a small one.  A steady row takes 134 vector instructions (175 before:
 // a vote and a comparison for each condition, neighbours' values through the LDS pipe, two
 // limiter branches, copies from row to row, which two rows of the loop written out spare;
 // four rows are no faster).  2000x2000: 54.9 us a step before, 49.7 now; 1000x800 20.8 and
@@ -878,7 +874,8 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
             const bool arr_on = on && track && !Arrival<T>::arrived(carr) && habs(eo - carr) > dif_at;
             buf_store<T>(eo, rs, (max_on ? vout : kDropOffset) + o.emax, so);
             buf_store<T>(tnow, rs, (arr_on ? vout : kDropOffset) + o.arr, so);
-            if (on) dtmin = Num<float>::min(dtmin, (float)Num<T>::div(cfl2 * g.q.A, W2));  // halo lanes: dropped below
+            const T dtc = W2 < Num<T>::eps ? Num<T>::big : Num<T>::div(cfl2 * g.q.A, W2);
+            if (on) dtmin = Num<float>::min(dtmin, (float)dtc);  // halo lanes: dropped below
             const T val = dt * g.q.invA;
             const T qx = Num<T>::mad(val, X2, i2.qx), qy = Num<T>::mad(val, Y2, i2.qy);
             if (on) nan_acc = Num<T>::mad(s2, T(0), Num<T>::mad(qx, T(0), Num<T>::mad(qy, T(0), nan_acc)));
@@ -915,7 +912,7 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
     // (the minima are taken over the wavefront first: a face joins the eta of one lane with
     // the depth of another)
     const T floor_h = wave_min(lane == 0 || lane == 63 ? emin : Num<T>::min(emin, smin)) + wave_min(Dmin);
-    const bool valid = floor_h > tmax(a.hpos, T(kDeepFloor));
+    const bool valid = floor_h > tmax(a.hpos, T(0));
     // a strip whose check failed is redone, and checked, as general tiles
     if (valid) raise_health(a, out_col && nan_acc != nan_acc);
     dtmin_out = out_col ? dtmin : 3.0e38f;
