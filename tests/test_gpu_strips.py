@@ -56,3 +56,13 @@ def test_rows_beyond_the_pole():
     b = _run(pr, 7, kernel="sweep_general")
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("nx,ny,precision", [(2803, 2701, 0), (1997, 1901, 1)])
+def test_strips_in_reverse_order(nx, ny, precision):
+    """State above the size from which every other step walks the strips backwards."""
+    pr = make_problem(nx=nx, ny=ny, seed=9, coast=("north",))
+    a = _run(pr, 7, precision=precision)
+    b = _run(pr, 7, precision=precision, kernel="sweep_general")
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)

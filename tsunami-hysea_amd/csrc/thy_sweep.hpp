@@ -964,12 +964,16 @@ __device__ __forceinline__ float tile_or_strips(const ArgsAt<T> args, const Bloc
 
 // Work items, one per workgroup: a general tile (x0, y0 << 4 | rows), or four deep-water
 // strips (index of the first in the strip list, 0).  `strip`: a deep item's strip of this
-// wavefront; x0 < 0: none.
-template <typename T> __device__ __forceinline__ int2 item_origin(const StepArgs<T> &a, const int2 it, bool &tile, int &rows) {
+// wavefront; x0 < 0: none.  flip > 0: the strips in reverse order, in place of the item's
+// those mirrored over the list's `flip` groups of 8 items (an item of the same XCD).
+template <typename T>
+__device__ __forceinline__ int2 item_origin(const StepArgs<T> &a, const int2 it, bool &tile, int &rows, const int flip) {
     rows = it.y & 15;
     tile = rows != 0;
     if (tile) return make_int2(it.x, it.y >> 4);
-    const int2 strip = uniform_load(a.deep + it.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    const int g = it.x / SW_WAVES;
+    const int first = flip > 0 ? ((flip - 1 - (g >> 3)) * 8 + (g & 7)) * SW_WAVES : it.x;
+    const int2 strip = uniform_load(a.deep + first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     rows = strip.y & 2047;
     return make_int2(strip.x, strip.y >> 11);
 }
@@ -977,7 +981,7 @@ template <typename T> __device__ __forceinline__ int2 item_origin(const StepArgs
 // One step of one grid in one launch, a workgroup per work item.  Workgroup 0 is the
 // step's writer.
 template <typename T>
-__global__ void __launch_bounds__(64 * SW_WAVES, sizeof(T) == 4 ? 5 : 2) k_sweep(const StepArgs<T> args_, const int slot) {
+__global__ void __launch_bounds__(64 * SW_WAVES, sizeof(T) == 4 ? 5 : 2) k_sweep(const StepArgs<T> args_, const int slot, const int flip) {
     __shared__ TileLds<T> s;
     __shared__ BlockCtl<T> bc;
     __shared__ float s_red[SW_WAVES];
@@ -990,7 +994,7 @@ __global__ void __launch_bounds__(64 * SW_WAVES, sizeof(T) == 4 ? 5 : 2) k_sweep
     if (tid == 0) begin_step(a, slot, bid == 0, bc, kDtParts);
     bool tile;
     int rows;
-    const int2 o = item_origin(a, w, tile, rows);
+    const int2 o = item_origin(a, w, tile, rows, flip);
     __syncthreads();
     if (!bc.run) return;
     if (bid == 0) {
@@ -1036,7 +1040,7 @@ __global__ void __launch_bounds__(64 * SW_WAVES, 5) k_batch(const BatchArgs q, c
     if (tid == 0) begin_step(a, slot, w.writer != 0, bc, kDtParts);
     bool tile;
     int rows;
-    const int2 o = item_origin(a, w.it, tile, rows);
+    const int2 o = item_origin(a, w.it, tile, rows, 0);
     __syncthreads();
     if (!bc.run) return;
     if (w.writer) {
