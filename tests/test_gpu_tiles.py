@@ -73,3 +73,21 @@ def test_land(lake):
         out.append((s.field("arrival_times"), s.field("max_height")))
         s.close()
     assert np.array_equal(out[0][0] < 0, out[1][0] < 0) and np.array_equal(out[0][1] < -9000, out[1][1] < -9000)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny", [(700, 300), (300, 130), (90, 45)])
+def test_tiles_of_mixed_heights(nx, ny, precision):
+    """Tiles made lower along the coast (the default) against tiles of one height, of eight
+    rows and of five: the same faces and the same sums, bit for bit."""
+    from thysea import native
+    pr = make_problem(nx=nx, ny=ny, seed=nx, coast=("north", "east"))
+    out = []
+    for rows in (0, 8, 5):
+        s = native.Solver(pr, general_rows=rows, precision=precision)
+        s.run(max_steps=18, steps_per_sync=6)
+        out.append(s.state() + (s.field("max_height"), s.field("arrival_times")))
+        s.close()
+    for o in out[1:]:
+        for x, y in zip(out[0], o):
+            assert np.array_equal(x, y)

@@ -395,22 +395,32 @@ int pick_tile(thy_ctx *c) {
 
 // Rows per deep-water strip of a grid of `rows` segment rows (56-column segments times
 // rows) that is stepped alone.  A strip's time is a chain of rows with a halo of 5: with few
-// rows the step is the time of one strip, so strips are short; with many they are as tall as
-// leaves the device one round of them (20 wavefronts a CU).  Measured (us per step):
-// 1000x800 (14400) 19.8 / 25.2 / 32.7 at 8 / 16 / 24 rows; 2000x2000 (72000) 58.9 / 54.7 /
-// 54.2 / 62.2 at 8 / 16 / 24 / 32; 4000x3000 (216000) 139.6 / 132.0 / 141.6 at 16 / 32 / 48.
+// rows the step is the time of one strip, so strips are short; with many the halo's work
+// counts.  Measured (us per step): 1000x800 (14400 rows) 17.2 / 19.3 / 19.4 at 8 / 12 / 16
+// rows; 1400x1200 (30000) 28.7 / 26.4 / 31.9 at 8 / 16 / 24; 2000x2000 (72000) 47.7 / 46.6 /
+// 48.0 at 16 / 24 / 28, FP64 124.2 / 118.9 / 122.4 at 16 / 24 / 32; 2500x2500 (112500) 59.2 /
+// 59.0 / 66.5 at 16 / 24 / 32; 4000x3000 (216000) 126.0 / 135.8 / 122.4 / 139.5 at 16 / 24 /
+// 32 / 40.
 int default_strip_rows(const size_t rows, const int ncu) {
-    const size_t per = rows / ((size_t)ncu * 20);
-    return (int)std::min<size_t>(32, std::max<size_t>(8, (per + 4) / 8 * 8));
+    const size_t per = rows / ncu;
+    return per < 80 ? 8 : (per < 200 ? 16 : (per < 560 ? 24 : 32));
 }
 
-// rows per general tile of a grid stepped alone: half tiles while the tiles are few enough
-// to run side by side (the step then waits for one of them: 240x200 14.3 against 17.7 us,
-// 1501x607 21.4 against 34.7), whole ones, with less halo, when they are many (2000x2000
-// 58.9 against 65.0 us)
+// Rows per general tile of a grid stepped alone.  Whole tiles have the least halo.  On a
+// small grid the step is the time of one tile, so tiles are lower there, the more the
+// smaller it is (240x200, 3.9 segment rows a CU: 12.8 / 13.3 / 15.3 us at 3 / 4 / 8 rows;
+// 1000x800, 56 rows: 19.1 / 17.2 at 4 / 8).
 int default_tile_rows(const size_t rows, const int ncu) {
-    return rows <= (size_t)ncu * 128 ? kTileRows / 2 : kTileRows;
+    return (int)std::min<size_t>(kTileRows, 3 + rows / ((size_t)ncu * 8));
 }
+
+// Listed faces (the estimate of find_coast) above which a tile of a grid stepped alone is
+// made lower, down to kTileLow rows: the step would wait for the tiles along the coast.
+// Above about 130 segment rows a CU no tile reaches it: many tiles share a CU there, and
+// lower ones only add halo.  Us a step without this rule and with it: 1501x607 29.4 and
+// 19.2, 800x900 27.7 and 17.0, 731x412 17.8 and 15.4, 1000x800 16.9 and 16.6.
+constexpr int kTileLow = 3;
+int tile_budget(const size_t rows, const int ncu) { return (int)std::min<size_t>(100000, 5 * rows / ncu); }
 
 // items in order, dealt in eight runs of (nearly) equal length, one per XCD: the workgroup
 // at list slot b runs on XCD b mod 8, so each XCD sweeps one contiguous band and items side
@@ -497,12 +507,13 @@ void find_coast(thy_ctx *c, const T *D) {
     }
 }
 
-// Work lists with deep-water strips of up to S rows and tiles of up to R rows.  Each
+// Work lists with deep-water strips of up to S rows and tiles of up to R rows (above
+// kTileLow only as many as keep the tile's cost within `budget`).  Each
 // segment's column is cut into blocks of 8 rows between the border bands; a block is deep
 // when its rows y0-4 .. y1+3 and its 64 columns are clear of the grid edges (no clamping,
 // no first-order band), of the sponges, and of coast.  Runs of deep blocks become strips of
 // nearly equal height, the rest tiles, in order of their cost.
-int build_lists(thy_ctx *ctx, WorkLists &w, int S, const int R) {
+int build_lists(thy_ctx *ctx, WorkLists &w, int S, const int R, const int budget) {
     const int nx = ctx->nx, ny = ctx->ny;
     const int nseg = (nx + SW_OUT - 1) / SW_OUT;
     const int spi = ctx->prm.sponge_izq, spd = ctx->prm.sponge_der, sps = ctx->prm.sponge_sup, spn = ctx->prm.sponge_inf;
@@ -514,10 +525,15 @@ int build_lists(thy_ctx *ctx, WorkLists &w, int S, const int R) {
     const int ya = std::max(6, sps + 2), yb = ny - std::max(6, spn + 2);  // rows a deep block may take
     std::vector<int2> strips;
     std::vector<std::pair<int, int2>> tiles;  // (cost, tile)
+    // listed faces of rows y .. y+n-1 with the halo, those of the first-order bands included
+    auto cost = [&](const int sgi, const int y, const int n) {
+        return between(ctx->cost, sgi, y - 2, y + n + 2) + (y < 4 ? 3 * SW_OUT : 0) + (y + n > ny - 4 ? 3 * SW_OUT : 0);
+    };
     auto add_tiles = [&](const int sgi, const int y0, const int y1) {
-        for (int y = y0; y < y1; y += R) {
-            const int n = std::min(R, y1 - y);
-            tiles.emplace_back(between(ctx->cost, sgi, y - 2, y + n + 2), make_int2(sgi * SW_OUT, y << 4 | n));
+        for (int y = y0, n; y < y1; y += n) {
+            n = std::min(R, y1 - y);
+            while (n > kTileLow && cost(sgi, y, n) > budget) n--;
+            tiles.emplace_back(cost(sgi, y, n), make_int2(sgi * SW_OUT, y << 4 | n));
         }
     };
     for (int sgi = 0; sgi < nseg; sgi++) {
@@ -568,8 +584,10 @@ int build_alone(thy_ctx *ctx, const int S, const int R) {
     ctx->srows = S;
     ctx->trows = R;
     // where the default is the shortest strip, taller ones only leave the device idle
-    const int def = default_strip_rows(segment_rows(ctx), ctx->ncu);
-    return build_lists(ctx, ctx->alone, def <= 8 ? std::min(S, def) : S, R);
+    const size_t rows = segment_rows(ctx);
+    const int def = default_strip_rows(rows, ctx->ncu);
+    const int budget = ctx->prm.general_rows > 0 ? INT_MAX : tile_budget(rows, ctx->ncu);
+    return build_lists(ctx, ctx->alone, def <= 8 ? std::min(S, def) : S, R, budget);
 }
 
 // the lists of an uploaded state
@@ -588,7 +606,7 @@ int build_order(thy_ctx *ctx, const T *D) {
 // grids: tiles are whole, and strips of 16 rows cost the least (24 scenarios of 1000x800:
 // 128.6 / 123.0 / 126.4 / 126.4 / 133.3 ms at 8 / 16 / 24 / 32 / 48 rows).
 int build_batched(thy_ctx *ctx) {
-    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 16, kTileRows);
+    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 16, kTileRows, INT_MAX);
 }
 
 template <typename T>
