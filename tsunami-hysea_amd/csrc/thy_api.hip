@@ -15,12 +15,18 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/thysea.h"
@@ -813,6 +819,95 @@ int initial_dt_t(thy_ctx *ctx, double *dt) {
     return THY_OK;
 }
 
+// A large device buffer into the caller's pageable memory.  The runtime's own copy goes
+// through one thread (or pins the caller's pages); here the data passes through pinned memory
+// in chunks, and several threads copy them on, so that the page faults of a new buffer are
+// taken side by side too.  The helper threads make no HIP calls and have ended on return.
+// Two fields of 4000x3000 into new arrays: 7.5 to 9.8 ms before, 3.3 now (29 GB/s); of
+// 2000x2000 1.95 and 1.25; 1500x1400 (8.4 MB) 1.05 and 0.85; of 1400x1200 (6.7 MB, below the
+// line) the runtime's copy takes 0.82.
+constexpr size_t kChunk = 2u << 20, kLargeCopy = 8u << 20;
+constexpr int kCopyThreads = 8;
+
+int read_large(thy_ctx *ctx, char *out, const char *src, const size_t bytes) {
+    const int n = (int)((bytes + kChunk - 1) / kChunk);
+    struct Run {
+        hipStream_t q;
+        char *pin = nullptr;
+        std::vector<hipEvent_t> ev;        // one per slot
+        std::vector<std::thread> helpers;
+        std::atomic<int> ready{0}, next{0};  // chunks that have arrived; the next to be copied on
+        std::unique_ptr<std::atomic<bool>[]> done;
+        std::atomic<bool> stop{false};
+        void join() {
+            for (std::thread &t : helpers) t.join();
+            helpers.clear();
+        }
+        ~Run() {
+            stop = true;
+            join();
+            (void)hipStreamSynchronize(q);
+            for (hipEvent_t e : ev) (void)hipEventDestroy(e);
+            Pool::get().host_free(pin);
+        }
+    } run;
+    run.q = ctx->stream;
+    // the block that staged the upload of the state, if it is there; else a smaller one
+    size_t room = 4 * (size_t)ctx->pitch * ctx->ny * ctx->esz;
+    run.pin = (char *)Pool::get().host_cached(room);
+    if (!run.pin) {
+        room = 8 * kChunk;
+        HIPCHK(Pool::get().host_alloc((void **)&run.pin, room));
+    }
+    const int slots = (int)std::min<size_t>({room / kChunk, (size_t)n, (size_t)64});
+    run.done.reset(new std::atomic<bool>[n]);
+    for (int i = 0; i < n; i++) run.done[i] = false;
+    for (int i = 0; i < slots; i++) {
+        hipEvent_t e;
+        HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        run.ev.push_back(e);
+    }
+    auto size_of = [&](const int c) { return std::min(kChunk, bytes - (size_t)c * kChunk); };
+    auto copy_on = [&](const int c) {
+        memcpy(out + (size_t)c * kChunk, run.pin + (size_t)(c % slots) * kChunk, size_of(c));
+        run.done[c] = true;
+    };
+    auto helper = [&] {
+        for (;;) {
+            const int c = run.next++;
+            if (c >= n) return;
+            while (run.ready <= c) {
+                if (run.stop) return;
+                std::this_thread::yield();
+            }
+            copy_on(c);
+        }
+    };
+    try {
+        const int cpus = (int)std::thread::hardware_concurrency();
+        for (int t = 0; t < std::min({kCopyThreads, std::max(1, cpus / 2), n}); t++) run.helpers.emplace_back(helper);
+    } catch (const std::system_error &) {
+        // as many as there are; with none this thread copies
+    }
+    for (int c = 0, sent = 0; c < n; c++) {
+        for (; sent < n && (sent < slots || run.done[sent - slots]); sent++) {
+            HIPCHK(hipMemcpyAsync(run.pin + (size_t)(sent % slots) * kChunk, src + (size_t)sent * kChunk, size_of(sent),
+                                  hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(hipEventRecord(run.ev[sent % slots], ctx->stream));
+        }
+        if (c >= sent) {  // its slot is still being copied on
+            std::this_thread::yield();
+            c--;
+            continue;
+        }
+        HIPCHK(hipEventSynchronize(run.ev[c % slots]));
+        run.ready = c + 1;
+        if (run.helpers.empty()) copy_on(c);
+    }
+    run.join();
+    return THY_OK;
+}
+
 template <typename T>
 int get_field_t(thy_ctx *ctx, int field, float *out) {
     const int64_t n = (int64_t)ctx->nx * ctx->ny;
@@ -825,6 +920,13 @@ int get_field_t(thy_ctx *ctx, int field, float *out) {
                        (const T *)ctx->emax, (const T *)ctx->arr, ctx->nx, ctx->ny, ctx->pitch, (T)ctx->prm.eps_h,
                        ctx->prm.H, ctx->prm.Q, ctx->prm.T, ctx->outbuf);
     HIPCHK(hipGetLastError());
+    if (n * sizeof(float) >= kLargeCopy) {
+        try {
+            return read_large(ctx, (char *)out, (const char *)ctx->outbuf, n * sizeof(float));
+        } catch (const std::bad_alloc &) {
+            return fail(ctx, THY_ERR_HOST_MEMORY, "no host memory to read a field");
+        }
+    }
     HIPCHK(hipMemcpyAsync(out, ctx->outbuf, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return THY_OK;
