@@ -66,3 +66,18 @@ def test_strips_in_reverse_order(nx, ny, precision):
     b = _run(pr, 7, precision=precision, kernel="sweep_general")
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("n", [1, 3, 5])
+def test_batch_in_reverse_order(n):
+    """Batches below and above the size from which every other step walks the strips
+    backwards, the first scenario without a coast, against each scenario alone."""
+    from thysea import serving
+    prs = [make_problem(nx=1450 + 57 * i, ny=1310 - 31 * i, seed=9 + i, coast=("north", "east") if i else (), t_sim=60.0)
+           for i in range(n)]
+    rec_b, res_b, _ = serving.run_batched(prs, steps_per_sync=6, keep=range(n))
+    rec_s, res_s = serving.run_sequential(prs, steps_per_sync=6, keep=range(n))
+    for i in range(n):
+        assert rec_b[i]["steps"] == rec_s[i]["steps"] > 6
+        for key in ("max_height", "arrival_times"):
+            assert np.array_equal(res_b[i][key], res_s[i][key]), (i, key)

@@ -445,26 +445,30 @@ std::vector<int2> xcd_runs(const std::vector<int2> &items, const int per) {
     return out;
 }
 
-// A step's work items.  What takes longest goes first, so that the short items fill in at
-// the end: a tile takes 10 to 25 us, a strip of deep water about 1 us a row.  Strips of up to
-// 8 rows follow the tiles; taller ones start with them, the tiles spread behind (`lag` times
-// thinner than even: tiles are bound by arithmetic, strips by memory, and side by side they
-// share a CU).  4000x3000 at 32 rows: 160 us tiles first, 147 strips first, 135 lag 2;
-// 2000x2000 at 16 rows: 60.1, 64.4, 57.6 lag 1.5.  Groups of 8 start on the same XCD.
+// The order of a step's work items, in groups of 8 that start on the same XCD.  What takes
+// longest goes first, so that the short items fill in at the end: a tile takes 10 to 25 us, a
+// strip of deep water about 1 us a row.  Tall strips start with the tiles, those spread
+// behind, `lag` times thinner than even: tiles are bound by arithmetic, strips by memory, and
+// side by side they share a CU.  With lag 0 the tiles go first.  emit(tile, i): the next item
+// is the i-th of its kind, or none (i < 0).
+template <typename F> void spread_items(const size_t n_tiles, const size_t n_strips, const double lag, const F &emit) {
+    const size_t tg = (n_tiles + 7) / 8, dg = (n_strips + 7) / 8;
+    for (size_t t = 0, d = 0; t < tg || d < dg;) {
+        const bool tile = t < tg && (d >= dg || (double)t * dg * lag <= (double)d * tg);
+        const size_t g = tile ? t++ : d++, n = tile ? n_tiles : n_strips;
+        for (size_t k = g * 8; k < g * 8 + 8; k++) emit(tile, k < n ? (int)k : -1);
+    }
+}
+
+// The items of a grid stepped alone.  Strips of up to 8 rows follow the tiles.  4000x3000 at
+// 32 rows: 160 us tiles first, 147 strips first, 135 lag 2; 2000x2000 at 16 rows: 60.1, 64.4,
+// 57.6 lag 1.5.
 std::vector<int2> interleave(const std::vector<int2> &tiles, const int n_deep, const int strip_rows) {
     std::vector<int2> out;
     const double lag = strip_rows <= 8 ? 0.0 : (strip_rows <= 16 ? 1.5 : 2.0);
-    const size_t tg = (tiles.size() + 7) / 8, dg = (n_deep + 7) / 8;
-    size_t t = 0, d = 0;
-    while (t < tg || d < dg) {
-        const bool tile = t < tg && (d >= dg || (double)t * dg * lag <= (double)d * tg);
-        for (size_t k = 0; k < 8; k++) {
-            if (tile && t * 8 + k < tiles.size()) out.push_back(tiles[t * 8 + k]);
-            if (!tile && (int)(d * 8 + k) < n_deep) out.push_back(make_int2((int)(d * 8 + k) * SW_WAVES, 0));
-        }
-        if (tile) t++;
-        else d++;
-    }
+    spread_items(tiles.size(), n_deep, lag, [&](const bool tile, const int i) {
+        if (i >= 0) out.push_back(tile ? tiles[i] : make_int2(i * SW_WAVES, 0));
+    });
     return out;
 }
 
@@ -609,10 +613,10 @@ int build_order(thy_ctx *ctx, const T *D) {
 }
 
 // The lists a batch steps the scenario by.  Its scenarios fill the device whatever their
-// grids: tiles are whole, and strips of 16 rows cost the least (24 scenarios of 1000x800:
-// 128.6 / 123.0 / 126.4 / 126.4 / 133.3 ms at 8 / 16 / 24 / 32 / 48 rows).
+// grids: tiles are whole, and strips of 24 rows cost the least (GPU time of 24 scenarios of
+// 1000x800: 88.0 / 86.3 / 85.7 ms at 16 / 24 / 32 rows; a mix of 12 grids 76.9 / 75.8 / 76.6).
 int build_batched(thy_ctx *ctx) {
-    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 16, kTileRows, INT_MAX);
+    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 24, kTileRows, INT_MAX);
 }
 
 template <typename T>
@@ -1765,7 +1769,7 @@ struct thy_batch {
     BatchItem *d_items = nullptr;   // a workgroup's work each; the captured grid covers item_cap
     int *d_count = nullptr;         // items in the list
     int item_cap = 0;
-    std::vector<BatchItem> h_items;
+    std::vector<BatchItem> h_items, h_back;  // of even and of odd steps: the halves of d_items
     int h_count = 0;
     Ctrl *d_ctrl = nullptr;
     Ctrl *h_ctrl = nullptr;              // pinned: control blocks gathered after a launch
@@ -1801,10 +1805,13 @@ int list_cap(size_t n) {
     return c;
 }
 
-// The workgroups of the running scenarios: every general tile, costliest cost class first,
-// then the deep-water strips, scenario by scenario, four to a workgroup in the scenario's
-// own order (its runs per XCD: each scenario starts at a multiple of 8).  A scenario's
-// writer is its first item.
+// The workgroups of the running scenarios: the general tiles of all, costliest first, spread
+// among the deep-water strips, scenario by scenario, four to a workgroup in the scenario's own
+// order (its runs per XCD: each scenario starts at a multiple of 8).  A scenario's writer is
+// its first item.  The second half of the list, for every other step, has the strips in
+// reverse where the states together exceed the cache (as in launch_step_t).  24 scenarios of
+// 1000x800, GPU time: 97.2 ms with the tiles first, 89.3 spread, 88.0 with every other step
+// reversed, 86.3 with strips of 24 rows too; a mix of 12 grids 85.9, 78.7, 76.9, 75.8.
 int batch_items(thy_batch *b) {
     struct G { int cls; BatchItem it; };
     std::vector<G> gv;
@@ -1819,15 +1826,26 @@ int batch_items(thy_batch *b) {
             gv.push_back({w.tcost_h[p], BatchItem{i, p == 0 ? 1 : 0, w.tile_h[p]}});
     }
     std::stable_sort(gv.begin(), gv.end(), [](const G &x, const G &y) { return x.cls > y.cls; });
-    for (const G &g : gv) b->h_items.push_back(g.it);
+    std::vector<BatchItem> strips;
+    size_t bytes = 0;
     for (int i = 0; i < b->capacity; i++) {
         if (b->state[i] != THY_SLOT_RUNNING) continue;
         const WorkLists &w = b->ctx[i]->batched;
-        if (w.n_deep > 0)
-            while (b->h_items.size() % 8) b->h_items.push_back(BatchItem{-1, 0, make_int2(0, 0)});
         for (int p = 0; p < w.n_deep; p += SW_WAVES)
-            b->h_items.push_back(BatchItem{i, (p == 0 && w.tile_h.empty()) ? 1 : 0, make_int2(p, 0)});
+            strips.push_back(BatchItem{i, (p == 0 && w.tile_h.empty()) ? 1 : 0, make_int2(p, 0)});
+        while (strips.size() % 8) strips.push_back(BatchItem{-1, 0, make_int2(0, 0)});
+        bytes += b->ctx[i]->state_bytes;
     }
+    auto fill = [&](std::vector<BatchItem> &out, const bool back) {
+        const int last = (int)strips.size() / 8 - 1;
+        out.clear();
+        spread_items(gv.size(), strips.size(), 2.0, [&](const bool tile, const int i) {
+            if (i < 0) out.push_back(BatchItem{-1, 0, make_int2(0, 0)});
+            else out.push_back(tile ? gv[i].it : strips[back ? (last - i / 8) * 8 + i % 8 : i]);
+        });
+    };
+    fill(b->h_items, false);
+    fill(b->h_back, bytes > kCacheBytes);
     const int cap = list_cap(b->h_items.size());
     if (cap != b->item_cap) {
         // the captured launches hold the old list and grid size
@@ -1838,14 +1856,17 @@ int batch_items(thy_batch *b) {
         dev_free(b->d_items);
         b->d_items = nullptr;
         b->item_cap = 0;
-        BHIPCHK(dev_alloc(&b->d_items, (size_t)cap * sizeof(BatchItem)));
+        BHIPCHK(dev_alloc(&b->d_items, 2 * (size_t)cap * sizeof(BatchItem)));
         b->item_cap = cap;
     }
     b->h_count = (int)b->h_items.size();
     // ordered before the next launch on the batch stream; the host list lives in b
-    if (!b->h_items.empty())
+    if (!b->h_items.empty()) {
         BHIPCHK(hipMemcpyAsync(b->d_items, b->h_items.data(), b->h_items.size() * sizeof(BatchItem), hipMemcpyHostToDevice,
                                b->stream));
+        BHIPCHK(hipMemcpyAsync(b->d_items + b->item_cap, b->h_back.data(), b->h_back.size() * sizeof(BatchItem),
+                               hipMemcpyHostToDevice, b->stream));
+    }
     BHIPCHK(hipMemcpyAsync(b->d_count, &b->h_count, sizeof(int), hipMemcpyHostToDevice, b->stream));
     BHIPCHK(hipStreamSynchronize(b->stream));
     b->dirty = false;
@@ -1857,12 +1878,13 @@ int batch_graph(thy_batch *b) {
     if (b->gexec) return THY_OK;
     BatchArgs q;
     q.args = b->d_args;
-    q.items = b->d_items;
     q.n_items = b->d_count;
     hipGraph_t g;
     BHIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < b->K; k++)
+    for (int k = 0; k < b->K; k++) {
+        q.items = b->d_items + (k % 2) * b->item_cap;
         hipLaunchKernelGGL(k_batch, dim3(b->item_cap), dim3(64 * SW_WAVES), 0, b->stream, q, k % 3);
+    }
     BHIPCHK(hipStreamEndCapture(b->stream, &g));
     BHIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
     (void)hipGraphDestroy(g);

@@ -1034,10 +1034,10 @@ __global__ void __launch_bounds__(64 * SW_WAVES, sizeof(T) == 4 ? 5 : 2) k_sweep
 // ---------------------------------------------------------------------------
 // Many grids per launch.  Each scenario keeps its own state, control block and dt slots; a
 // step of the batch advances every running scenario by one of its own steps in one launch:
-// the general tiles of all scenarios, costliest first, then their deep-water strips, four
-// of one scenario to a workgroup.  The item flagged as its scenario's writer publishes the
-// next control block.  Item counts are read on the device, so one captured launch sequence
-// serves a changing item list up to the captured grid size.
+// their deep-water strips, four of one scenario to a workgroup, and among them the general
+// tiles of all, costliest first.  The item flagged as its scenario's writer publishes the next
+// control block.  Item counts are read on the device, so one captured launch sequence serves a
+// changing item list up to the captured grid size.
 // ---------------------------------------------------------------------------
 struct BatchItem {
     int slot;    // scenario slot (-1: padding)
