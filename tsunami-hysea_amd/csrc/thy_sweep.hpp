@@ -33,8 +33,16 @@ __device__ __forceinline__ float dpp_left(float v) {
 __device__ __forceinline__ float dpp_right(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
 }
-__device__ __forceinline__ double dpp_left(double v) { return __shfl_up(v, 1, 64); }
-__device__ __forceinline__ double dpp_right(double v) { return __shfl_down(v, 1, 64); }
+__device__ __forceinline__ double dpp_left(double v) {
+    const int2 b = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, 0x138, 0xf, 0xf, true),
+                                                __builtin_amdgcn_update_dpp(0, b.y, 0x138, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ double dpp_right(double v) {
+    const int2 b = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, 0x130, 0xf, 0xf, true),
+                                                __builtin_amdgcn_update_dpp(0, b.y, 0x130, 0xf, 0xf, true)));
+}
 
 // read-only table entry at a wavefront-uniform address (scalar load)
 template <typename S> __device__ __forceinline__ S uniform_load(const S *p) {
