@@ -460,12 +460,13 @@ template <typename F> void spread_items(const size_t n_tiles, const size_t n_str
     }
 }
 
-// The items of a grid stepped alone.  Strips of up to 8 rows follow the tiles.  4000x3000 at
-// 32 rows: 160 us tiles first, 147 strips first, 135 lag 2; 2000x2000 at 16 rows: 60.1, 64.4,
-// 57.6 lag 1.5.
+// The items of a grid stepped alone.  Strips of up to 8 rows follow the tiles; the taller they
+// are, the earlier the last of them has to start.  4000x3000, us a step at lag 1.5 / 2 / 3 / 5:
+// 121.5 / 122.1 / 122.9 / 125.6 with strips of 16 rows, 126.4 / 122.3 / 118.7 / 127.5 with 32,
+// 134.3 / 133.7 / 127.8 / 117.8 with 48; tiles first 139 to 154, spread evenly 128 to 145.
 std::vector<int2> interleave(const std::vector<int2> &tiles, const int n_deep, const int strip_rows) {
     std::vector<int2> out;
-    const double lag = strip_rows <= 8 ? 0.0 : (strip_rows <= 16 ? 1.5 : 2.0);
+    const double lag = strip_rows <= 8 ? 0.0 : 0.11 * strip_rows;
     spread_items(tiles.size(), n_deep, lag, [&](const bool tile, const int i) {
         if (i >= 0) out.push_back(tile ? tiles[i] : make_int2(i * SW_WAVES, 0));
     });
