@@ -22,6 +22,9 @@ template <> struct Num<float> {
     static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
     static __device__ __forceinline__ float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
     static __device__ __forceinline__ float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
+    static __device__ __forceinline__ float plain_rcp(float x) { return rcp(x); }
+    static __device__ __forceinline__ float plain_div(float a, float b) { return div(a, b); }
+    static __device__ __forceinline__ float plain_sqrt(float x) { return sqrt(x); }
     // a * b + c rounded once (v_fma_f32).  The library is compiled without automatic
     // contraction, so every fused product is written out here, at the same place in each
     // copy of a formula, and all kernels round it the same way.
@@ -49,10 +52,43 @@ template <> struct Num<double> {
     static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
     static __device__ __forceinline__ double div(double a, double b) { return a / b; }
     static __device__ __forceinline__ double sqrt(double x) { return ::sqrt(x); }
+    // The same for a divisor and a radicand that are positive (a divisor may be negative) and
+    // between 1e-100 and 1e100, as all are in deep water: Newton's iteration from the hardware
+    // estimate, the quotient corrected by its residual (Markstein), and the square root with its
+    // half reciprocal (Goldschmidt), corrected twice.  As accurate as the general forms, without
+    // their scaling and special cases (8 instructions instead of 11, 11 instead of 20).
+    static __device__ __forceinline__ double newton_rcp(double b) {
+        double r = __builtin_amdgcn_rcp(b);
+        r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+        return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    }
+    static __device__ __forceinline__ double plain_rcp(double b) {
+        const double r = newton_rcp(b);
+        return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    }
+    // a / b with r = newton_rcp(b), for several quotients by one divisor
+    static __device__ __forceinline__ double plain_div(double a, double b, double r) {
+        const double q = a * r;
+        return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+    }
+    static __device__ __forceinline__ double plain_div(double a, double b) { return plain_div(a, b, newton_rcp(b)); }
+    static __device__ __forceinline__ double plain_sqrt(double x) {
+        const double y = __builtin_amdgcn_rsq(x);
+        double g = x * y, h = 0.5 * y;
+        const double d = __builtin_fma(-h, g, 0.5);
+        h = __builtin_fma(h, d, h);
+        g = __builtin_fma(g, d, g);
+        g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+        return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    }
     // FP64 keeps the product and the sum rounded separately, as the oracle rounds them
     static __device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
     static __device__ __forceinline__ double div_sqrt(double a, double x) { return a / ::sqrt(x); }
-    static __device__ __forceinline__ double min(double a, double b) { return a < b ? a : b; }
+    static __device__ __forceinline__ double min(double a, double b) {
+        double m;
+        asm("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+        return m;
+    }
     static __device__ __forceinline__ double exp(double x) { return ::exp(x); }
     static __device__ __forceinline__ double pow43(double x) { return ::pow(x, 4.0 / 3.0); }
 };

@@ -95,8 +95,8 @@ template <typename T>
 __device__ __forceinline__ MF<T> fast_mom_x(const DC<T> &a, const DC<T> &b, T deta, T il, T kd, T dt) {
     MF<T> o;
     const T hij = T(0.5) * (a.h + b.h);
-    const T uij = Num<T>::div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
-    const T lmax = habs(uij) + Num<T>::sqrt(hij);
+    const T uij = Num<T>::plain_div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
+    const T lmax = habs(uij) + Num<T>::plain_sqrt(hij);
     const bool up = uij < T(0);
     const T uu = up ? b.un : a.un;
     const T qnn = up ? b.qn : a.qn;
@@ -118,8 +118,8 @@ __device__ __forceinline__ MF<T> fast_mom_y(const DC<T> &a, const DC<T> &b, T de
     MF<T> o;
     const T g0 = f.cos0, g1 = f.cos1, ic0 = f.ic0, ic1 = f.ic1, len = f.len;
     const T hij = T(0.5) * (a.h + b.h);
-    const T uij = Num<T>::div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
-    const T lmax = habs(uij) + Num<T>::sqrt(hij);
+    const T uij = Num<T>::plain_div(Num<T>::mad(a.s, a.un, b.s * b.un), a.s + b.s + Num<T>::eps);
+    const T lmax = habs(uij) + Num<T>::plain_sqrt(hij);
     deta = Num<T>::mad(-(uij * uij), f.gd, f.gh * deta);
     const bool up = uij < T(0);
     const T uu = up ? b.un : a.un;
@@ -652,7 +652,7 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
             }
             // e*, D, sqrt(h*), qy/h*, qx, qy of row g-1 for the y faces
             T s2 = re[0], D2 = rD[0], qx2 = rqx[0], qy2 = rqy[0];
-            T sq2 = Num<T>::sqrt(s2 + D2), v2 = qy2 * Num<T>::rcp(s2 + D2);
+            T sq2 = Num<T>::plain_sqrt(s2 + D2), v2 = qy2 * Num<T>::plain_rcp(s2 + D2);
             T X2 = T(0), Y2 = T(0), W2 = T(0);  // accumulators of row g-1
 #pragma unroll
             for (int t = 0; t <= KR; t++) {
@@ -661,7 +661,7 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
                 const int g = y0 + f;
                 const T s1 = re[t + 1], D1 = rD[t + 1], qx1 = rqx[t + 1], qy1 = rqy[t + 1];
                 const T h1 = s1 + D1;
-                const T sq1 = Num<T>::sqrt(h1), ih = Num<T>::rcp(h1);
+                const T sq1 = Num<T>::plain_sqrt(h1), ih = Num<T>::plain_rcp(h1);
                 const T u1 = qx1 * ih, v1 = qy1 * ih;
                 // x faces of row g and the y face between rows g-1 and g
                 const bool xs = f < fb;
@@ -871,8 +871,8 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
             s1 = Num<T>::mad(dt * g.p.invA, m1, i1.e);
             smin = Num<T>::min(smin, s1);
             hs1 = s1 + i1.D;
-            sq1 = Num<T>::sqrt(hs1);
-            const T ih = Num<T>::rcp(hs1);
+            sq1 = Num<T>::plain_sqrt(hs1);
+            const T ih = Num<T>::plain_rcp(hs1);
             u1 = i1.qx * ih;
             v1 = i1.qy * ih;
         }
@@ -908,7 +908,7 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
             const bool arr_on = on && track && !Arrival<T>::arrived(carr) && habs(eo - carr) > dif_at;
             buf_store<T>(eo, rs, (max_on ? vout : kDropOffset) + o.emax, so);
             buf_store<T>(tnow, rs, (arr_on ? vout : kDropOffset) + o.arr, so);
-            const T dtc = W2 < Num<T>::eps ? Num<T>::big : Num<T>::div(cfl2 * g.q.A, W2);
+            const T dtc = W2 < Num<T>::eps ? Num<T>::big : Num<T>::plain_div(cfl2 * g.q.A, W2);
             if (on) dtmin = Num<float>::min(dtmin, (float)dtc);  // halo lanes: dropped below
             const T val = dt * g.q.invA;
             const T qx = Num<T>::mad(val, X2, i2.qx), qy = Num<T>::mad(val, Y2, i2.qy);
