@@ -71,6 +71,7 @@ struct thy_ctx {
     int ng = 0, gcap = 0;
     double *okada_def = nullptr;
     OkadaRow *okada_row = nullptr;     // per row of the grid
+    OkadaPlane *okada_plane = nullptr; // of the fault in hand
     double *mass_partial = nullptr;
     float *outbuf = nullptr;
     hipStream_t stream = nullptr;
@@ -764,27 +765,21 @@ int apply_okada_t(thy_ctx *ctx, const thy_fault *f, int crop_flag, double crop_v
     OkadaFault of;
     of.lon_c = f->lon_c; of.lat_c = f->lat_c; of.depth = f->depth_c; of.L = f->length; of.W = f->width;
     of.H = ctx->prm.H;
-    const double rad = 3.14159265358979323846 / 180.0;
-    of.ss = sin(rad * f->strike); of.cs = cos(rad * f->strike);
-    of.sd = sin(f->dip * (6.283185307179586 / 360.0)); of.cd = cos(f->dip * (6.283185307179586 / 360.0));
-    if (std::fabs(of.cd) < 1e-6) {
-        of.cd = 0.0;
-        if (of.sd > 0.0) of.sd = 1.0;
-        if (of.sd < 0.0) of.sd = -1.0;
-    }
-    of.d1 = f->slip * cos(rad * f->rake); of.d2 = f->slip * sin(rad * f->rake);
+    of.strike = f->strike; of.dip = f->dip; of.rake = f->rake; of.slip = f->slip;
     of.lon0 = ctx->lon[0];
     of.dlon = (ctx->lon[ctx->nx - 1] - ctx->lon[0]) / (ctx->nx - 1);
     T *const e = (T *)ctx->e[ctx->cur], *const D = (T *)ctx->D, *const arr = (T *)ctx->arr;
+    hipLaunchKernelGGL(k_okada_plane, dim3(1), dim3(64), 0, ctx->stream, of, ctx->okada_plane);
+    HIPCHK(hipGetLastError());
     if (!def_out && crop_flag != 1) {
-        hipLaunchKernelGGL((k_okada_add<T>), dim3(grid_1d(n)), dim3(256), 0, ctx->stream, of, ctx->okada_row, ctx->nx,
+        hipLaunchKernelGGL((k_okada_add<T>), dim3(grid_1d(n)), dim3(256), 0, ctx->stream, of, ctx->okada_plane, ctx->okada_row, ctx->nx,
                            ctx->ny, ctx->pitch, crop_flag == 2 ? crop_value : -1.0, e, D, arr);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         return THY_OK;
     }
     HIPCHK(hipMemsetAsync(&ctx->scratch_u[1], 0, sizeof(unsigned int), ctx->stream));
-    hipLaunchKernelGGL(k_okada, dim3(grid_1d(n)), dim3(256), 0, ctx->stream, of, ctx->okada_row, ctx->nx, ctx->ny,
+    hipLaunchKernelGGL(k_okada, dim3(grid_1d(n)), dim3(256), 0, ctx->stream, of, ctx->okada_plane, ctx->okada_row, ctx->nx, ctx->ny,
                        ctx->okada_def, &ctx->scratch_u[1]);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL((k_okada_apply<T>), dim3(grid_1d(n)), dim3(256), 0, ctx->stream, ctx->okada_def, ctx->nx,
@@ -1283,13 +1278,11 @@ int thy_create(const thy_grid *g, const thy_params *p, thy_ctx **out) {
     {
         // the latitudes Okada uses are uniform (src/GPU/ShallowWater.cu:215-218)
         const double lat0 = ctx->lat[0], dlat = (ctx->lat[ctx->ny - 1] - ctx->lat[0]) / (ctx->ny - 1);
-        std::vector<OkadaRow> r(ctx->ny);
-        for (int j = 0; j < ctx->ny; j++) {
-            const double lat = lat0 + j * dlat, rlat = lat * 0.017453292371619689, cl = cos(rlat);
-            r[j] = OkadaRow{lat, cl, sin(rlat) * cl, cos(rlat * 2.0)};
-        }
-        HIPCHK(dev_alloc((void **)&ctx->okada_row, r.size() * sizeof(OkadaRow)));
-        HIPCHK(ctx_copy(ctx, ctx->okada_row, r.data(), r.size() * sizeof(OkadaRow), hipMemcpyHostToDevice));
+        HIPCHK(dev_alloc((void **)&ctx->okada_row, ctx->ny * sizeof(OkadaRow)));
+        HIPCHK(dev_alloc((void **)&ctx->okada_plane, sizeof(OkadaPlane)));
+        hipLaunchKernelGGL(k_okada_rows, dim3((ctx->ny + 255) / 256), dim3(256), 0, ctx->stream, lat0, dlat, ctx->ny,
+                           ctx->okada_row);
+        HIPCHK(hipGetLastError());
     }
     if ((r = ctx->prec ? upload_geometry<double>(ctx) : upload_geometry<float>(ctx)) != THY_OK) return r;
     // zero state so that padding columns hold finite values
@@ -1314,7 +1307,7 @@ void thy_destroy(thy_ctx *ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     drop_graphs(ctx);
     void *ptrs[] = {ctx->state, ctx->row, ctx->fy, ctx->deep_row, ctx->area_d, ctx->ctrl, ctx->dtmin, ctx->scratch_u,
-                    ctx->ftime, ctx->gpos, ctx->gbuf, ctx->gtime, ctx->okada_def, ctx->okada_row, ctx->mass_partial, ctx->outbuf,
+                    ctx->ftime, ctx->gpos, ctx->gbuf, ctx->gtime, ctx->okada_def, ctx->okada_row, ctx->okada_plane, ctx->mass_partial, ctx->outbuf,
                     ctx->steplog, ctx->alone.deep, ctx->alone.items, ctx->batched.deep, ctx->batched.items, ctx->health};
     for (void *q : ptrs)
         dev_free(q);

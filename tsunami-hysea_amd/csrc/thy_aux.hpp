@@ -81,172 +81,167 @@ __global__ void __launch_bounds__(256) k_initial_dt(const StepArgs<T> a, int cur
 // Corner guards, singular cases and log branches follow DC3D (:661-714, :72-157).
 // Projection: Gauss-Krueger about the fault centroid (src/GPU/prtoxy.cu:33-54).
 // ---------------------------------------------------------------------------
-// What bounds it is FP64 arithmetic (one thread evaluates some ten square roots, inverse
-// tangents and logarithms for 8 bytes written), so the work is to call fewer of them:
-//   * the sums over the four corners are taken inside the functions: the logarithms of a
-//     sum over corners become one logarithm of a quotient of products (8 -> 2, none
-//     without strike slip), and two inverse tangents become one of a complex product,
-//     atan(a1/b1) - atan(a2/b2) = arg((b1 + i a1)(b2 - i a2)) for b1, b2 > 0, exact since
-//     the difference lies within (-pi, pi) (8 -> 4, and their 8 quotients go with them);
-//   * square roots and quotients shared between corners are taken once;
-//   * sines and cosines of the fault's angles come with it, those of a row's latitude from
-//     a table of the grid.
-// Either form of a sum rounds to a few units of the largest term.
-// Per fault on 2000x2000 cells: 882 us before, 204 now (181 registers, 2 wavefronts a SIMD, before; 118 and 4 now).
+// What bounds it is FP64 arithmetic: some eight inverse tangents, eight logarithms, thirty
+// quotients and ten square roots a cell for 8 bytes written.  Sums over the corners inside the
+// logarithms and tangents need fewer (204 us a fault), but round otherwise, and a cell whose
+// rise comes close to the arrival threshold then arrives a step earlier or later.  So every
+// sum keeps its terms and its order, and what is saved leaves each value as it is:
+//   * quotients and square roots without scaling and special cases, one reciprocal for all
+//     quotients by the same divisor;
+//   * the functions of the fault's angles and of a row's latitude come from tables;
+//   * logarithms only with strike slip, tangents only with dip slip;
+//   * a loop over the corners holds the registers of one.
+// Per fault on 2000x2000 cells: 882 us before, 330 now (181 registers and 2 wavefronts a SIMD
+// before, 114 and 4 now).
 // ---------------------------------------------------------------------------
 struct OkadaFault {
-    double lon_c, lat_c, depth, L, W, H;
-    double ss, cs;          // sine and cosine of the strike
-    double sd, cd;          // of the dip (cd 0 and sd +-1 within 1e-6 of vertical)
-    double d1, d2;          // slip components
+    double lon_c, lat_c, depth, L, W, H, strike, dip, rake, slip;
     double lon0, dlon;
+};
+
+// functions of a fault's angles
+struct OkadaPlane {
+    double ss, cs;                   // sine and cosine of the strike
+    double sd, cd, sdcd, cdcd;       // of the dip (cd 0 and sd +-1 within 1e-6 of vertical)
+    double kcd, rcd, rH;             // 1 / cdcd, newton_rcp of cdcd and of H
+    double d1, d2, c1, c2;           // slip components, and over 2 pi
 };
 
 // functions of a grid row's latitude that the projection uses
 struct OkadaRow {
-    double lat, cl, slcl, c2;  // latitude (degrees), cos, sin * cos, cos of the double angle
+    double lat, sl, cl, hv2, c2;  // latitude (degrees), sin, cos, half of v2, cos of the double angle
 };
 
-// a / b for b in the normal range, its reciprocal by Newton's iteration from the hardware
-// estimate and the quotient corrected by its residual
-__device__ __forceinline__ double okada_div(const double a, const double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-    const double q = a * r;
-    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+__global__ void k_okada_rows(const double lat0, const double dlat, const int ny, OkadaRow *rows) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= ny) return;
+    OkadaRow r;
+    r.lat = lat0 + j * dlat;
+    const double rlat = r.lat * 0.017453292371619689;
+    r.sl = sin(rlat);
+    r.cl = cos(rlat);
+    r.hv2 = (r.cl * 0.0067397251 * r.cl + 1.0) * 0.5;
+    r.c2 = cos(rlat * 2.0);
+    rows[j] = r;
 }
 
-// atan(a1 / b1) - atan(a2 / b2)
-__device__ __forceinline__ double okada_datan(double a1, double b1, double a2, double b2) {
-    if (b1 < 0.0) { a1 = -a1; b1 = -b1; }
-    if (b2 < 0.0) { a2 = -a2; b2 = -b2; }
-    return atan2(__builtin_fma(a1, b2, -(a2 * b1)), __builtin_fma(b1, b2, a1 * a2));
+__global__ void k_okada_plane(const OkadaFault f, OkadaPlane *out) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    const double RAD = 3.14159265358979323846 / 180.0, pi2 = 6.283185307179586;
+    OkadaPlane o;
+    o.ss = sin(RAD * f.strike);
+    o.cs = cos(RAD * f.strike);
+    o.sd = sin(f.dip * (pi2 / 360.0));
+    o.cd = cos(f.dip * (pi2 / 360.0));
+    if (fabs(o.cd) < 1e-6) {
+        o.cd = 0.0;
+        if (o.sd > 0.0) o.sd = 1.0;
+        if (o.sd < 0.0) o.sd = -1.0;
+    }
+    o.sdcd = o.sd * o.cd;
+    o.cdcd = o.cd * o.cd;
+    o.kcd = 1.0 / o.cdcd;
+    o.rcd = Num<double>::newton_rcp(o.cdcd);
+    o.rH = Num<double>::newton_rcp(f.H);
+    o.d1 = f.slip * cos(RAD * f.rake);
+    o.d2 = f.slip * sin(RAD * f.rake);
+    o.c1 = o.d1 / pi2;
+    o.c2 = o.d2 / pi2;
+    *out = o;
 }
 
 // x, y: position along and across the strike
-__device__ __forceinline__ double okada_uz(const OkadaFault &f, const double x, const double y) {
-    constexpr double alp3 = 0.5;  // (1 - alpha) / alpha with alpha = 2/3
-    constexpr double pi2 = 6.283185307179586;
-    const double sd = f.sd, cd = f.cd;
-    const double sdcd = sd * cd, cdcd = cd * cd;
-    double xi[2] = {x + 0.5 * f.L, x - 0.5 * f.L};
+__device__ __forceinline__ double okada_uz(const OkadaFault &f, const OkadaPlane &o, const double x, const double y) {
+    using N = Num<double>;
+    const double alpha = 2.0 / 3.0;
+    const double alp3 = (1.0 - alpha) / alpha;
+    const double sd = o.sd, cd = o.cd, sdcd = o.sdcd, cdcd = o.cdcd;
+    double xi0 = x - -0.5 * f.L, xi1 = x - 0.5 * f.L;
+    if (fabs(xi0) < 1e-6) xi0 = 0.0;
+    if (fabs(xi1) < 1e-6) xi1 = 0.0;
     const double p = y * cd + f.depth * sd;
     double q = y * sd - f.depth * cd;
-    double et[2] = {p + 0.5 * f.W, p - 0.5 * f.W};
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        if (fabs(xi[k]) < 1e-6) xi[k] = 0.0;
-        if (fabs(et[k]) < 1e-6) et[k] = 0.0;
-    }
+    double et0 = p - -0.5 * f.W, et1 = p - 0.5 * f.W;
     if (fabs(q) < 1e-6) q = 0.0;
-    if (q == 0.0 && ((xi[0] * xi[1] <= 0.0 && et[0] * et[1] == 0.0) || (et[0] * et[1] <= 0.0 && xi[0] * xi[1] == 0.0)))
+    if (fabs(et0) < 1e-6) et0 = 0.0;
+    if (fabs(et1) < 1e-6) et1 = 0.0;
+    if (q == 0.0 && ((xi0 * xi1 <= 0.0 && et0 * et1 == 0.0) || (et0 * et1 <= 0.0 && xi0 * xi1 == 0.0)))
         return 0.0;  // on a fault edge
     const double q2 = q * q;
-    double r[2][2], xx[2];  // [j][k]: corner (xi[j], et[k])
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        xx[j] = sqrt(xi[j] * xi[j] + q2);
-#pragma unroll
-        for (int k = 0; k < 2; k++) r[j][k] = sqrt(xi[j] * xi[j] + et[k] * et[k] + q2);
-    }
+    // (x is 0 or at least 1e-12)
+    auto root = [](const double x) { return x == 0.0 ? 0.0 : N::plain_sqrt(x); };
+    const double r12 = root(xi0 * xi0 + et1 * et1 + q2);
+    const double r21 = root(xi1 * xi1 + et0 * et0 + q2);
+    const double r22 = root(xi1 * xi1 + et1 * et1 + q2);
     // corners beyond the end of the fault's edge lines, where r + xi or r + et cancels
-    bool kxi[2], ket[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        kxi[k] = xi[0] < 0.0 && r[1][k] + xi[1] < 1e-6;
-        ket[k] = et[0] < 0.0 && r[k][1] + et[1] < 1e-6;
-    }
-    // sums over the corners with the sign of each: `s` of the rational terms, the numerator
-    // and denominator of the logarithms' quotients, and the four tangents
-    double s1 = 0.0, s2 = 0.0;
-    double ln[2] = {1.0, 1.0}, le[2] = {1.0, 1.0};  // prod (r + d), prod (r + et): [0] corners with +, [1] with -
-    double ta[2][2], tb[2][2], wa[2][2], wb[2][2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const double X = xi[j], E = et[k], R = r[j][k];
-            const double sg = (j + k != 1) ? 1.0 : -1.0;
-            const int m = j + k != 1 ? 0 : 1;
-            ta[j][k] = 0.0; tb[j][k] = 1.0;
-            wa[j][k] = 0.0; wb[j][k] = 1.0;
-            if (R == 0.0) continue;
-            const double yy = E * cd + q * sd;
-            const double rd = R + (E * sd - q * cd);
-            const double x11 = kxi[k] ? 0.0 : okada_div(1.0, R * (R + X));
-            const double y11 = ket[j] ? 0.0 : okada_div(1.0, R * (R + E));
-            const double ird = okada_div(1.0, rd);
-            if (q != 0.0) { ta[j][k] = X * E; tb[j][k] = q * R; }
-            double i3 = 0.0, i4 = 0.0;  // the parts of I3 sd and I4 sdcd outside logarithms and tangents
+    const bool kxi0 = xi0 < 0.0 && r21 + xi1 < 1e-6, kxi1 = xi0 < 0.0 && r22 + xi1 < 1e-6;
+    const bool ket0 = et0 < 0.0 && r12 + et1 < 1e-6, ket1 = et0 < 0.0 && r22 + et1 < 1e-6;
+    double uz = 0.0;
+#pragma unroll 1
+    for (int c = 0; c < 4; c++) {
+        const bool j = (c & 1) != 0, k = (c & 2) != 0;
+        const double X = j ? xi1 : xi0, E = k ? et1 : et0;
+        const bool kxi = k ? kxi1 : kxi0, ket = j ? ket1 : ket0;
+        const double xi2 = X * X;
+        const double r = root(xi2 + E * E + q2);
+        if (r == 0.0) continue;
+        const double yy = E * cd + q * sd;
+        const double dd = E * sd - q * cd;
+        const double rd = r + dd, ird = N::newton_rcp(rd);
+        double b1 = 0.0, b2 = 0.0;
+        if (o.d1 != 0.0) {
+            const double l = log(ket ? r - E : r + E), ale = ket ? -l : l, lrd = log(rd);
+            const double y11 = ket ? 0.0 : N::plain_rcp(r * (r + E));
+            double ai3;
+            if (cd != 0.0) ai3 = N::plain_div(N::plain_div(yy * cd, rd, ird) - ale + sd * lrd, cdcd, o.rcd);
+            else ai3 = (N::plain_div(E, rd, ird) + N::plain_div(yy * q, rd * rd) - ale) / 2.0;
+            const double ai2 = lrd + ai3 * sd;
+            b1 += o.c1 * (N::plain_div(-q, r) + N::plain_div(alp3 * yy, rd, ird) * sd);
+            b2 += o.c1 * (q * (q * y11) - alp3 * ai2 * sd);
+        }
+        if (o.d2 != 0.0) {
+            const double tt = (q == 0.0) ? 0.0 : atan(N::plain_div(X * E, q * r));
+            const double qx = q * (kxi ? 0.0 : N::plain_rcp(r * (r + X)));
+            double ai4 = 0.0;
             if (cd != 0.0) {
                 if (X != 0.0) {
-                    i4 = X * ird * sdcd;
-                    wa[j][k] = E * (xx[j] + q * cd) + xx[j] * (R + xx[j]) * sd;
-                    wb[j][k] = X * (R + xx[j]) * cd;
+                    const double xx = root(xi2 + q2);
+                    ai4 = o.kcd * (N::plain_div(X, rd, ird) * sdcd +
+                                   2.0 * atan(N::plain_div(E * (xx + q * cd) + xx * (r + xx) * sd, X * (r + xx) * cd)));
                 }
-                i3 = yy * cd * ird;
             } else {
-                i3 = (E + yy * q * ird) * ird;
-                i4 = 0.5 * X * yy * ird * ird;
+                ai4 = N::plain_div(X * yy, rd * rd) / 2.0;
             }
-            if (f.d1 != 0.0) {
-                const double b1 = alp3 * yy * ird * sd - okada_div(q, R);
-                // ai2 = log(rd) + ai3 sd: its rational part here, its logarithms below
-                const double a2 = cd != 0.0 ? okada_div(i3, cdcd) * sd : 0.5 * i3 * sd;
-                s1 += sg * (b1 * sd + (q * q * y11 - alp3 * a2 * sd) * cd);
-                ln[m] *= rd;
-                le[m] *= ket[j] ? okada_div(1.0, R - E) : R + E;
-            }
-            if (f.d2 != 0.0) {
-                const double b1 = -E * q * x11 - alp3 * X * ird * sdcd;
-                const double a4 = cd != 0.0 ? okada_div(i4, cdcd) : i4;
-                s2 += sg * (b1 * sd + (q2 * x11 + alp3 * a4 * sdcd) * cd);
-            }
+            b1 += o.c2 * (-E * qx - tt - N::plain_div(alp3 * X, rd, ird) * sdcd);
+            b2 += o.c2 * (q * qx + alp3 * ai4 * sdcd);
         }
-    }
-    double uz = 0.0;
-    if (f.d1 != 0.0) {
-        // sum of ai2's logarithms: log(rd) + sd (sd log(rd) - ale) / cd^2, = log(rd) - sd ale / 2
-        // for a vertical fault
-        const double lr = log(okada_div(ln[0], ln[1])), la = log(okada_div(le[0], le[1]));
-        const double a2 = cd != 0.0 ? lr + okada_div(sd * lr - la, cdcd) * sd : lr - 0.5 * la * sd;
-        uz += f.d1 * okada_div(s1 - alp3 * a2 * sd * cd, pi2);
-    }
-    if (f.d2 != 0.0) {
-        // sum of -atan(X E / (q R)) sd
-        const double tt = okada_datan(ta[0][0], tb[0][0], ta[0][1], tb[0][1]) -
-                          okada_datan(ta[1][0], tb[1][0], ta[1][1], tb[1][1]);
-        s2 -= tt * sd;
-        if (cd != 0.0) {
-            const double w = okada_datan(wa[0][0], wb[0][0], wa[0][1], wb[0][1]) -
-                             okada_datan(wa[1][0], wb[1][0], wa[1][1], wb[1][1]);
-            s2 += alp3 * okada_div(2.0 * w, cdcd) * sdcd * cd;
-        }
-        uz += f.d2 * okada_div(s2, pi2);
+        const double v = b1 * sd + b2 * cd;
+        uz += j == k ? v : -v;
     }
     return uz;
 }
 
 __device__ __forceinline__ void gauss_krueger(const OkadaRow &g, const double lon, const double lat0, const double lon0,
                                               double &x, double &y) {
+    using N = Num<double>;
     const double D2R = 0.017453292371619689;
-    const double v2 = g.cl * 0.0067397251 * g.cl + 1.0;
     const double al = lon - lon0;
-    const double ph1 = g.lat + v2 * 0.5 * al * al * g.slcl * D2R;
-    const double s1 = sin(ph1 * D2R), s2 = sin((ph1 + lat0) * 0.5 * D2R);
-    const double u = 1.0 - s2 * 0.0066946053 * s2, dd = sqrt(u);
-    const double r = okada_div(6335.4607362597517, u * dd);
-    const double an = okada_div(6378.16, sqrt(1.0 - s1 * 0.0066946053 * s1));
-    y = okada_div((ph1 - lat0) * r, 57.29578);
-    x = okada_div(al * g.cl * an, 57.29578) * (okada_div(al * al * g.c2, 19696.838434850401) + 1.0);
+    const double ph1 = g.lat + g.hv2 * al * al * g.sl * g.cl * D2R;
+    const double rph1 = ph1 * D2R;
+    const double rph2 = (ph1 + lat0) * 0.5 * D2R;
+    const double s1 = sin(rph1), s2 = sin(rph2);
+    const double dd = N::plain_sqrt(1.0 - s2 * 0.0066946053 * s2);
+    const double r = N::plain_div(6335.4607362597517, dd * (dd * dd));
+    const double an = N::plain_div(6378.16, N::plain_sqrt(1.0 - s1 * 0.0066946053 * s1));
+    y = N::plain_div(ph1 - lat0, N::plain_div(57.29578, r));
+    x = N::plain_div(al * g.cl, N::plain_div(57.29578, an)) * (N::plain_div(al * al * g.c2, 19696.838434850401) + 1.0);
 }
 
 // U_Z / H of the cell (i, row)
-__device__ __forceinline__ double okada_cell(const OkadaFault &f, const OkadaRow &g, const int i) {
+__device__ __forceinline__ double okada_cell(const OkadaFault &f, const OkadaPlane &o, const OkadaRow &g, const int i) {
     double xp, yp;
     gauss_krueger(g, f.lon0 + i * f.dlon, f.lat_c, f.lon_c, xp, yp);
-    return okada_uz(f, xp * f.ss + yp * f.cs, -xp * f.cs + yp * f.ss) / f.H;
+    return Num<double>::plain_div(okada_uz(f, o, xp * o.ss + yp * o.cs, -xp * o.cs + yp * o.ss), f.H, o.rH);
 }
 
 // add a cell's displacement (src/GPU/Deformacion.cu:22-53); eta_ini += U_Z, but a cell
@@ -260,13 +255,14 @@ __device__ __forceinline__ void okada_add(const double u, const int64_t o, T *e,
 
 // U_Z of every cell into `def` and its largest magnitude (for the relative crop), as a
 // float (src/GPU/Deformacion.cu:13-20,132-136)
-__global__ void __launch_bounds__(256) k_okada(const OkadaFault f, const OkadaRow *rows, int nx, int ny, double *def,
+__global__ void __launch_bounds__(256) k_okada(const OkadaFault f, const OkadaPlane *plane, const OkadaRow *rows, int nx, int ny, double *def,
                                                unsigned int *absmax) {
+    const OkadaPlane o = *plane;
     float m = 0.f;
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < (int64_t)nx * ny;
          c += (int64_t)gridDim.x * blockDim.x) {
         const int j = (int)(c / nx), i = (int)(c - (int64_t)j * nx);
-        const double uz = okada_cell(f, rows[j], i);
+        const double uz = okada_cell(f, o, rows[j], i);
         def[c] = uz;
         m = fmaxf(m, (float)fabs(uz));
     }
@@ -278,12 +274,13 @@ __global__ void __launch_bounds__(256) k_okada(const OkadaFault f, const OkadaRo
 // U_Z of every cell, cropped at an absolute height (thr <= 0: not cropped) and added at
 // once: where the crop does not depend on the largest U_Z, the field needs no second pass
 template <typename T>
-__global__ void __launch_bounds__(256) k_okada_add(const OkadaFault f, const OkadaRow *rows, int nx, int ny, int P,
+__global__ void __launch_bounds__(256) k_okada_add(const OkadaFault f, const OkadaPlane *plane, const OkadaRow *rows, int nx, int ny, int P,
                                                    const double thr, T *e, T *D, T *arr) {
+    const OkadaPlane o = *plane;
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < (int64_t)nx * ny;
          c += (int64_t)gridDim.x * blockDim.x) {
         const int j = (int)(c / nx), i = (int)(c - (int64_t)j * nx);
-        double u = okada_cell(f, rows[j], i);
+        double u = okada_cell(f, o, rows[j], i);
         if (fabs(u) < thr) u = 0.0;
         okada_add(u, (int64_t)j * P + i, e, D, arr);
     }
