@@ -1,6 +1,5 @@
 """Fields large enough to be read in chunks by several threads: every cell arrives in its
-place, with a staging block as large as the field, with a small one, and read from two
-threads at once.
+place, with the library's caches filled and emptied, and read from two threads at once.
 
 Tolerance: a field is one FP32 rounding (6e-8) away from a depth times the problem's scale,
 which the state gives in FP64; 1e-6 of the peak."""

@@ -823,9 +823,11 @@ int initial_dt_t(thy_ctx *ctx, double *dt) {
 // through one thread (or pins the caller's pages); here the data passes through pinned memory
 // in chunks, and several threads copy them on, so that the page faults of a new buffer are
 // taken side by side too.  The helper threads make no HIP calls and have ended on return.
-// Two fields of 4000x3000 into new arrays: 7.5 to 9.8 ms before, 3.3 now (29 GB/s); of
-// 2000x2000 1.95 and 1.25; 1500x1400 (8.4 MB) 1.05 and 0.85; of 1400x1200 (6.7 MB, below the
-// line) the runtime's copy takes 0.82.
+// The pinned block is one of its own, of 8 chunks: 16 are no faster, and with the block that
+// staged the upload, whose lines then lie in other cores' caches, the next upload took 31 ms
+// instead of 21 (2000x2000) and 90 instead of 61 (4000x3000).  Four fields of 4000x3000: 19.3
+// ms with the runtime's copy, 6.9 with this one; of 2000x2000 6.5 and 3.3, 1500x1450 (8.7 MB
+// each) 4.2 and 2.3; of 1400x1200 (6.7 MB, below the line) the runtime's is as fast.
 constexpr size_t kChunk = 2u << 20, kLargeCopy = 8u << 20;
 constexpr int kCopyThreads = 8;
 
@@ -852,13 +854,8 @@ int read_large(thy_ctx *ctx, char *out, const char *src, const size_t bytes) {
         }
     } run;
     run.q = ctx->stream;
-    // the block that staged the upload of the state, if it is there; else a smaller one
-    size_t room = 4 * (size_t)ctx->pitch * ctx->ny * ctx->esz;
-    run.pin = (char *)Pool::get().host_cached(room);
-    if (!run.pin) {
-        room = 8 * kChunk;
-        HIPCHK(Pool::get().host_alloc((void **)&run.pin, room));
-    }
+    const size_t room = 8 * kChunk;
+    HIPCHK(Pool::get().host_alloc((void **)&run.pin, room));
     const int slots = (int)std::min<size_t>({room / kChunk, (size_t)n, (size_t)64});
     run.done.reset(new std::atomic<bool>[n]);
     for (int i = 0; i < n; i++) run.done[i] = false;

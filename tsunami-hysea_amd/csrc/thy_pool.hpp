@@ -33,11 +33,6 @@ class Pool {
     hipError_t dev_alloc(void **p, size_t bytes) { return alloc(dev_, p, bytes); }
     void dev_free(void *p) { give_back(dev_, p); }
     hipError_t host_alloc(void **p, size_t bytes) { return alloc(host_, p, bytes); }
-    // a cached block of that size, or null: nothing is allocated
-    void *host_cached(size_t bytes) {
-        std::lock_guard<std::mutex> g(m_);
-        return take(host_, size_class(bytes));
-    }
     void host_free(void *p) { give_back(host_, p); }
 
     // a pair of streams (default priority), cached or new; non-blocking, so that work
@@ -150,7 +145,14 @@ class Pool {
         const size_t c = size_class(bytes);
         {
             std::lock_guard<std::mutex> g(m_);
-            if ((*p = take(h, c))) return hipSuccess;
+            auto it = h.free.find(c);
+            if (it != h.free.end() && !it->second.empty()) {
+                *p = it->second.back();
+                it->second.pop_back();
+                h.cached -= c;
+                h.live[*p] = c;
+                return hipSuccess;
+            }
         }
         hipError_t e = raw_alloc(h, p, c);
         if (e != hipSuccess) {
@@ -169,17 +171,6 @@ class Pool {
         std::lock_guard<std::mutex> g(m_);
         h.live[*p] = c;
         return hipSuccess;
-    }
-
-    // a cached block of size class c, or null (with m_ held)
-    static void *take(Heap &h, const size_t c) {
-        auto it = h.free.find(c);
-        if (it == h.free.end() || it->second.empty()) return nullptr;
-        void *p = it->second.back();
-        it->second.pop_back();
-        h.cached -= c;
-        h.live[p] = c;
-        return p;
     }
 
     void give_back(Heap &h, void *p) {
