@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(256) k_initial_dt(const StepArgs<T> a, int cur
 //   * the functions of the fault's angles and of a row's latitude come from tables;
 //   * logarithms only with strike slip, tangents only with dip slip;
 //   * a loop over the corners holds the registers of one.
-// Per fault on 2000x2000 cells: 882 us before, 330 now (181 registers and 2 wavefronts a SIMD
+// Per fault on 2000x2000 cells: 882 us before, 311 now (181 registers and 2 wavefronts a SIMD
 // before, 114 and 4 now).
 // ---------------------------------------------------------------------------
 struct OkadaFault {
