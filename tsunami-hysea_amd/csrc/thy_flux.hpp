@@ -25,6 +25,7 @@ template <> struct Num<float> {
     static __device__ __forceinline__ float plain_rcp(float x) { return rcp(x); }
     static __device__ __forceinline__ float plain_div(float a, float b) { return div(a, b); }
     static __device__ __forceinline__ float plain_sqrt(float x) { return sqrt(x); }
+    static __device__ __forceinline__ float depth_sqrt(float x) { return sqrt(x); }
     // a * b + c rounded once (v_fma_f32).  The library is compiled without automatic
     // contraction, so every fused product is written out here, at the same place in each
     // copy of a formula, and all kernels round it the same way.
@@ -52,11 +53,12 @@ template <> struct Num<double> {
     static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
     static __device__ __forceinline__ double div(double a, double b) { return a / b; }
     static __device__ __forceinline__ double sqrt(double x) { return ::sqrt(x); }
-    // The same for a divisor and a radicand that are positive (a divisor may be negative) and
-    // between 1e-100 and 1e100, as all are in deep water: Newton's iteration from the hardware
-    // estimate, the quotient corrected by its residual (Markstein), and the square root with its
-    // half reciprocal (Goldschmidt), corrected twice.  As accurate as the general forms, without
-    // their scaling and special cases (8 instructions instead of 11, 11 instead of 20).
+    // The same for a finite divisor (of either sign) and a positive radicand between 1e-100 and
+    // 1e100, as all are in deep water and those of the other faces that are no exponentials:
+    // Newton's iteration from the hardware estimate, the quotient corrected by its residual
+    // (Markstein), and the square root with its half reciprocal (Goldschmidt), corrected twice.
+    // As accurate as the general forms, without their scaling and special cases (8 instructions
+    // instead of 11, 11 instead of 20).
     static __device__ __forceinline__ double newton_rcp(double b) {
         double r = __builtin_amdgcn_rcp(b);
         r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
@@ -81,9 +83,11 @@ template <> struct Num<double> {
         g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
         return __builtin_fma(__builtin_fma(-g, g, x), h, g);
     }
+    // of a depth, which may be 0
+    static __device__ __forceinline__ double depth_sqrt(double x) { return x == 0.0 ? x : plain_sqrt(x); }
     // FP64 keeps the product and the sum rounded separately, as the oracle rounds them
     static __device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
-    static __device__ __forceinline__ double div_sqrt(double a, double x) { return a / ::sqrt(x); }
+    static __device__ __forceinline__ double div_sqrt(double a, double x) { return plain_div(a, plain_sqrt(x)); }
     static __device__ __forceinline__ double min(double a, double b) {
         double m;
         asm("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
@@ -131,13 +135,13 @@ template <typename T> __device__ __forceinline__ T limiter(T p0m, T p0, T p1, T 
     c0 = tabs(c0);
     c1 = tabs(c1);
     if (c0 < Num<T>::eps) return T(1);
-    T aux = tabs(Num<T>::div(c1 - c0, c1 + c0));
+    T aux = tabs(Num<T>::plain_div(c1 - c0, c1 + c0));
     c1 = T(0.5) * (c1 + c0) * Num<T>::mad(-(aux * aux), aux, T(1));
     // with r = p / q the smaller over the larger, sg r (1 + r) / (1 + r^2) =
     // sg p (q + p) / (q^2 + p^2): one division instead of two
     const bool big0 = c0 > c1;
     const T pn = big0 ? c1 : c0, qd = (big0 ? c0 : c1) + Num<T>::eps;
-    return Num<T>::div(sg * pn * (qd + pn), Num<T>::mad(qd, qd, pn * pn));
+    return Num<T>::plain_div(sg * pn * (qd + pn), Num<T>::mad(qd, qd, pn * pn));
 }
 
 // max(e1 + Dm, 0) - max(e0 + Dm, 0) with Dm = min(D0, D1)  (src/GPU/Arista_kernel.cu:201-202)
@@ -151,7 +155,7 @@ template <typename T> __device__ __forceinline__ T deta_of(T e0, T e1, T D0, T D
 template <typename T> __device__ __forceinline__ T blend(T hij, T hpos, bool alfa_cero) {
     if (alfa_cero) return T(0);
     if (hij < hpos)
-        return Num<T>::rcp(T(1) + Num<T>::exp(T(-15) * (T(1) - Num<T>::div(T(0.5) * hpos, hij + Num<T>::eps))));
+        return Num<T>::rcp(T(1) + Num<T>::exp(T(-15) * (T(1) - Num<T>::plain_div(T(0.5) * hpos, hij + Num<T>::eps))));
     return T(1);
 }
 
@@ -217,10 +221,10 @@ __device__ __forceinline__ T mass_waf(const bool yface, SC<T> m, SC<T> a, SC<T> 
     T u1 = b.f * q1;
     q0 = u0 * a.h;
     q1 = u1 * b.h;
-    T s0 = Num<T>::sqrt(a.h), s1 = Num<T>::sqrt(b.h);
-    T uij = Num<T>::div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
+    T s0 = Num<T>::depth_sqrt(a.h), s1 = Num<T>::depth_sqrt(b.h);
+    T uij = Num<T>::plain_div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
     T val = valf * dt;   // 2*len*dt/(A0+A1) with len/cos for x
-    T c0 = Num<T>::sqrt(hij);
+    T c0 = Num<T>::plain_sqrt(hij);
     T l1 = tmin(uij - c0, u0 - s0);
     T l2 = tmax(uij + c0, u1 + s1);
     T lmax = tmax(tabs(l2), tabs(l1));
@@ -233,7 +237,7 @@ __device__ __forceinline__ T mass_waf(const bool yface, SC<T> m, SC<T> a, SC<T> 
     if (tabs(l1 - l2) >= Num<T>::eps) {
         T alr = Num<T>::mad(val * l1, xiL, sgn(l1) * (T(1) - xiL));
         T blr = Num<T>::mad(val * l2, xiR, sgn(l2) * (T(1) - xiR));
-        a0 = Num<T>::div((alr - blr) * (l1 * l2), l2 - l1);
+        a0 = Num<T>::plain_div((alr - blr) * (l1 * l2), l2 - l1);
     } else {
         a0 = lmax;
     }
@@ -293,10 +297,10 @@ __device__ __forceinline__ MF<T> mom_waf(const bool yface, SC<T> m, SC<T> a, SC<
     T f0 = a.f, f1 = b.f;
     T u0 = f0 * q0, u1 = f1 * q1;
     if (!yface) { q0 = u0 * h0; q1 = u1 * h1; }
-    T s0 = Num<T>::sqrt(h0), s1 = Num<T>::sqrt(h1);
-    T uij = Num<T>::div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
+    T s0 = Num<T>::depth_sqrt(h0), s1 = Num<T>::depth_sqrt(h1);
+    T uij = Num<T>::plain_div(Num<T>::mad(s0, u0, s1 * u1), s0 + s1 + Num<T>::eps);
     T val = valf * dt;
-    T c0 = Num<T>::sqrt(hij);
+    T c0 = Num<T>::plain_sqrt(hij);
     T l1 = tmin(uij - c0, u0 - s0);
     T l2 = tmax(uij + c0, u1 + s1);
     T lmax = tmax(tabs(l2), tabs(l1));
@@ -320,7 +324,7 @@ __device__ __forceinline__ MF<T> mom_waf(const bool yface, SC<T> m, SC<T> a, SC<
         T ft = uu * qt * L;
         sm_t = ft;
         sp_t = -ft;
-        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::div(p.hpos, hij)))));
+        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::plain_div(p.hpos, hij)))));
         T des = cd * val * lmax * lmax * dq * L;
         if (!yface) des *= normal;
         sm_n -= des * ic0;
@@ -336,7 +340,7 @@ __device__ __forceinline__ MF<T> mom_waf(const bool yface, SC<T> m, SC<T> a, SC<
     if (tabs(l1 - l2) >= Num<T>::eps) {
         T alr = Num<T>::mad(val * l1, xiL, sgn(l1) * (T(1) - xiL));
         T blr = Num<T>::mad(val * l2, xiR, sgn(l2) * (T(1) - xiR));
-        T aux = Num<T>::rcp(l2 - l1);
+        T aux = Num<T>::plain_rcp(l2 - l1);
         a0 = (alr - blr) * (l1 * l2) * aux;
         a1 = Num<T>::mad(blr, l2, -(alr * l1)) * aux;
     } else {

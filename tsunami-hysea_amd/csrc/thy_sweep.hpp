@@ -713,7 +713,7 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
                     // metrics from the state before the step (src/GPU/Metrics.cu:23-42,57-77)
                     const bool max_on = out_col && eo > cmax && eo + D2 > a.eps_h;
                     const bool arr_on = out_col && a.track_arrival && !Arrival<T>::arrived(carr) && tabs(eo - carr) > a.dif_at;
-                    const T dtc = (W2 < Num<T>::eps) ? Num<T>::big : Num<T>::div(T(2) * a.cfl * rg.A, W2);
+                    const T dtc = (W2 < Num<T>::eps) ? Num<T>::big : Num<T>::plain_div(T(2) * a.cfl * rg.A, W2);
                     dtmin = fminf(dtmin, (float)dtc);  // halo lanes are dropped at the end
                     const T val = dt * rg.invA;
                     T qx = Num<T>::mad(val, X2, qx2), qy = Num<T>::mad(val, Y2, qy2);
