@@ -376,7 +376,7 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
         for (int t = 0; t < KL; t++) {
             const int i = wv + t * W;
             const T h = v[t][0] + v[t][1];
-            still = still && !(h > Num<T>::eps) && v[t][2] == T(0) && v[t][3] == T(0);
+            still = still && h <= Num<T>::eps && v[t][2] == T(0) && v[t][3] == T(0);  // (no NaN)
             if (i < m + 8) {
                 const int p = i * 64 + lane;
                 s.in[0][p] = v[t][0];
@@ -405,8 +405,8 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
     const int gw = per ? cx : gx;
     const mask64 first = __ballot(gw < 2 || gw > nx - 2);
     const T *const e_ = s.in[0], *const D_ = s.in[1], *const qx_ = s.in[2], *const qy_ = s.in[3];
-    // Land: every cell of the tile and its halo dry and without discharge, clear of the
-    // sponges.  Every face is then zero and the update leaves e (its depth stays 0) and
+    // Land: every cell of the tile and its halo dry and without discharge (a depth that is not
+    // a number takes the other way, where the health check finds it), clear of the sponges.  Every face is then zero and the update leaves e (its depth stays 0) and
     // zero discharges; the arrival rule may still record the start (a dry cell's eta_ini
     // is a marker).
     __syncthreads();
