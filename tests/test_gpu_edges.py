@@ -33,3 +33,24 @@ def test_land_that_is_not_finite(kernel):
         s.step(1e-4)
     assert e.value.code == native.STATUS_CODES["NONFINITE"]
     s.close()
+
+
+@pytest.mark.parametrize("kernel", ["sweep", "sweep_general", "tile"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_without_a_state(kernel, precision):
+    """A context without an upload holds dry cells of depth 0: it steps and runs, and stays
+    as it is (a run has no wave to wait for, so its first step may reach the end); an upload
+    afterwards gives the run of a fresh context."""
+    from thysea import native
+    pr = make_problem(nx=190, ny=61, seed=9)
+    s = native.Solver(pr, upload=False, kernel=kernel, precision=precision)
+    assert s.step(1e-4) > 0
+    assert s.run(max_steps=7, faults=[])["steps"] >= 1
+    assert all(np.all(x == 0) for x in (s.state()[0], s.state()[2], s.state()[3]))
+    s.upload(pr.h, pr.H, pr.qx, pr.qy)
+    f = native.Solver(pr, kernel=kernel, precision=precision)
+    for x in (s, f):
+        x.run(max_steps=7)
+    assert all(np.array_equal(a, b) for a, b in zip(s.state(), f.state()))
+    s.close()
+    f.close()

@@ -493,7 +493,7 @@ size_t segment_rows(const thy_ctx *c) { return (size_t)((c->nx + SW_OUT - 1) / S
 // Coast along the row sweep's 56-column segments.  A segment row is coastal when any cell of
 // its 64 columns is shallower than 3 hpos (or dry).  Its cost is an estimate of the faces
 // that will not take the deep form: those of the wet cells shallower than hpos and of the
-// cells on either side of a shoreline.
+// cells on either side of a shoreline.  D null: no state yet, depth 0 everywhere.
 template <typename T>
 void find_coast(thy_ctx *c, const T *D) {
     const int nx = c->nx, ny = c->ny, P = c->pitch;
@@ -504,11 +504,11 @@ void find_coast(thy_ctx *c, const T *D) {
     for (int j = 0; j < ny; j++) {
         for (int sgi = 0; sgi < nseg; sgi++) {
             const int xa = std::max(0, sgi * SW_OUT - SW_HALO), xb = std::min(nx, sgi * SW_OUT + SW_OUT + SW_HALO);
-            const T *d = D + (size_t)j * P;
-            bool any = false;
+            const T *d = D ? D + (size_t)j * P : nullptr;
+            bool any = !D;
             for (int i = xa; i < xb && !any; i++) any = d[i] <= thr;
             int n = 0;
-            for (int i = xa; any && i < xb; i++) {
+            for (int i = xa; d && any && i < xb; i++) {
                 const bool dry = d[i] <= T(0);
                 n += (!dry && d[i] <= hpos) || (i > xa && dry != (d[i - 1] <= T(0)));
             }
@@ -602,16 +602,22 @@ int build_alone(thy_ctx *ctx, const int S, const int R) {
     return build_lists(ctx, ctx->alone, def <= 8 ? std::min(S, def) : S, R, budget);
 }
 
-// the lists of an uploaded state
+// the lists of an uploaded state (D null: of the state a context has before one)
 template <typename T>
 int build_order(thy_ctx *ctx, const T *D) {
     if (ctx->kernel == 1) return THY_OK;
     find_coast(ctx, D);
-    ctx->uploaded = true;
+    ctx->uploaded = D != nullptr;
     ctx->batched.n_items = 0;  // built again when a batch asks for them
     const size_t rows = segment_rows(ctx);
     return build_alone(ctx, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : default_strip_rows(rows, ctx->ncu),
                        ctx->prm.general_rows > 0 ? std::min(ctx->prm.general_rows, kTileRows) : default_tile_rows(rows, ctx->ncu));
+}
+
+// a context may be stepped before a state was uploaded
+int need_lists(thy_ctx *ctx) {
+    if (ctx->kernel == 1 || ctx->alone.n_items > 0) return THY_OK;
+    return ctx->prec ? build_order<double>(ctx, nullptr) : build_order<float>(ctx, nullptr);
 }
 
 // The lists a batch steps the scenario by.  Its scenarios fill the device whatever their
@@ -1452,6 +1458,7 @@ int thy_step(thy_ctx *ctx, double dt, double *dt_next) {
     RelaxedCapture relaxed;
     if (!ctx) return THY_ERR_INVALID;
     int r;
+    if ((r = need_lists(ctx)) != THY_OK) return r;
     Ctrl c = idle_ctrl(ctx);
     c.dt = dt;
     c.dt_valid = 1;
@@ -1641,6 +1648,7 @@ static int prepare_run(thy_ctx *ctx, const thy_run_config *cfg, thy_run_result *
     if (cfg->n_faults < 0 || (cfg->n_faults > 0 && !cfg->faults) || (cfg->n_gauges > 0 && !cfg->gauge_pos))
         return fail(ctx, THY_ERR_INVALID, "bad run configuration");
     int r;
+    if ((r = need_lists(ctx)) != THY_OK) return r;
     memset(res, 0, sizeof(*res));
     ctx->batch_ready = false;  // a run prepared before is replaced
     ctx->K = cfg->steps_per_sync > 0 ? cfg->steps_per_sync : 24;
