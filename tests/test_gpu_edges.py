@@ -54,3 +54,14 @@ def test_without_a_state(kernel, precision):
     assert all(np.array_equal(a, b) for a, b in zip(s.state(), f.state()))
     s.close()
     f.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kernel", ["sweep", "tile"])
+def test_infinite_threshold(kernel, precision):
+    """hpos infinite: every face takes the WAF flux with blend weight 0, as the limit of the
+    formulas says (exp of an infinite argument)."""
+    from test_gpu_tiles import _replay
+    pr = make_problem(nx=130, ny=44, seed=3)
+    pr.hpos = float("inf")
+    _replay(pr, 8, precision=precision, kernel=kernel)
