@@ -760,7 +760,7 @@ __device__ __forceinline__ void block_dt_min(const StepArgs<T> &a, const int slo
 // the 2s faces: no sponge and no near-dry update, no clamped columns or rows.  Every
 // wavefront checks at run time the conditions under which the general faces take the 2s
 // branch (every loaded row deeper than hpos; every h* row that a face's stencil reaches
-// deeper than hpos).  A strip whose check fails commits no dt and is redone as general
+// deeper than hpos).  The rows of a strip where they do not hold are redone as general
 // tiles by its workgroup in the same launch (tile_or_strips); both evaluate the deep faces
 // with the same functions, so the split changes no result.
 // ---------------------------------------------------------------------------
@@ -777,13 +777,18 @@ __device__ __forceinline__ double here(double v) { return v; }
 // accumulation order is that of the general tiles (x faces, lower y face, upper y face), so
 // the values are the same.
 //
-// The conditions under which the general faces take the 2s branch and its eta difference is
-// e1 - e0 (every row y0-4 .. y1+3 and every h* deeper than hpos on every lane, both eta of a
-// face above the shallower bed, no h* clipped at the bed) follow from one: the lowest eta
-// plus the smallest depth of the strip exceeds hpos.  (A rounded sum is monotonic in its
-// terms.)  Two running minima a row take the place of a vote for each.  Returns whether it
-// held; if not, the caller redoes the strip (its writes are then rewritten and its dt is
-// dropped).
+// kCareful false: the conditions under which the general faces take the 2s branch and its
+// eta difference is e1 - e0 (every h and h* deeper than hpos, both eta of a face above the
+// shallower bed, no h* clipped at the bed) follow from one: the lowest eta plus the smallest
+// depth exceeds hpos.  (A rounded sum is monotonic in its terms.)  It is taken over two
+// columns and some eight rows at a time, with three running minima a row: over more, a
+// trough would meet the bed of a shallow far from it (with the minima of a whole strip, a
+// 2000x2000 step with 4.5 m troughs ten rows off ridges 5 m deep and hpos 1 m took 243 us
+// instead of the 40 of a level sea; it takes 40).  Returns false where it fails, and the caller takes the strip again with
+// kCareful true: the eta difference in its general form, and h and h* compared with hpos row
+// by row.  Row y needs the inputs of rows y-4 .. y+4 and h* of rows y-2 .. y+2; the rows for
+// which one of them is too shallow lie in [ya, yb), for the caller to redo (what was stored
+// for them is then overwritten); the others are done, their dt and health included.
 //
 // Bound by memory on a large grid (4000x3000, all deep: 111 us a step, 3.9 TB/s of the nine
 // arrays, whatever the strip height, and no less with two rows of cells in flight), by the
@@ -792,9 +797,9 @@ __device__ __forceinline__ double here(double v) { return v; }
 // limiter branches, copies from row to row, which two rows of the loop written out spare;
 // four rows are no faster).  2000x2000: 54.9 us a step before, 49.7 now; 1000x800 20.8 and
 // 18.6; FP64 2000x2000 143.5 and 134.3.
-template <typename T>
+template <typename T, bool kCareful>
 __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<T> &bc, const int x0, const int y0,
-                                           const int rows, float &dtmin_out) {
+                                           const int rows, float &dtmin_out, int &ya, int &yb) {
     const int lane = threadIdx.x & 63;
     const bool c1 = __builtin_amdgcn_readfirstlane(bc.cur) != 0;
     const T dt = (T)bc.dt;
@@ -825,10 +830,19 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
     const DeepRow<T> *const geo = a.deep_row;
     float dtmin = 3.0e38f;
     T nan_acc = T(0);  // turns NaN when a stored value is not finite
-    // rows y0-4 and y1+3 enter only the conditions
-    T smin = Num<T>::big;  // of h* (lanes 0 and 63 lack a face and are left out)
-    T emin = tmin(buf_load<T>(rs, ve, (y0 - 4) * P), buf_load<T>(rs, ve, (y1 + 3) * P));
-    T Dmin = tmin(buf_load<T>(rs, vD, (y0 - 4) * P), buf_load<T>(rs, vD, (y1 + 3) * P));
+    const T least = tmax(a.hpos, T(0));
+    // rows y0-4 and y1+3 enter only the conditions, as inputs
+    const bool first_ok = __all(buf_load<T>(rs, ve, (y0 - 4) * P) + buf_load<T>(rs, vD, (y0 - 4) * P) > least);
+    const bool last_ok = __all(buf_load<T>(rs, ve, (y1 + 3) * P) + buf_load<T>(rs, vD, (y1 + 3) * P) > least);
+    // kCareful false: least eta of the inputs, eta of h* and depth since the last check
+    T emin = Num<T>::big, smin = Num<T>::big, Dmin = Num<T>::big;
+    // kCareful true: the rows from lo on, and before hi, are those that need a cell too shallow;
+    // dt of rows r-3 and r-4, and whether those rows (bits 0 and 1), or a row that is kept, hold
+    // a value that is not finite
+    int lo = first_ok ? y1 : y0, hi = first_ok ? y0 : y0 + 1;
+    float d1 = 3.0e38f, d2 = 3.0e38f;
+    unsigned bad_rows = 0u;
+    bool bad = false;
     // pipeline registers: rows r-2 and r-1 with their depths, h* of row r-2 with sqrt(h*)
     // and qy/h*, mass accumulator of row r-1, momentum accumulators of row r-2
     RowCell<T> i2 = RowCell<T>{T(0), T(0), T(0), T(0)}, i1 = i2;
@@ -836,6 +850,16 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
     T X2 = T(0), Y2 = T(0), W2 = T(0);
     RowCell<T> buf = load_row((y0 - 3) * P);
     T pm = buf_load<T>(rs, vm, y0 * P), pt = buf_load<T>(rs, va, y0 * P);
+    auto spoil = [&](const int ya, const int yb) {
+        lo = min(lo, ya);
+        hi = max(hi, yb);
+    };
+    // row y, whose inputs have all been seen, is done unless one of them was too shallow
+    auto keep = [&](const int y) {
+        if (y >= lo && y < hi) return;
+        dtmin = fminf(dtmin, d2);
+        bad = bad || (bad_rows & 2u);
+    };
     // One row of the pipeline.  In the steady state (rows y0+2 .. y1) every stage applies,
     // so the stage conditions drop out at compile time; the other rows keep them.  Both
     // forms evaluate the same expressions.
@@ -853,8 +877,13 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
         }
         const int ju = r - 2, j1 = r - 1;  // the row updated in this iteration, the row of h*
         const T h0 = i0.e + i0.D;
-        emin = Num<T>::min(emin, i0.e);
-        Dmin = Num<T>::min(Dmin, i0.D);
+        if constexpr (!kCareful) {
+            emin = Num<T>::min(emin, i0.e);
+            Dmin = Num<T>::min(Dmin, i0.D);
+        }
+        if constexpr (kCareful) {
+            if (!__all(h0 > least)) spoil(r - 4, r + 5);
+        }
         // mass x faces of row r (h* rows y0-2 .. y1+1), y face r between rows r-1 and r
         // (faces y0-2 .. y1+2).  The limiter rarely acts: one test for both faces.
         T m0 = T(0);
@@ -869,8 +898,11 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
         T s1 = T(0), hs1 = T(0), sq1 = T(0), u1 = T(0), v1 = T(0);
         if (kS || (j1 >= y0 - 2 && j1 <= y1 + 1)) {
             s1 = Num<T>::mad(dt * g.p.invA, m1, i1.e);
-            smin = Num<T>::min(smin, s1);
+            if constexpr (!kCareful) smin = Num<T>::min(smin, s1);
             hs1 = s1 + i1.D;
+            if constexpr (kCareful) {
+                if (!__all(lane == 0 || lane == 63 || hs1 > least)) spoil(j1 - 2, j1 + 3);  // (these lack a face)
+            }
             sq1 = Num<T>::plain_sqrt(hs1);
             const T ih = Num<T>::plain_rcp(hs1);
             u1 = i1.qx * ih;
@@ -881,7 +913,8 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
         if (kS || (j1 >= y0 && j1 < y1)) {
             const DC<T> A{dpp_left(hs1), dpp_left(i1.qx), dpp_left(i1.qy), dpp_left(sq1), dpp_left(u1)};
             const DC<T> B{hs1, i1.qx, i1.qy, sq1, u1};
-            const MF<T> f = fast_mom_x(A, B, s1 - dpp_left(s1), g.p.ilx, g.p.kdx, dt);
+            const T sL = dpp_left(s1), deta = kCareful ? deta_of(sL, s1, dpp_left(i1.D), i1.D) : s1 - sL;
+            const MF<T> f = fast_mom_x(A, B, deta, g.p.ilx, g.p.kdx, dt);
             X1 = here(-f.pn - dpp_right(f.mn));
             Y1 = here(-f.pt - dpp_right(f.mt));
             W1 = here(f.w + dpp_right(f.w));
@@ -889,7 +922,7 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
         // momentum y face r-1 between rows r-2 and r-1 (faces y0 .. y1)
         if (kS || (j1 >= y0 && j1 <= y1)) {
             const DC<T> A{hs2, i2.qy, i2.qx, sq2, v2}, B{hs1, i1.qy, i1.qx, sq1, v1};
-            const MF<T> f = fast_mom_y(A, B, s1 - s2, g.p, dt);
+            const MF<T> f = fast_mom_y(A, B, kCareful ? deta_of(s2, s1, i2.D, i1.D) : s1 - s2, g.p, dt);
             Y2 -= f.mn;
             X2 -= f.mt;
             W2 += f.w;
@@ -909,10 +942,17 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
             buf_store<T>(eo, rs, (max_on ? vout : kDropOffset) + o.emax, so);
             buf_store<T>(tnow, rs, (arr_on ? vout : kDropOffset) + o.arr, so);
             const T dtc = W2 < Num<T>::eps ? Num<T>::big : Num<T>::plain_div(cfl2 * g.q.A, W2);
-            if (on) dtmin = Num<float>::min(dtmin, (float)dtc);  // halo lanes: dropped below
             const T val = dt * g.q.invA;
             const T qx = Num<T>::mad(val, X2, i2.qx), qy = Num<T>::mad(val, Y2, i2.qy);
-            if (on) nan_acc = Num<T>::mad(s2, T(0), Num<T>::mad(qx, T(0), Num<T>::mad(qy, T(0), nan_acc)));
+            if constexpr (kCareful) {
+                keep(r - 4);
+                d2 = d1;
+                d1 = on ? (float)dtc : 3.0e38f;
+                bad_rows = bad_rows << 1 | (on && __any(out_col && bad_cell(s2, qx, qy)) ? 1u : 0u);
+            } else {
+                if (on) dtmin = Num<float>::min(dtmin, (float)dtc);  // halo lanes: dropped below
+                if (on) nan_acc = Num<T>::mad(s2, T(0), Num<T>::mad(qx, T(0), Num<T>::mad(qy, T(0), nan_acc)));
+            }
             buf_store<T>(s2, rs, kS || on ? we : kDropOffset, so);
             buf_store<T>(qx, rs, kS || on ? wqx : kDropOffset, so);
             buf_store<T>(qy, rs, kS || on ? wqy : kDropOffset, so);
@@ -931,67 +971,94 @@ __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<
     // only has the previous rows to account for (their stores may stay in flight while the
     // next row loads), instead of a full wait every row.
     __builtin_amdgcn_s_waitcnt(0);
+    int r = y0 - 3;
+    ya = yb = 0;
+    // kCareful false: the condition for the rows since the last check; the next ones begin
+    // with the faces between rows r-2 and r-1
+    auto check = [&] {
+        const T e = lane == 0 || lane == 63 ? emin : Num<T>::min(emin, smin);  // (these lack a face)
+        const T E = Num<T>::min(e, dpp_left(e)), D = Num<T>::min(Dmin, dpp_left(Dmin));
+        emin = Num<T>::big;
+        smin = s2;
+        Dmin = Num<T>::min(i1.D, i2.D);
+        return kCareful || __all(lane == 0 || E + D > least) != 0;
+    };
     // rows y0-3 .. y1+2: the halo rows at either end (and a last row without a partner)
     // with the stage conditions, the steady state without them
-    int r = y0 - 3;
 #pragma unroll 1
     for (; r <= y0 + 1; r++) row(r, Edge{});
+    bool valid = kCareful || (first_ok && last_ok && check());
 #pragma unroll 1
-    for (; r + 1 <= y1; r += 2) {
-        row(r, Steady{});
-        row(r + 1, Steady{});
+    while (valid && r < y1) {
+        const int re = kCareful ? y1 : min(r + 7, y1);
+#pragma unroll 1
+        for (; r < re; r += 2) {
+            row(r, Steady{});
+            row(r + 1, Steady{});
+        }
+        valid = check();
     }
+    if (!valid) return false;
 #pragma unroll 1
     for (; r <= y1 + 2; r++) row(r, Edge{});
-    // (the minima are taken over the wavefront first: a face joins the eta of one lane with
-    // the depth of another)
-    const T floor_h = wave_min(lane == 0 || lane == 63 ? emin : Num<T>::min(emin, smin)) + wave_min(Dmin);
-    const bool valid = floor_h > tmax(a.hpos, T(0));
-    // a strip whose check failed is redone, and checked, as general tiles
-    if (valid) raise_health(a, out_col && nan_acc != nan_acc);
+    if constexpr (kCareful) {
+        if (!last_ok) spoil(y1 - 1, y1);
+        keep(y1 - 1);
+        if (lo < hi) {
+            ya = max(y0, lo);
+            yb = min(y1, hi);
+        }
+    } else {
+        if (!check()) return false;
+        bad = out_col && nan_acc != nan_acc;
+    }
+    raise_health(a, bad);
     dtmin_out = out_col ? dtmin : 3.0e38f;
-    return valid;
+    return true;
 }
 
 // One workgroup's share of a step.  A tile item: the general tile (x0, y0, rows).  A deep
-// item: the strip (x0, y0, rows) of each wavefront; a strip whose check fails is redone
-// here, tile by tile, by the whole workgroup (the values it has stored are overwritten;
-// its metric updates used the state before the step and stand).
+// item: the strip (x0, y0, rows) of each wavefront; the rows that deep_strip leaves undone
+// are redone here, tile by tile, by the whole workgroup (the values it has stored are
+// overwritten; its metric updates used the state before the step and stand).
 template <typename T>
 __device__ __forceinline__ float tile_or_strips(const ArgsAt<T> args, const BlockCtl<T> &bc, const bool tile, int x0, int y0,
                                                 int rows, TileLds<T> &s, int *s_fail) {
     float dtmin = 3.0e38f;
-    int n_tiles = 1, per = 1;
     if (!tile) {
         const int wv = threadIdx.x >> 6;
-        bool ok = true;
-        if (x0 >= 0) ok = deep_strip(again<T>(args), bc, x0, y0, rows, dtmin);
-        if (!ok) {
-            dtmin = 3.0e38f;
-            __threadfence();  // its stores land before those that replace them
+        int ya = 0, yb = 0;
+        if (x0 >= 0 && !deep_strip<T, false>(again<T>(args), bc, x0, y0, rows, dtmin, ya, yb)) {
+            deep_strip<T, true>(again<T>(args), bc, x0, y0, rows, dtmin, ya, yb);
+            // its stores reach the L2, which every wavefront of the workgroup writes through
+            // to, before those that replace them (a fence for other XCDs would write it back)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         if ((threadIdx.x & 63) == 0) {
-            s_fail[3 * wv] = ok ? -1 : x0;
-            s_fail[3 * wv + 1] = y0;
-            s_fail[3 * wv + 2] = ok ? 0 : rows;
+            s_fail[3 * wv] = x0;
+            s_fail[3 * wv + 1] = ya;
+            s_fail[3 * wv + 2] = yb - ya;
         }
         __syncthreads();
-        int most = 0;
-        for (int w = 0; w < SW_WAVES; w++) most = max(most, __builtin_amdgcn_readfirstlane(s_fail[3 * w + 2]));
-        if (most == 0) return dtmin;
-        per = (most + kTileRows - 1) / kTileRows;
-        n_tiles = SW_WAVES * per;
     }
-    for (int t = 0; t < n_tiles; t++) {
-        if (!tile) {  // tile t - w * per of the strip of wavefront w
-            const int w = t / per, d = (t - w * per) * kTileRows;
+    for (int w = 0, t = 0;;) {
+        if (!tile) {  // tile t of the rows left by wavefront w
+            int n = 0, tiles = 0;
+            for (; w < SW_WAVES; w++, t = 0) {
+                n = __builtin_amdgcn_readfirstlane(s_fail[3 * w + 2]);
+                tiles = (n + kTileRows - 1) / kTileRows;
+                if (t < tiles) break;
+            }
+            if (w == SW_WAVES) break;
+            const int ya = __builtin_amdgcn_readfirstlane(s_fail[3 * w + 1]), d = n * t / tiles;
             x0 = __builtin_amdgcn_readfirstlane(s_fail[3 * w]);
-            y0 = __builtin_amdgcn_readfirstlane(s_fail[3 * w + 1]) + d;
-            rows = min(kTileRows, __builtin_amdgcn_readfirstlane(s_fail[3 * w + 2]) - d);
-            if (x0 < 0 || rows <= 0) continue;
+            y0 = ya + d;
+            rows = n * (t + 1) / tiles - d;
+            t++;
             __syncthreads();  // the tile before still uses the rows in LDS
         }
         dtmin = fminf(dtmin, general_tile(args, bc, x0, y0, rows, s));
+        if (tile) break;
     }
     return dtmin;
 }
