@@ -154,11 +154,10 @@ template <typename T> __device__ __forceinline__ T deta_of(T e0, T e1, T D0, T D
 }
 
 // 2s/WAF blend: src/GPU/Arista_kernel.cu:205-208
-// (hpos may be infinite: the general quotient)
 template <typename T> __device__ __forceinline__ T blend(T hij, T hpos, bool alfa_cero) {
     if (alfa_cero) return T(0);
     if (hij < hpos)
-        return Num<T>::rcp(T(1) + Num<T>::exp(T(-15) * (T(1) - Num<T>::div(T(0.5) * hpos, hij + Num<T>::eps))));
+        return Num<T>::rcp(T(1) + Num<T>::exp(T(-15) * (T(1) - Num<T>::plain_div(T(0.5) * hpos, hij + Num<T>::eps))));
     return T(1);
 }
 
@@ -327,7 +326,7 @@ __device__ __forceinline__ MF<T> mom_waf(const bool yface, SC<T> m, SC<T> a, SC<
         T ft = uu * qt * L;
         sm_t = ft;
         sp_t = -ft;
-        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::div(p.hpos, hij)))));
+        T cd = T(0.5) * (T(1) - Num<T>::div(p.cvis, T(1) + Num<T>::exp(T(-20) * (T(1) - Num<T>::plain_div(p.hpos, hij)))));
         T des = cd * val * lmax * lmax * dq * L;
         if (!yface) des *= normal;
         sm_n -= des * ic0;
