@@ -69,8 +69,7 @@ typedef struct thy_params {
     int kernel;        /* step kernel: 0 row sweep, deep-water strips and general tiles (default),
                           1 2D LDS tiles, 2 row sweep with general tiles everywhere */
     int strip_rows;    /* row-sweep kernel: most rows of a deep-water strip, 0: default (by the
-                          grid's size, 8 to 32; 24 in a batch).  A small grid stepped alone
-                          takes strips of at most 8 rows */
+                          grid's size, 8 to 32; 24 in a batch) */
     int general_rows;  /* row-sweep kernel: rows per general tile, at most 8 are used, 0: default
                           (by the grid's size and the coast, 3 to 8; 8 in a batch) */
 } thy_params;

@@ -1,0 +1,29 @@
+"""Heights of strips and tiles that a caller asks for are the ones that run.  No result depends
+on them, so they show in the time of a step: heights are chosen that cost several times the
+default's (a strip is a chain of rows, 0.5 us each and more), and the bounds are half of that."""
+import numpy as np
+import pytest
+
+from conftest import make_problem
+
+pytestmark = pytest.mark.gpu
+
+
+def _us(s, n=48, reps=5):
+    """Us a step of a run in progress, the median of reps."""
+    return float(np.median([s.run_more(n)["seconds"] for _ in range(reps)])) / n * 1e6
+
+
+def _solver(pr, **kw):
+    from thysea import native
+    s = native.Solver(pr, **kw)
+    s.run(max_steps=48, steps_per_sync=48)
+    return s
+
+
+def test_tall_strips_on_a_small_grid():
+    """One strip of deep water from border to border, where the default has strips of 8 rows."""
+    pr = make_problem(nx=1000, ny=800, seed=9, coast=(), seamounts=0, t_sim=1e6)
+    a, b = _solver(pr), _solver(pr, strip_rows=788)
+    assert _us(b) > 4 * _us(a)
+    assert all(np.array_equal(x, y) for x, y in zip(a.state(), b.state()))

@@ -598,11 +598,8 @@ int build_alone(thy_ctx *ctx, const int S, const int R) {
     drop_graphs(ctx);  // the captured step sequences hold the old lists and grid sizes
     ctx->srows = S;
     ctx->trows = R;
-    // where the default is the shortest strip, taller ones only leave the device idle
-    const size_t rows = segment_rows(ctx);
-    const int def = default_strip_rows(rows, ctx->ncu);
-    const int budget = ctx->prm.general_rows > 0 ? INT_MAX : tile_budget(rows, ctx->ncu);
-    return build_lists(ctx, ctx->alone, def <= 8 ? std::min(S, def) : S, R, budget);
+    const int budget = ctx->prm.general_rows > 0 ? INT_MAX : tile_budget(segment_rows(ctx), ctx->ncu);
+    return build_lists(ctx, ctx->alone, S, R, budget);
 }
 
 // the lists of an uploaded state (D null: of the state a context has before one)
