@@ -198,12 +198,13 @@ size_t thy_footprint(int nx, int ny, const thy_params *params);
 int thy_copy_probe(size_t bytes, int reps, double *ms_per_copy);
 
 /* Strip-height autotuner of the row-sweep kernel.  No reference counterpart (the
-   reference has one fixed launch shape).  For pairs of strip height and tile height (16/4,
-   16/8, 24/8, 32/8, 36/8, 40/8, 48/8) it captures 32 steps from the current state
-   into a graph (each step redoes the same step), times `reps` replays (HIP events,
-   median) and keeps the fastest; the state, control
+   reference has one fixed launch shape).  For the pair of strip height and tile height in
+   use, and others (16/4, 16/8, 24/8, 32/8, 36/8, 40/8, 48/8), it captures 32 steps from the
+   current state into a graph (each step redoes the same step), times `reps` replays (HIP
+   events, median) and keeps the fastest, also over later uploads; the state, control
    blocks and dt slots are left as they were.  Call after thy_upload_state, before or
-   between runs.  general_rows may be null. */
+   between runs.  Returns the heights kept; general_rows may be null.  On a grid whose
+   default strip height is 8 the tuner's strips have 8 rows too, and 16 stands for them. */
 int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, double *ms_per_step);
 
 /* Wall time (ms) of the last kernel launch group, for benchmarking. */

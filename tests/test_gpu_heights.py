@@ -27,3 +27,26 @@ def test_tall_strips_on_a_small_grid():
     a, b = _solver(pr), _solver(pr, strip_rows=788)
     assert _us(b) > 4 * _us(a)
     assert all(np.array_equal(x, y) for x, y in zip(a.state(), b.state()))
+
+
+def test_autotune_starts_from_the_heights_in_use():
+    """FP64 500x400 without a coast is fastest with strips lower than any the tuner tries (3 rows
+    against 8: a chain of 11 rows against 16, 14 us against 17); they stay."""
+    pr = make_problem(nx=500, ny=400, seed=9, coast=(), seamounts=0, t_sim=1e6)
+    s = _solver(pr, precision=1, strip_rows=3)
+    before = s.state()
+    assert s.autotune(5)[0] == 3
+    assert all(np.array_equal(x, y) for x, y in zip(before, s.state()))
+
+
+def test_tuned_heights_survive_an_upload():
+    """A height that autotune replaced does not come back with the next state."""
+    pr = make_problem(nx=1000, ny=800, seed=9, coast=(), seamounts=0, t_sim=1e6)
+    s = _solver(pr, strip_rows=788)
+    slow = _us(s)
+    rows, _ = s.autotune(5)
+    assert rows < 100 and _us(s) < slow / 4
+    s.upload(pr.h, pr.H, pr.qx, pr.qy)
+    s.run(max_steps=48, steps_per_sync=48)
+    assert _us(s) < slow / 4
+    assert s.autotune(5)[0] < 100

@@ -91,6 +91,7 @@ struct thy_ctx {
     int kernel = 0;              // 0 row sweep (deep-water strips and general tiles), 1 2D tiles, 2 general tiles only
     int srows = 24;              // row sweep: rows per deep-water strip
     int trows = kTileRows;       //   rows per general tile
+    int tuned_srows = 0, tuned_trows = 0;  // the heights thy_autotune chose (0: it has not run)
     int tuning = 0;              // launches recorded for timing replays publish no control block
     int ncu = 256;               // compute units of the device
     bool uploaded = false;       // row sweep: the lists describe an uploaded state
@@ -593,9 +594,10 @@ int build_lists(thy_ctx *ctx, WorkLists &w, int S, const int R, const int budget
 }
 
 // the lists of a run alone, with deep-water strips of S rows and tiles of R rows
-int build_alone(thy_ctx *ctx, const int S, const int R) {
+int build_alone(thy_ctx *ctx, int S, const int R) {
     if (ctx->kernel == 1) return THY_OK;
     drop_graphs(ctx);  // the captured step sequences hold the old lists and grid sizes
+    S = std::min(S, 2047);  // (a strip's record holds its height in 11 bits)
     ctx->srows = S;
     ctx->trows = R;
     const int budget = ctx->prm.general_rows > 0 ? INT_MAX : tile_budget(segment_rows(ctx), ctx->ncu);
@@ -609,6 +611,7 @@ int build_order(thy_ctx *ctx, const T *D) {
     find_coast(ctx, D);
     ctx->uploaded = D != nullptr;
     ctx->batched.n_items = 0;  // built again when a batch asks for them
+    if (ctx->tuned_srows > 0) return build_alone(ctx, ctx->tuned_srows, ctx->tuned_trows);
     const size_t rows = segment_rows(ctx);
     return build_alone(ctx, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : default_strip_rows(rows, ctx->ncu),
                        ctx->prm.general_rows > 0 ? std::min(ctx->prm.general_rows, kTileRows) : default_tile_rows(rows, ctx->ncu));
@@ -1386,14 +1389,25 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
     c.dt = dt;
     c.dt_valid = 1;
     c.cur = ctx->cur;
-    // (strip rows, tile rows)
-    const int cand[][2] = {{16, 4}, {16, 8}, {24, 8}, {32, 8}, {36, 8}, {40, 8}, {48, 8}};
-    int best = ctx->srows, best_g = ctx->trows;
+    // The heights in use, then those of a table of which none is built twice.  On a grid whose
+    // default is 8 rows the table's strips are cut to 8: taller ones only leave the device
+    // idle there (us a step at 8 / 16 / 24 rows: 131x97 11.8 / 13.2 / 16.3, 500x400 12.4 / 15.2 /
+    // 18.4, 1000x800 15.9 / 18.1 / 22.0).  The table's name for the default is then 16.
+    struct Pair { int name, strip, tile; };
+    const int def = default_strip_rows(segment_rows(ctx), ctx->ncu);
+    const bool own = ctx->prm.strip_rows > 0;
+    const int table[][2] = {{16, 4}, {16, 8}, {24, 8}, {32, 8}, {36, 8}, {40, 8}, {48, 8}};
+    std::vector<Pair> cand = {{!own && ctx->srows == 8 ? 16 : ctx->srows, ctx->srows, ctx->trows}};
+    for (const auto &sg : table) {
+        const Pair p{sg[0], def <= 8 ? def : sg[0], sg[1]};
+        bool known = sg[0] > ctx->ny;
+        for (const Pair &q : cand) known = known || (q.strip == p.strip && q.tile == p.tile);
+        if (!known) cand.push_back(p);
+    }
+    Pair best = cand[0];
     double best_ms = 1e30;
-    for (const auto &sg : cand) {
-        const int S = sg[0];
-        if (S > ctx->ny && S != cand[0][0]) continue;
-        if ((r = build_alone(ctx, S, sg[1])) != THY_OK) return r;
+    for (const Pair &sg : cand) {
+        if ((r = build_alone(ctx, sg.strip, sg.tile)) != THY_OK) return r;
         // kSeq steps captured into one graph and replayed, as a run replays its steps.
         // The launches cycle through the three launch slots as in a run, but publish no
         // control block: every slot holds the same control block, each step reads the
@@ -1440,16 +1454,17 @@ int thy_autotune(thy_ctx *ctx, int reps, int *strip_rows, int *general_rows, dou
         const double med = t[t.size() / 2];
         if (med < best_ms) {
             best_ms = med;
-            best = S;
-            best_g = sg[1];
+            best = sg;
         }
     }
-    if ((r = build_alone(ctx, best, best_g)) != THY_OK) return r;
+    if ((r = build_alone(ctx, best.strip, best.tile)) != THY_OK) return r;
+    ctx->tuned_srows = best.strip;
+    ctx->tuned_trows = best.tile;
     ctx->slot = saved_slot;
     HIPCHK(ctx_copy(ctx, ctx->ctrl, saved, sizeof(saved), hipMemcpyHostToDevice));
     HIPCHK(ctx_copy(ctx, ctx->dtmin, saved_dt.data(), saved_dt.size() * sizeof(unsigned int), hipMemcpyHostToDevice));
-    if (strip_rows) *strip_rows = best;
-    if (general_rows) *general_rows = ctx->trows;
+    if (strip_rows) *strip_rows = best.name;
+    if (general_rows) *general_rows = best.tile;
     if (ms_best) *ms_best = best_ms;
     return THY_OK;
 }
