@@ -50,3 +50,20 @@ def test_tuned_heights_survive_an_upload():
     s.run(max_steps=48, steps_per_sync=48)
     assert _us(s) < slow / 4
     assert s.autotune(5)[0] < 100
+
+
+def test_tile_height_in_a_batch():
+    """Tiles of one row load nine for it, and are eight times as many."""
+    from thysea import serving
+    pr = make_problem(nx=700, ny=600, seed=9, coast=("north", "east"), t_sim=120.0)
+    us, res = {}, {}
+    for rows in (0, 8, 1):
+        kw = dict(kernel="sweep_general", general_rows=rows)
+        gpu = []
+        for _ in range(3):
+            rec, out, g = serving.run_batched([pr] * 8, steps_per_sync=24, keep=range(8), solver_kw=kw)
+            gpu.append(g)
+        us[rows], res[rows] = float(np.median(gpu)), out
+    assert us[1] > 2 * us[8] and us[0] < 1.5 * us[8], us
+    for i in range(8):
+        assert np.array_equal(res[1][i]["max_height"], res[8][i]["max_height"])

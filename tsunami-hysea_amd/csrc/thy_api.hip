@@ -627,7 +627,8 @@ int need_lists(thy_ctx *ctx) {
 // grids: tiles are whole, and strips of 24 rows cost the least (GPU time of 24 scenarios of
 // 1000x800: 88.0 / 86.3 / 85.7 ms at 16 / 24 / 32 rows; a mix of 12 grids 76.9 / 75.8 / 76.6).
 int build_batched(thy_ctx *ctx) {
-    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 24, kTileRows, INT_MAX);
+    const int R = ctx->prm.general_rows > 0 ? std::min(ctx->prm.general_rows, kTileRows) : kTileRows;
+    return build_lists(ctx, ctx->batched, ctx->prm.strip_rows > 0 ? ctx->prm.strip_rows : 24, R, INT_MAX);
 }
 
 template <typename T>
