@@ -65,3 +65,27 @@ def test_infinite_threshold(kernel, precision):
     pr = make_problem(nx=130, ny=44, seed=3)
     pr.hpos = float("inf")
     _replay(pr, 8, precision=precision, kernel=kernel)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("borders", [(1, 1, 1, 1), (1, -1, 2, 2)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 6, 7, 8])
+def test_every_face_listed_in_rounds(rows, borders, precision):
+    """hpos above every depth lists all faces of a tile: a tile of m rows has 57 m + 56 (m + 1)
+    of them in the momentum pass, and 508 are taken at a time, those of 4 rows."""
+    from test_gpu_tiles import _replay
+    assert 4 * 57 + 5 * 56 == 508 and (rows * 57 + (rows + 1) * 56 > 508) == (rows > 4)
+    pr = make_problem(nx=185, ny=45, seed=3, borders=borders)
+    pr.hpos = 10.0
+    _replay(pr, 8, precision=precision, general_rows=rows)
+
+
+def test_every_face_listed_in_a_batch():
+    """A batch's tiles have 8 rows: the same results as alone, with tiles of other heights."""
+    from thysea import serving
+    pr = make_problem(nx=190, ny=61, seed=9, t_sim=60.0)
+    pr.hpos = 10.0
+    kw = dict(steps_per_sync=6, keep=[0])
+    (ra, a, _), (rb, b) = serving.run_batched([pr], **kw), serving.run_sequential([pr], **kw)
+    assert ra[0]["steps"] == rb[0]["steps"] > 6
+    assert all(np.array_equal(a[0][k], b[0][k]) for k in ("max_height", "arrival_times"))

@@ -241,7 +241,7 @@ template <typename T> __device__ __forceinline__ SC<T> sc_of(T e, T D, T qn, T q
 // 8 rows: taller tiles would have less halo (4 of 12 rows in the mass pass), but at 8 the
 // tile's LDS (31 KB in FP32) lets five workgroups share a CU, as their registers do.
 constexpr int kTileRows = 8;
-constexpr int kTileHalf = 3;  // rows whose momentum faces always fit the result table
+constexpr int kTileHalf = 4;  // rows whose momentum faces always fit the result table
 
 using mask64 = unsigned long long;
 
@@ -251,21 +251,30 @@ template <typename T> struct alignas(16) FaceOut {
 
 template <typename T> struct TileLds {
     static constexpr int G = kTileRows;
-    static constexpr int kFluxes = 2 * (G + 5) * 64;
-    static constexpr int kResults = kFluxes / 4;  // listed momentum faces at a time
-    static_assert(kResults >= kTileHalf * 57 + (kTileHalf + 1) * 56, "a round of kTileHalf rows fits");
+    // listed momentum faces at a time: those of kTileHalf rows, two for each thread.  Where
+    // every face is listed (a shelf shallower than hpos) a tile of 8 rows takes two such rounds;
+    // with three of 3, 3 and 2 rows, in twice as many passes of the workgroup, a step of
+    // 2000x2000 took 261 us and takes 226 (FP64 811 and 656).
+    static constexpr int kResults = kTileHalf * 57 + (kTileHalf + 1) * 56;
+    static_assert(kResults <= 2 * 64 * SW_WAVES, "two faces a thread");
     T in[4][(G + 8) * 64];   // e, D, qx, qy of rows y0-4 .. y0+m+3
     T es[(G + 4) * 64];      // e* of rows y0-2 .. y0+m+1
+    // a listed face: direction << 15 | row << 6 | lane
     union {
-        T F[2][(G + 5) * 64];     // mass fluxes of the x faces (row, lane) and y faces
-        FaceOut<T> R[kResults];   // results of the listed momentum faces
+        struct {
+            T F[2][(G + 5) * 64];   // mass fluxes of the x faces (row, lane) and y faces
+            unsigned short mass_list[(G + 4) * 61 + (G + 5) * 60];
+        };
+        struct {  // (once the fluxes have been read)
+            FaceOut<T> R[kResults];  // results of the listed momentum faces
+            unsigned short list[kResults];
+        };
     };
     RowGeo<T> row[G + 4];    // of rows y0-2 ..
     FaceGeoY<T> fy[G + 5];   // of faces y0-2 ..
     mask64 deep[G + 8], dry[G + 8];    // lanes deeper than hpos / dry (h <= eps), by row
     mask64 sdeep[G + 4], sdry[G + 4];  // the same of h*
     int still[SW_WAVES];               // the wavefront's rows are land
-    unsigned short list[(G + 4) * 61 + (G + 5) * 60];  // direction << 15 | row << 6 | lane
 };
 
 // Lane l holds the masks of row l: the lanes whose x face, and whose lower y face, take the
@@ -483,8 +492,8 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
             s.F[1][j * 64 + lane] = Fy;
             if (wx | wy) {
                 const int b = __builtin_amdgcn_readlane(rf.base, j);
-                if (lane_of(wx)) s.list[b + rank_of(wx)] = (unsigned short)(j << 6 | lane);
-                if (lane_of(wy)) s.list[b + __popcll(wx) + rank_of(wy)] = (unsigned short)(0x8000 | j << 6 | lane);
+                if (lane_of(wx)) s.mass_list[b + rank_of(wx)] = (unsigned short)(j << 6 | lane);
+                if (lane_of(wy)) s.mass_list[b + __popcll(wx) + rank_of(wy)] = (unsigned short)(0x8000 | j << 6 | lane);
             }
         }
     }
@@ -524,7 +533,7 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
     if (nm) {
         const StepArgs<T> &a = again<T>(args);
         for (int k = tid; k < nm; k += 64 * W) {
-            const int code = s.list[k], l = code & 63, j = (code >> 6) & 31;
+            const int code = s.mass_list[k], l = code & 63, j = (code >> 6) & 31;
             const Listed f = listed(a, code, j);
             const int p = (j + 2) * 64 + l, st = f.yf ? 64 : 1;
             const T *const qn = f.yf ? qy_ : qx_;
