@@ -75,7 +75,6 @@ struct thy_ctx {
     double *mass_partial = nullptr;
     float *outbuf = nullptr;
     hipStream_t stream = nullptr;
-    hipStream_t side = nullptr;          // the other stream of the cached pair
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // two replays in flight: start / end / control-copied events, pinned copies of the
     // control block, the last launch's dt partials and the health flag after each replay
@@ -1226,7 +1225,7 @@ int thy_create(const thy_grid *g, const thy_params *p, thy_ctx **out) {
     ctx->state_bytes = (size_t)state_arrays(p) * ctx->pitch * ctx->ny * ctx->esz;
     if (ctx->kernel != 1 && ctx->state_bytes > (size_t)INT32_MAX) ctx->kernel = 1;
     HIPCHK(hipSetDevice(0));
-    HIPCHK(Pool::get().get_streams(ctx->stream, ctx->side));
+    HIPCHK(Pool::get().get_stream(ctx->stream));
     {
         int dev = 0;
         HIPCHK(hipGetDevice(&dev));
@@ -1311,7 +1310,6 @@ void thy_destroy(thy_ctx *ctx) {
     if (!ctx) return;
     // no queued work may still use what goes back to the caches
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     drop_graphs(ctx);
     void *ptrs[] = {ctx->state, ctx->row, ctx->fy, ctx->deep_row, ctx->area_d, ctx->ctrl, ctx->dtmin, ctx->scratch_u,
                     ctx->ftime, ctx->gpos, ctx->gbuf, ctx->gtime, ctx->okada_def, ctx->okada_row, ctx->okada_plane, ctx->mass_partial, ctx->outbuf,
@@ -1326,7 +1324,7 @@ void thy_destroy(thy_ctx *ctx) {
     Pool::get().host_free(ctx->h_snap);
     Pool::get().host_free(ctx->h_aux);
     Pool::get().host_free(ctx->h_dt);
-    if (ctx->stream) Pool::get().put_streams(ctx->stream, ctx->side);
+    if (ctx->stream) Pool::get().put_stream(ctx->stream);
     delete ctx;
 }
 
@@ -1772,7 +1770,7 @@ struct thy_batch {
     int capacity = 0;
     size_t budget = 0, used = 0;
     int K = 24;
-    hipStream_t stream = nullptr, side = nullptr;
+    hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_done = nullptr;   // end of a launch's work (admissions queue copies after it)
     std::vector<thy_ctx *> ctx;     // per slot; nullptr when free
@@ -1965,9 +1963,9 @@ int thy_batch_create(int capacity, size_t hbm_budget, int steps_per_sync, thy_ba
     b->state.assign(capacity, THY_SLOT_FREE);
     b->res.assign(capacity, thy_run_result{});
     b->launched.assign(capacity, 0);
-    // cached streams: creating and destroying streams with every batch would shift how
-    // the runtime spreads streams over the hardware queues
-    BHIPCHK(Pool::get().get_streams(b->stream, b->side));
+    // (a cached stream: creating and destroying streams with every batch would shift how
+    // the runtime spreads streams over the hardware queues)
+    BHIPCHK(Pool::get().get_stream(b->stream));
     BHIPCHK(hipEventCreate(&b->ev0));
     BHIPCHK(hipEventCreate(&b->ev1));
     BHIPCHK(hipEventCreateWithFlags(&b->ev_done, hipEventDisableTiming));
@@ -1985,7 +1983,6 @@ void thy_batch_destroy(thy_batch *b) {
     RelaxedCapture relaxed;
     if (!b) return;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
-    if (b->side) (void)hipStreamSynchronize(b->side);
     Pool::get().host_free(b->h_ctrl);
     Pool::get().host_free(b->h_args);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
@@ -1995,7 +1992,7 @@ void thy_batch_destroy(thy_batch *b) {
     hipEvent_t evs[] = {b->ev0, b->ev1, b->ev_done};
     for (hipEvent_t e : evs)
         if (e) (void)hipEventDestroy(e);
-    if (b->stream) Pool::get().put_streams(b->stream, b->side);
+    if (b->stream) Pool::get().put_stream(b->stream);
     delete b;
 }
 

@@ -1,5 +1,5 @@
 // Process-wide caches behind the library's allocations: device blocks, pinned host
-// blocks and stream pairs.
+// blocks and streams.
 //
 // hipFree and hipHostFree wait for the whole device, and a stream costs milliseconds
 // to create.  A server that admits and retires scenarios continuously would pay both
@@ -16,7 +16,6 @@
 #include <cstdlib>
 #include <mutex>
 #include <unordered_map>
-#include <utility>
 #include <vector>
 
 namespace thy {
@@ -35,54 +34,35 @@ class Pool {
     hipError_t host_alloc(void **p, size_t bytes) { return alloc(host_, p, bytes); }
     void host_free(void *p) { give_back(host_, p); }
 
-    // a pair of streams (default priority), cached or new; non-blocking, so that work
-    // other code puts on the null stream does not order against them
-    hipError_t get_streams(hipStream_t &a, hipStream_t &b) {
+    // a stream (default priority), cached or new; non-blocking, so that work other code puts
+    // on the null stream does not order against it
+    hipError_t get_stream(hipStream_t &s) {
         {
             std::lock_guard<std::mutex> g(m_);
             if (!streams_.empty()) {
-                a = streams_.back().first;
-                b = streams_.back().second;
+                s = streams_.back();
                 streams_.pop_back();
                 return hipSuccess;
             }
         }
-        return new_streams(a, b);
+        return hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
     }
-
-    // a new pair, not from the cache
-    hipError_t new_streams(hipStream_t &a, hipStream_t &b) {
-        a = b = nullptr;
-        // the runtime gives a new stream the hardware queue that serves the fewest
-        // streams; the two of a pair are created back to back (no other thread's stream
-        // in between), so that unless one queue serves two streams fewer than every
-        // other, they go to two different queues and their launches overlap
-        std::lock_guard<std::mutex> g(create_m_);
-        hipError_t e = hipStreamCreateWithFlags(&a, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipStreamCreateWithFlags(&b, hipStreamNonBlocking);
-        if (e != hipSuccess) {
-            if (a) (void)hipStreamDestroy(a);
-            a = b = nullptr;
-        }
-        return e;
-    }
-    // streams with no queued work left
-    void put_streams(hipStream_t a, hipStream_t b) {
+    // a stream with no queued work left
+    void put_stream(hipStream_t s) {
         {
             std::lock_guard<std::mutex> g(m_);
-            if (streams_.size() < kMaxStreamPairs) {
-                streams_.emplace_back(a, b);
+            if (streams_.size() < kMaxStreams) {
+                streams_.push_back(s);
                 return;
             }
         }
-        (void)hipStreamDestroy(a);
-        (void)hipStreamDestroy(b);
+        (void)hipStreamDestroy(s);
     }
 
     // release every cached block and stream
     void trim() {
         std::vector<void *> d, h;
-        std::vector<std::pair<hipStream_t, hipStream_t>> s;
+        std::vector<hipStream_t> s;
         {
             std::lock_guard<std::mutex> g(m_);
             take_all(dev_, d);
@@ -91,10 +71,7 @@ class Pool {
         }
         for (void *p : d) (void)hipFree(p);
         for (void *p : h) (void)hipHostFree(p);
-        for (auto &x : s) {
-            (void)hipStreamDestroy(x.first);
-            (void)hipStreamDestroy(x.second);
-        }
+        for (hipStream_t x : s) (void)hipStreamDestroy(x);
     }
 
     size_t cached_device_bytes() {
@@ -103,7 +80,7 @@ class Pool {
     }
 
   private:
-    static constexpr size_t kMaxStreamPairs = 64;
+    static constexpr size_t kMaxStreams = 64;
     struct Heap {
         bool host = false;
         size_t cached = 0, limit = 0;
@@ -199,9 +176,8 @@ class Pool {
     }
 
     std::mutex m_;
-    std::mutex create_m_;  // stream pairs are created one pair at a time
     Heap dev_, host_;
-    std::vector<std::pair<hipStream_t, hipStream_t>> streams_;
+    std::vector<hipStream_t> streams_;
 };
 
 inline hipError_t dev_alloc(void **p, size_t bytes) { return Pool::get().dev_alloc(p, bytes); }

@@ -304,10 +304,6 @@ __device__ __forceinline__ bool lane_of(const mask64 m) { return __builtin_amdgc
 __device__ __forceinline__ int rank_of(const mask64 m) {  // set bits below this lane
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
-__device__ __forceinline__ mask64 uniform_mask(const mask64 m) {
-    return ((mask64)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
-           (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m);
-}
 // x faces (lane = the face's high cell) whose four cells / two cells are all in m
 __device__ __forceinline__ mask64 all4(const mask64 m) { return m & (m << 1) & (m << 2) & (m >> 1); }
 __device__ __forceinline__ mask64 both(const mask64 m) { return m & (m << 1); }
