@@ -1195,7 +1195,12 @@ size_t thy_footprint(int nx, int ny, const thy_params *p) {
     const size_t n = pitch * ny;
     size_t bytes = (size_t)state_arrays(p) * n * esz;
     bytes += (size_t)nx * ny * (8 + 4);                 // okada scratch (double) + output staging (float)
-    bytes += (size_t)(ny + 1) * 64 * 2;                 // geometry
+    // row tables: geometry, deep-water records, mass weight, Okada
+    const size_t row = esz == 8 ? sizeof(RowGeo<double>) + sizeof(FaceGeoY<double>) + sizeof(DeepRow<double>)
+                                : sizeof(RowGeo<float>) + sizeof(FaceGeoY<float>) + sizeof(DeepRow<float>);
+    bytes += (size_t)(ny + 1) * (row + sizeof(double) + sizeof(OkadaRow));
+    // work lists, of a run alone and of a batch: no more items and strips than lowest tiles
+    bytes += 2 * ((size_t)nx / SW_OUT + 1) * ((size_t)ny / kTileLow + 1) * sizeof(int2);
     return bytes;
 }
 
