@@ -406,11 +406,11 @@ int pick_tile(thy_ctx *c) {
 // Rows per deep-water strip of a grid of `rows` segment rows (56-column segments times
 // rows) that is stepped alone.  A strip's time is a chain of rows with a halo of 5: with few
 // rows the step is the time of one strip, so strips are short; with many the halo's work
-// counts.  Measured (us per step): 1000x800 (14400 rows) 17.2 / 19.3 / 19.4 at 8 / 12 / 16
-// rows; 1400x1200 (30000) 28.7 / 26.4 / 31.9 at 8 / 16 / 24; 2000x2000 (72000) 47.7 / 46.6 /
-// 48.0 at 16 / 24 / 28, FP64 124.2 / 118.9 / 122.4 at 16 / 24 / 32; 2500x2500 (112500) 59.2 /
-// 59.0 / 66.5 at 16 / 24 / 32; 4000x3000 (216000) 126.0 / 135.8 / 122.4 / 139.5 at 16 / 24 /
-// 32 / 40.
+// counts.  Measured (us per step, coasts in the north and east): 1000x800 (14400 rows) 18.7 /
+// 19.5 / 20.2 at 8 / 12 / 16 rows; 1400x1200 (30000) 29.0 / 25.8 / 29.1 at 8 / 16 / 24; 2000x2000
+// (72000) 45.5 / 43.8 / 44.3 at 16 / 24 / 28, FP64 110.8 / 107.8 / 106.5 at 16 / 24 / 32;
+// 2500x2500 (112500) 61.2 / 59.7 / 61.3 at 16 / 24 / 32; 4000x3000 (216000) 120.6 / 118.6 /
+// 119.2 / 120.4 at 16 / 24 / 32 / 40.
 int default_strip_rows(const size_t rows, const int ncu) {
     const size_t per = rows / ncu;
     return per < 80 ? 8 : (per < 200 ? 16 : (per < 560 ? 24 : 32));
@@ -418,8 +418,8 @@ int default_strip_rows(const size_t rows, const int ncu) {
 
 // Rows per general tile of a grid stepped alone.  Whole tiles have the least halo.  On a
 // small grid the step is the time of one tile, so tiles are lower there, the more the
-// smaller it is (240x200, 3.9 segment rows a CU: 12.8 / 13.3 / 15.3 us at 3 / 4 / 8 rows;
-// 1000x800, 56 rows: 19.1 / 17.2 at 4 / 8).
+// smaller it is (240x200, 3.9 segment rows a CU: 11.8 / 12.3 / 14.4 us at 3 / 4 / 8 rows;
+// 1000x800, 56 rows: 18.6 / 15.9 at 4 / 8).
 int default_tile_rows(const size_t rows, const int ncu) {
     return (int)std::min<size_t>(kTileRows, 3 + rows / ((size_t)ncu * 8));
 }
@@ -427,8 +427,8 @@ int default_tile_rows(const size_t rows, const int ncu) {
 // Listed faces (the estimate of find_coast) above which a tile of a grid stepped alone is
 // made lower, down to kTileLow rows: the step would wait for the tiles along the coast.
 // Above about 130 segment rows a CU no tile reaches it: many tiles share a CU there, and
-// lower ones only add halo.  Us a step without this rule and with it: 1501x607 29.4 and
-// 19.2, 800x900 27.7 and 17.0, 731x412 17.8 and 15.4, 1000x800 16.9 and 16.6.
+// lower ones only add halo.  Us a step without this rule and with it, a coast in the north:
+// 1501x607 24.3 and 17.9, 800x900 23.5 and 15.7, 731x412 16.5 and 14.5, 1000x800 24.3 and 16.4.
 constexpr int kTileLow = 3;
 int tile_budget(const size_t rows, const int ncu) { return (int)std::min<size_t>(100000, 5 * rows / ncu); }
 
@@ -1780,7 +1780,7 @@ struct thy_batch {
     hipEvent_t ev_done = nullptr;   // end of a launch's work (admissions queue copies after it)
     std::vector<thy_ctx *> ctx;     // per slot; nullptr when free
     std::vector<size_t> bytes;      // admitted footprint per slot
-    std::vector<int> srows;         // strip height in the slot's argument block
+    std::vector<int> srows;         // strip height of the context's own lists at admission
     std::vector<int> state;         // THY_SLOT_*
     std::vector<thy_run_result> res;
     StepArgs<float> *d_args = nullptr;
@@ -1837,7 +1837,8 @@ int batch_items(thy_batch *b) {
     for (int i = 0; i < b->capacity; i++) {
         if (b->state[i] != THY_SLOT_RUNNING) continue;
         const thy_ctx *c = b->ctx[i];
-        // the lists must be those of the argument block
+        // a context that was tuned after its admission is refused: its own launches replayed
+        // steps on the buffers and control blocks that the batch advances
         if (c->srows != b->srows[i]) return bfail(b, THY_ERR_INVALID, "strip height changed after admission");
         const WorkLists &w = c->batched;
         for (size_t p = 0; p < w.tile_h.size(); p++)

@@ -85,14 +85,15 @@ __global__ void __launch_bounds__(256) k_initial_dt(const StepArgs<T> a, int cur
 // quotients and ten square roots a cell for 8 bytes written.  Sums over the corners inside the
 // logarithms and tangents need fewer (204 us a fault), but round otherwise, and a cell whose
 // rise comes close to the arrival threshold then arrives a step earlier or later.  So every
-// sum keeps its terms and its order, and what is saved leaves each value as it is:
+// sum keeps its terms and its order, and what is saved leaves each value as it is, or rounds
+// a quotient or root in another way at most (none of the faults tried shows a difference):
 //   * quotients and square roots without scaling and special cases, one reciprocal for all
 //     quotients by the same divisor;
 //   * the functions of the fault's angles and of a row's latitude come from tables;
 //   * logarithms only with strike slip, tangents only with dip slip;
 //   * a loop over the corners holds the registers of one.
-// Per fault on 2000x2000 cells: 882 us before, 311 now (181 registers and 2 wavefronts a SIMD
-// before, 114 and 4 now).
+// Per fault on 2000x2000 cells: 319 us, with 114 registers and 4 wavefronts a SIMD; 882 us in
+// the general forms without tables (181 registers, 2 wavefronts).
 // ---------------------------------------------------------------------------
 struct OkadaFault {
     double lon_c, lat_c, depth, L, W, H, strike, dip, rake, slip;

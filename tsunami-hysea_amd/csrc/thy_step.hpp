@@ -93,12 +93,11 @@ template <typename T> struct alignas(32) DeepRow {
 
 // The dt minimum of a launch is kept as kDtParts partial minima (float bits; for
 // positive floats the unsigned order is the float order), one 64-byte line apart:
-// atomics on one line are applied one after another.  The launches of one grid fold
-// one minimum per workgroup into partial 0, and the next launch reads that one word.
-// The batch launches fold one per wavefront (several thousand per launch for a large
-// grid) into partial (wavefront index mod kDtParts), so that the launch does not wait
-// for a queue of atomics on one line, and read all partials.  The writer of a launch
-// resets every partial of the next launch's slot.
+// atomics on one line are applied one after another.  Workgroup b of the row sweep (one
+// grid or a batch; several thousand workgroups on a large grid) folds its minimum into
+// partial b mod kDtParts, so that a launch does not wait for a queue of atomics on one
+// line, and the next launch's workgroups read all partials; k_step uses partial 0 alone.
+// The writer of a launch resets every partial of the next launch's slot.
 constexpr int kDtParts = 8;
 constexpr int kDtStride = 16;  // words: one 64-byte line per partial
 constexpr int kDtSlot = kDtParts * kDtStride;

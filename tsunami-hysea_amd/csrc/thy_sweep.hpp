@@ -67,8 +67,9 @@ template <typename T> __device__ __forceinline__ const StepArgs<T> &again(ArgsAt
 // Deep-water forms of the face fluxes: the 2s branch that mass_flux / mom_flux take
 // when all four stencil depths exceed hpos outside the first-order band
 // (src/GPU/Arista_kernel.cu:545,653,1105,1214), written with the per-cell square
-// roots and velocities computed once per cell (the same arithmetic as the per-lane 2s
-// branch of the general faces, so either path gives a face the same value).
+// roots and velocities computed once per cell.  Strips and tiles both evaluate a deep face
+// through these, so either gives it the same value.  (k_step has its own 2s branch: in FP64
+// with the general quotients and roots, so its last place may differ.)
 // ---------------------------------------------------------------------------
 // Mass flux of the x face between hL and the row's cell (h1), and of the y face between h0
 // and h1: src/GPU/Arista_kernel.cu:79-95,118-130, 97-114,674-686 (Fx, Fy: normal discharge
@@ -234,9 +235,9 @@ template <typename T> __device__ __forceinline__ SC<T> sc_of(T e, T D, T qn, T q
 // A tile's time is a chain of latencies.  Everything it reads from memory (rows, row tables,
 // metrics) is requested at once, and so is everything a phase reads from LDS.  The rows'
 // masks are combined in one go, a row to a lane, in every wavefront alike, and a sum over the
-// lanes says where each row's faces go in the list (one atomic counter and one mask read per
-// row before).  A whole step of 240x200, where nothing else counts: 14.3 us before, 12.4 now
-// (with tiles of 3 rows instead of 4); 2000x2000, 1563 tiles: 50.4 and 46.4.
+// lanes says where each row's faces go in the list.  With an atomic counter and a mask read for
+// each row a whole step of 240x200, where nothing else counts, took 14.3 us where it takes 11.8
+// (tiles of 4 and of 3 rows); 2000x2000, 1563 tiles: 50.4 and 46.4.
 // ---------------------------------------------------------------------------
 // 8 rows: taller tiles would have less halo (4 of 12 rows in the mass pass), but at 8 the
 // tile's LDS (31 KB in FP32) lets five workgroups share a CU, as their registers do.
@@ -798,13 +799,13 @@ __device__ __forceinline__ double held(double v) { asm("" : "+v"(v)); return v; 
 // Returns whether it held; if not, the caller redoes the strip (its writes are then rewritten
 // and its dt is dropped).
 //
-// Bound by memory on a large grid (4000x3000, all deep: 111 us a step, 3.9 TB/s of the nine
-// arrays, whatever the strip height, and no less with two rows of cells in flight), by the
-// latency of a row on a small one.  A steady row takes 134 vector instructions (175 before:
-// a vote and a comparison for each condition, neighbours' values through the LDS pipe, two
-// limiter branches, copies from row to row, which two rows of the loop written out spare;
-// four rows are no faster).  2000x2000: 54.9 us a step before, 49.7 now; 1000x800 20.8 and
-// 18.6; FP64 2000x2000 143.5 and 134.3.
+// On a large grid vector issue and the traffic beyond the L2 bound it together (4000x3000, all
+// deep: 102 us a step, 4.2 TB/s of the nine arrays, and no less with two rows of cells in
+// flight), on a small one the latency of a row.  A steady row takes 132 vector instructions:
+// no vote or comparison for each condition, neighbours' values by lane moves, one test for
+// both limiters, and two rows of the loop written out, which spares the copies from row to row
+// (four rows are no faster).  With those it took 175, and 2000x2000 54.9 us a step where it
+// took 49.7 without, 1000x800 20.8 and 18.6, FP64 2000x2000 143.5 and 134.3.
 template <typename T>
 __device__ __forceinline__ bool deep_strip(const StepArgs<T> &a, const BlockCtl<T> &bc, const int x0, const int y0,
                                            const int rows, float &dtmin_out) {
