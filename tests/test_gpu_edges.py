@@ -89,3 +89,20 @@ def test_every_face_listed_in_a_batch():
     (ra, a, _), (rb, b) = serving.run_batched([pr], **kw), serving.run_sequential([pr], **kw)
     assert ra[0]["steps"] == rb[0]["steps"] > 6
     assert all(np.array_equal(a[0][k], b[0][k]) for k in ("max_height", "arrival_times"))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kernel", ["sweep", "sweep_general"])
+def test_dry_land_and_a_threshold_below_zero(kernel, precision):
+    """With hpos below 0 dry cells count as deep; land alone stays as it is all the same."""
+    from thysea import native
+    pr, D = _inland()
+    pr.H[:, :] = 0.0
+    pr.h = np.zeros_like(pr.h)
+    pr.hpos = -1.0
+    s = native.Solver(pr, kernel=kernel, precision=precision)
+    a = s.state()
+    assert s.step(1e-4) > 0
+    s.run(max_steps=3)
+    assert all(np.array_equal(x, y) for x, y in zip(a, s.state()))
+    s.close()

@@ -586,6 +586,8 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
     // rows outside the grid stand for the edge row (clamped stencils)
     const int jlo = max(0, 2 - y0), jhi = min(m + 3, ny + 1 - y0);
     auto row_j = [&](const int j) { return min(max(j, jlo), jhi); };
+    // with an hpos below 0 dry cells count as deep: faces between two of them are zero there too
+    const mask64 below = ah.hpos < T(0) ? ~0ull : 0ull;
     // ---- momentum pass, rows y0+r0 .. y0+r1-1 at a time: the whole tile, or kTileHalf rows
     // when its listed faces do not fit the result table ----
     for (int r0 = 0, r1 = m; r0 < m;) {
@@ -595,11 +597,11 @@ __device__ __forceinline__ float general_tile(const ArgsAt<T> args, const BlockC
             const int i = min(lane, m), g = y0 + i;
             const mask64 d2 = s.sdeep[i + 2], dy = s.sdeep[i] & s.sdeep[i + 1] & d2 & s.sdeep[i + 3];
             const bool in_x = lane >= r0 && lane < r1, in_y = lane >= r0 && lane <= r1;
-            rf.dx = in_x ? all4(d2) & ~first : 0ull;
-            rf.dy = in_y && !(g < 2 || g > ny - 2) ? dy : 0ull;
-            rf.wx = in_x ? ~rf.dx & ~both(s.sdry[i + 2]) & on_face & 0x1ffffffffffffff0ull : 0ull;  // lanes 4 .. 60
-            rf.wy = in_y ? ~rf.dy & ~(s.sdry[row_j(i + 1)] & s.sdry[row_j(i + 2)]) & on_cell & 0x0ffffffffffffff0ull
-                         : 0ull;  // lanes 4 .. 59
+            const mask64 bx = both(s.sdry[i + 2]), by = s.sdry[row_j(i + 1)] & s.sdry[row_j(i + 2)];
+            rf.dx = in_x ? all4(d2) & ~first & ~(bx & below) : 0ull;
+            rf.dy = in_y && !(g < 2 || g > ny - 2) ? dy & ~(by & below) : 0ull;
+            rf.wx = in_x ? ~rf.dx & ~bx & on_face & 0x1ffffffffffffff0ull : 0ull;  // lanes 4 .. 60
+            rf.wy = in_y ? ~rf.dy & ~by & on_cell & 0x0ffffffffffffff0ull : 0ull;  // lanes 4 .. 59
             return place_faces(rf);
         };
         int nq = classify();
