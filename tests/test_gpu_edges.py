@@ -106,3 +106,15 @@ def test_dry_land_and_a_threshold_below_zero(kernel, precision):
     s.run(max_steps=3)
     assert all(np.array_equal(x, y) for x, y in zip(a, s.state()))
     s.close()
+
+
+@pytest.mark.parametrize("t_end", [-1.0, float("nan")])
+def test_a_run_that_ends_before_it_starts(t_end):
+    """No step and no gauge sample, whatever the series interval."""
+    from thysea import native
+    pr = make_problem(nx=90, ny=40)
+    pr.gauge_pos, pr.series_interval, pr.t_end = np.array([5, 700], np.int32), 0.01, t_end
+    s = native.Solver(pr)
+    out = s.run(max_steps=5)
+    assert out["steps"] == 0 and out["n_samples"] == 0 and out["g_eta"].shape == (0, 2)
+    s.close()

@@ -1696,7 +1696,7 @@ static int prepare_run(thy_ctx *ctx, const thy_run_config *cfg, thy_run_result *
     if (cfg->n_gauges > 0 && cfg->series_interval >= 0.0) {
         double nsd = cfg->series_interval > 0.0 ? cfg->t_end / cfg->series_interval + 4.0 : 1e6;
         if (cfg->max_steps > 0 && cfg->series_interval <= 0.0) nsd = (double)cfg->max_steps + 2.0;
-        ctx->gcap = (int)std::min(nsd, 1e6);
+        if (nsd > 0.0) ctx->gcap = (int)std::min(nsd, 1e6);  // (a run that ends before its start has none)
     }
     HIPCHK(dev_alloc((void **)&ctx->gpos, std::max(1, ctx->ng) * sizeof(int)));
     if (ctx->ng) HIPCHK(ctx_copy(ctx, ctx->gpos, cfg->gauge_pos, ctx->ng * sizeof(int), hipMemcpyHostToDevice));
