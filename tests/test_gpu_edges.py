@@ -118,3 +118,17 @@ def test_a_run_that_ends_before_it_starts(t_end):
     out = s.run(max_steps=5)
     assert out["steps"] == 0 and out["n_samples"] == 0 and out["g_eta"].shape == (0, 2)
     s.close()
+
+
+@pytest.mark.parametrize("eps_h", [1e100, float("inf")])
+@pytest.mark.parametrize("kernel", ["sweep", "tile"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_every_cell_dry(precision, kernel, eps_h):
+    """eps_h above every depth: the run goes on, and every cell is written as dry."""
+    from thysea import native
+    pr = make_problem(nx=130, ny=44, seed=3)
+    pr.eps_h = eps_h
+    s = native.Solver(pr, precision=precision, kernel=kernel)
+    assert s.run(max_steps=6)["steps"] >= 1
+    assert np.all(np.isfinite(s.state()[0])) and np.all(s.field("eta") == np.float32(-9999))
+    s.close()

@@ -225,10 +225,12 @@ StepArgs<T> make_args(thy_ctx *c, const bool batch = false) {
     a.track_arrival = p.track_arrival;
     a.n_gauges = c->ng;
     a.bsup = (T)p.borde_sup; a.binf = (T)p.borde_inf; a.bizq = (T)p.borde_izq; a.bder = (T)p.borde_der;
-    a.cfl = (T)p.cfl; a.mf0 = (T)p.mf0; a.vmax = (T)p.vmax; a.eps_h = (T)p.eps_h;
+    a.cfl = (T)p.cfl; a.mf0 = (T)p.mf0; a.vmax = (T)p.vmax;
     // an infinite hpos as a large one: no depth reaches either and the exponentials of its
     // quotients saturate alike, but a quotient without special cases takes finite numbers
     a.hpos = (T)std::max(std::min(p.hpos, 1e30), -1e30);
+    // (the same for an eps_h whose fourth power overflows: every cell is dry with either)
+    a.eps_h = sizeof(T) == 8 ? (T)std::min(p.eps_h, 1e70) : (T)p.eps_h;
     a.cvis = (T)p.cvis; a.dif_at = (T)p.dif_at; a.sea_level = (T)p.sea_level;
     a.Href = (T)p.H; a.Q_over_H = (T)(p.Q / p.H);
     for (int b = 0; b < 2; b++) {
